@@ -14,8 +14,9 @@
 // contiguous, so one 16-byte LDS read feeds each MFMA operand.
 // The n_in -> width and width -> n_out layers (K = 8 or N = 2) are FP32
 // dot products on the vector units. GELU is the tanh form
-//   gelu(z) = z/2 (1 + tanh(sqrt(2/pi) (z + 0.044715 z^3))),
-// tanh from the exponential (tanh_fast).
+//   gelu(z) = z/2 (1 + tanh(sqrt(2/pi) (z + 0.044715 z^3))).
+// Widths 64, 128 and 256 (n_in <= 32) take the fused kernels further down
+// instead: one kernel for the whole network, one for all weight gradients.
 
 #include <cmath>
 #include <cstdint>
@@ -34,25 +35,24 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int kBM = 64, kBN = 128, kBK = 32, kPad = 8;
 constexpr int kLds = kBK + kPad;  // bf16 per LDS row
 
-// tanh(u) = 1 - 2 / (exp(2u) + 1) with the hardware exponential and
+// With u = sqrt(2/pi) (z + 0.044715 z^3) the tanh form is z sigma(2u):
+// (1 + tanh u) / 2 = 1 / (1 + exp(-2u)), one hardware exponential and one
 // reciprocal (relative error ~1e-6, far below the BF16 rounding the
-// activations take next; exp(2u) = inf gives 1, 0 gives -1). The
-// library tanhf made GELU 45 % of the fused inference time.
-__device__ __forceinline__ float tanh_fast(float u) {
-  return 1.0f - 2.0f * __builtin_amdgcn_rcpf(__expf(2.0f * u) + 1.0f);
+// activations take next), and no cancellation for negative z. exp(-2u) = inf
+// gives 0, 0 gives 1. Five ordinary and two quarter-rate instructions; they,
+// not the matrix cores, set the pace of the fused network.
+__device__ __forceinline__ float gelu_sigma(float z) {
+  const float k = -2.0f * 0.7978845608028654f * 1.4426950408889634f;  // -2 sqrt(2/pi) log2(e)
+  const float e = __builtin_amdgcn_exp2f(z * (k + k * 0.044715f * z * z));
+  return __builtin_amdgcn_rcpf(1.0f + e);
 }
 
-__device__ __forceinline__ float gelu(float z) {
-  const float c = 0.7978845608028654f;  // sqrt(2/pi)
-  const float u = c * (z + 0.044715f * z * z * z);
-  return 0.5f * z * (1.0f + tanh_fast(u));
-}
+__device__ __forceinline__ float gelu(float z) { return z * gelu_sigma(z); }
 
 __device__ __forceinline__ float dgelu(float z) {
   const float c = 0.7978845608028654f;
-  const float u = c * (z + 0.044715f * z * z * z);
-  const float t = tanh_fast(u);
-  return 0.5f * (1.0f + t) + 0.5f * z * (1.0f - t * t) * c * (1.0f + 3.0f * 0.044715f * z * z);
+  const float t = gelu_sigma(z);
+  return t + z * t * (1.0f - t) * (2.0f * c + 6.0f * c * 0.044715f * z * z);
 }
 
 struct GemmArgs {
@@ -300,151 +300,510 @@ __global__ void k_f32_to_bf16(const float* __restrict__ a, int64_t n, __bf16* __
   if (i < n) b[i] = __bf16(a[i]);
 }
 
-// Fused inference: the whole network for 128 rows per block (4 waves x 32
-// rows), activations kept in LDS between layers, hidden width x width layers
-// on MFMA with the weights read from L2. Same arithmetic and summation order
-// as forward(): first layer FP32 over the inputs, hidden layers in 16-wide k
-// chunks in increasing order, last layer FP32 over k in order; BF16
-// activations and weights, FP32 accumulation.
-constexpr int kInferRows = 128;
-constexpr int kInferMaxIn = 32;
-constexpr int kInferMaxLayers = 18;
+// ------------------------------------------------------- fused network
+// Widths 64, 128 and 256 with n_in <= 32: the whole network for 128 rows in
+// one workgroup of 4 waves, the activations (BF16) in LDS between layers,
+// every layer on MFMA with FP32 accumulation; in training the same kernel
+// goes on to the loss and back through the layers.
+//
+// Weights come as operand fragments: the 64 lanes' 8-element operands of one
+// MFMA in lane order, 1 KB contiguous (make_fragments lays them out once
+// per weight update). A wave owns 32 NT output columns for all rows, so no two
+// waves of a workgroup read the same weight and none goes through LDS; the
+// next four k-steps' fragments are loaded while the current four multiply,
+// and the next layer's first ones before the GELU epilogue. The weights
+// are the A operand: a lane then holds four consecutive outputs of one row
+// and stores them as 8 bytes. LDS (68 KB at width 256) and registers (256)
+// let two workgroups share a CU, so one's GELUs run beside the other's
+// MFMAs. Before, every wave computed 32 rows x all columns with the weights
+// staged through LDS (135 KB, one workgroup a CU): 1.5 LDS reads an MFMA
+// where 1 read of 8 cycles in 32 is the limit of four waves.
+// Measured (width 256, depth 4, n_in 7): inference of 912,673 rows 2310 ->
+// 542 us (670 TFLOP/s; the GELUs alone are ~0.35 ms of vector issue), four
+// Adam steps on 16,384 rows 5.95 -> 1.06 ms.
+//
+// Layer 0 takes its FP32 inputs as three BF16 parts of 8 bits each
+// (x = x1 + x2 + x3 exactly), times the same BF16 weight: exact products,
+// FP32 sums, as the scalar form. The same split serves dy and x in the
+// weight gradients.
+constexpr int kRows = 128;
+constexpr int kFusedMaxIn = 32;
+constexpr int kMaxLayers = 18;
+constexpr int kFrag = 512;  // bf16 per operand fragment
 
-struct InferArgs {
+struct FusedArgs {
   const float* X;
   int64_t M;
-  int nin, width, depth, nout;
-  const __bf16* w;     // BF16 weights, layer l at woff[l], [out][in]
-  const float* bias;   // FP32 biases, layer l at boff[l]
-  int64_t woff[kInferMaxLayers];
-  int64_t boff[kInferMaxLayers];
-  float* Y;
+  int nin, kp, depth, nout;  // kp: 3 nin + 1 rounded up to 32
+  const bf16x8* wf;          // forward fragments: layer 0, hidden layers, last layer
+  const bf16x8* wb;          // transposed fragments of the hidden layers (training)
+  const __bf16* wlast;       // last layer, [nout][width]
+  const float* bias;
+  int64_t boff[kMaxLayers];
+  float* Y;  // inference
+  // Training.
+  const float* T;
+  float scale;     // 1 / (M nout)
+  float4* z;       // pre-activations, in each thread's own order
+  bf16x8* hT;      // [layer][16-row chunk][32-column tile] fragments of h
+  bf16x8* dzT;     // same of dz
+  bf16x8* xT;      // [chunk][tile of kp columns]: x1 | x2 | x3 | 1
+  bf16x8* dyT;     // [chunk][tile of 3 nout columns]: dy1 | dy2 | dy3
+  double* loss;    // one partial sum per workgroup
+  int dy_lds;      // LDS offset of the rows' dy
 };
 
-// The weights of a hidden layer are staged through LDS in chunks of TC
-// output tiles (32 TC rows of W) shared by the block's 4 waves, instead of
-// every wave reading the whole layer from L2, double-buffered: each chunk's
-// global loads are issued into registers before the MFMA loop over the
-// previous chunk and stored to the other LDS buffer after it, so the L2
-// latency of the staging hides behind the MFMAs (the next layer's first
-// chunk is fetched during the current layer's last). The inputs of layer 0
-// use the same LDS region before the first chunk.
-template <int NT>
-__global__ __launch_bounds__(256) void k_mlp_infer(InferArgs g) {
-  constexpr int W = NT * 32;
-  constexpr int LD = W + 8;            // padded row (bf16) against LDS bank conflicts
-  constexpr int TC = NT < 2 ? NT : 2;  // output tiles per staged weight chunk
-  constexpr int NC = NT / TC;          // chunks per layer
-  constexpr int WROWS = 32 * TC;
-  constexpr int BUFB = WROWS * LD * 2;  // bytes of one chunk buffer
-  constexpr int VPT = WROWS * (W / 8) / 256;  // 16-byte vectors per thread and chunk
-  static_assert(VPT >= 1 && WROWS * (W / 8) % 256 == 0, "chunk does not split over 256 threads");
-  constexpr int WBYTES = 2 * BUFB > kInferRows * kInferMaxIn * 4 ? 2 * BUFB
-                                                                 : kInferRows * kInferMaxIn * 4;
-  __shared__ __bf16 act[kInferRows][LD];
-  __shared__ __attribute__((aligned(16))) unsigned char wbuf[WBYTES];
-  float (*xs)[kInferMaxIn] = reinterpret_cast<float (*)[kInferMaxIn]>(wbuf);
+// Fragments per layer.
+__host__ __device__ inline int64_t frags_first(int width, int kp) {
+  return int64_t(width / 32) * (kp / 16);
+}
+__host__ __device__ inline int64_t frags_hidden(int width) {
+  return int64_t(width / 32) * (width / 16);
+}
+
+// The three BF16 parts of an FP32 value, by truncation (exact remainders;
+// part 0 carries infinities and NaN alone).
+__device__ __forceinline__ float top_part(float x) {
+  return __uint_as_float(__float_as_uint(x) & 0xffff0000u);
+}
+__device__ __forceinline__ __bf16 split_part(float x, int part) {
+  if ((__float_as_uint(x) & 0x7f800000u) == 0x7f800000u) return part == 0 ? __bf16(x) : __bf16(0.0f);
+  const float x1 = top_part(x), r1 = x - x1, x2 = top_part(r1);
+  return __bf16(part == 0 ? x1 : part == 1 ? x2 : r1 - x2);
+}
+
+__device__ __forceinline__ uint32_t pack2(float a, float b) {
+  union {
+    __bf16 h[2];
+    uint32_t u;
+  } v;
+  v.h[0] = __bf16(a);
+  v.h[1] = __bf16(b);
+  return v.u;
+}
+
+template <int W>
+struct Tiling {
+  static constexpr int NT = W >= 256 ? 2 : 1;   // 32-column tiles per wave
+  static constexpr int WN = W / (32 * NT);      // waves along the columns
+  static constexpr int MT = 4 / (4 / WN);       // 32-row tiles per wave
+  static constexpr int LD = W + 8;              // padded LDS row (bf16): no bank conflicts
+  static constexpr int KC = W / 16;             // k-steps of a hidden layer
+  static constexpr int Q = MT * NT * 4;         // groups of 4 outputs per thread
+};
+
+// Workgroups a CU holds by LDS: 2 at width 256, 4 below.
+template <int W, bool TRAIN>
+__global__ __launch_bounds__(256, W >= 256 ? 2 : TRAIN && W >= 128 ? 3 : 4) void k_mlp_fused(FusedArgs g) {
+  using C = Tiling<W>;
+  constexpr int NT = C::NT, MT = C::MT, LD = C::LD, KC = C::KC, G = 4;
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  __bf16* act = reinterpret_cast<__bf16*>(lds);  // [kRows][LD]; first the split inputs
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int64_t r0 = int64_t(blockIdx.x) * kInferRows;
-  const int rows = int(min<int64_t>(kInferRows, g.M - r0));
-  for (int i = tid; i < kInferRows * g.nin; i += 256) {
-    const int r = i / g.nin, c = i - r * g.nin;
-    xs[r][c] = r < rows ? g.X[(r0 + r) * g.nin + c] : 0.0f;
-  }
-  __syncthreads();
-  // Chunk staging: registers <- global, then LDS buffer <- registers.
-  bf16x8 stage[VPT];
-  auto fetch = [&](int l, int ch) {
-    const __bf16* Wl = g.w + g.woff[l];
+  const int half = lane >> 5, col = lane & 31;
+  const int n0 = (wave % C::WN) * 32 * NT, m0 = (wave / C::WN) * 32 * MT;
+  const int64_t blk = blockIdx.x, r0 = blk * kRows;
+  const int rows = int(min<int64_t>(kRows, g.M - r0));
+  const int64_t nchunk = int64_t(gridDim.x) * (kRows / 16);
+
+  // Column-major fragments of an LDS matrix for the weight gradients.
+  auto transpose_out = [&](const __bf16* src, int ld, int tiles, bf16x8* dst) {
+    for (int f = wave; f < tiles * (kRows / 16); f += 4) {
+      const int mc = f / tiles, t = f - mc * tiles;
+      const __bf16* q = src + (mc * 16 + 8 * half) * ld + t * 32 + col;
+      bf16x8 v;
 #pragma unroll
-    for (int q = 0; q < VPT; ++q) {
-      const int v = tid + q * 256;
-      const int rr = v / (W / 8), cc = v - rr * (W / 8);
-      stage[q] = *reinterpret_cast<const bf16x8*>(Wl + int64_t(ch * WROWS + rr) * W + cc * 8);
+      for (int j = 0; j < 8; ++j) v[j] = q[j * ld];
+      dst[((blk * (kRows / 16) + mc) * tiles + t) * 64 + lane] = v;
     }
   };
-  auto commit = [&](int b) {
-    __bf16 (*wl)[LD] = reinterpret_cast<__bf16 (*)[LD]>(wbuf + b * BUFB);
+
+  f32x16 acc[MT][NT];
+  auto clear = [&] {
 #pragma unroll
-    for (int q = 0; q < VPT; ++q) {
-      const int v = tid + q * 256;
-      const int rr = v / (W / 8), cc = v - rr * (W / 8);
-      *reinterpret_cast<bf16x8*>(&wl[rr][cc * 8]) = stage[q];
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[m][t][r] = 0.0f;
+  };
+  bf16x8 pre[G][NT];  // the first fragments of the next hidden product
+  auto prefetch = [&](const bf16x8* w) {
+#pragma unroll
+    for (int q = 0; q < G; ++q)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) pre[q][t] = w[((n0 / 32 + t) * KC + q) * 64 + lane];
+  };
+  // acc = fragments w (rows n0 ..) times the activations, from pre on.
+  auto product = [&](const bf16x8* w) {
+    clear();
+    bf16x8 cur[G][NT];
+#pragma unroll
+    for (int k0 = 0; k0 < KC; k0 += G) {
+#pragma unroll
+      for (int q = 0; q < G; ++q)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          cur[q][t] = pre[q][t];
+          if (k0 + G < KC) pre[q][t] = w[((n0 / 32 + t) * KC + k0 + G + q) * 64 + lane];
+        }
+#pragma unroll
+      for (int q = 0; q < G; ++q)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+          const bf16x8 b = *reinterpret_cast<const bf16x8*>(
+              act + (m0 + m * 32 + col) * LD + (k0 + q) * 16 + 8 * half);
+#pragma unroll
+          for (int t = 0; t < NT; ++t)
+            acc[m][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cur[q][t], b, acc[m][t], 0, 0, 0);
+        }
     }
   };
-  if (g.depth > 1) fetch(1, 0);
-  // Layer 0: n_in -> W on the vector units, one output column per thread.
-  for (int n = tid; n < W; n += 256) {
-    float wr[kInferMaxIn];
-    for (int c = 0; c < g.nin; ++c) wr[c] = float(g.w[g.woff[0] + int64_t(n) * g.nin + c]);
-    const float bn = g.bias[g.boff[0] + n];
-    for (int r = 0; r < kInferRows; ++r) {
-      float z = bn;
-      for (int c = 0; c < g.nin; ++c) z += xs[r][c] * wr[c];
-      act[r][n] = __bf16(gelu(z));
-    }
-  }
-  __syncthreads();  // xs (the first buffers' region) is no longer read
-  if (g.depth > 1) commit(0);
-  __syncthreads();
-  // Hidden layers: each wave owns rows 32 wave .. 32 wave + 31 (it reads and
-  // writes only those rows of act between the block barriers).
-  const int row = wave * 32 + (lane & 31);
-  const int kh = 8 * (lane >> 5);
-  int buf = 0;
-  for (int l = 1; l < g.depth; ++l) {
-    f32x16 acc[NT];
+  // Visits this thread's groups of 4 outputs: (group, row, column, values).
+  auto each = [&](auto f) {
 #pragma unroll
     for (int t = 0; t < NT; ++t)
-      for (int r = 0; r < 16; ++r) acc[t][r] = 0.0f;
 #pragma unroll
-    for (int ch = 0; ch < NC; ++ch) {
-      const bool more = ch + 1 < NC || l + 1 < g.depth;
-      if (more) fetch(ch + 1 < NC ? l : l + 1, ch + 1 < NC ? ch + 1 : 0);
-      __bf16 (*wl)[LD] = reinterpret_cast<__bf16 (*)[LD]>(wbuf + buf * BUFB);
-#pragma unroll 2
-      for (int kc = 0; kc < W / 16; ++kc) {
-        const bf16x8 a = *reinterpret_cast<const bf16x8*>(&act[row][kc * 16 + kh]);
+      for (int q = 0; q < 4; ++q)
 #pragma unroll
-        for (int t = 0; t < TC; ++t) {
-          const bf16x8 b = *reinterpret_cast<const bf16x8*>(&wl[t * 32 + (lane & 31)][kc * 16 + kh]);
-          acc[ch * TC + t] =
-              __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc[ch * TC + t], 0, 0, 0);
-        }
-      }
-      if (more) commit(buf ^ 1);
-      __syncthreads();  // the other buffer is complete; this one is free again
-      buf ^= 1;
-    }
+        for (int m = 0; m < MT; ++m)
+          f((t * 4 + q) * MT + m, m0 + m * 32 + col, n0 + t * 32 + 8 * q + 4 * half,
+            make_float4(acc[m][t][4 * q], acc[m][t][4 * q + 1], acc[m][t][4 * q + 2],
+                        acc[m][t][4 * q + 3]));
+  };
+  auto put = [&](int r, int n, float a, float b, float c, float d) {
+    *reinterpret_cast<uint2*>(act + r * LD + n) = make_uint2(pack2(a, b), pack2(c, d));
+  };
+  auto zslot = [&](int l, int i) { return ((blk * g.depth + l) * C::Q + i) * 256 + tid; };
+  // z = acc + bias, h = gelu(z) of layer l into the activations.
+  auto activate = [&](int l) {
     const float* bl = g.bias + g.boff[l];
+    __syncthreads();  // every wave has read the previous activations
+    each([&](int i, int r, int n, float4 v) {
+      const float4 b = *reinterpret_cast<const float4*>(bl + n);
+      v = make_float4(v.x + b.x, v.y + b.y, v.z + b.z, v.w + b.w);
+      if constexpr (TRAIN) g.z[zslot(l, i)] = v;
+      put(r, n, gelu(v.x), gelu(v.y), gelu(v.z), gelu(v.w));
+    });
+    __syncthreads();
+  };
+
+  // Layer 0 from the split inputs (stored over the activations).
+  const int lx = g.kp + 8;
+  for (int i = tid; i < kRows * g.kp; i += 256) {
+    const int r = i / g.kp, k = i - r * g.kp;
+    const int part = k / g.nin, c = k - part * g.nin;
+    __bf16 v = __bf16(k == 3 * g.nin ? 1.0f : 0.0f);
+    if (part < 3) v = split_part(r < rows ? g.X[(r0 + r) * g.nin + c] : 0.0f, part);
+    act[r * lx + k] = v;
+  }
+  const bf16x8* whid = g.wf + frags_first(W, g.kp) * 64;
+  if (g.depth > 1) prefetch(whid);
+  __syncthreads();
+  clear();
+  for (int kc = 0; kc < g.kp / 16; ++kc) {
+    bf16x8 a[NT];
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const int n = t * 32 + (lane & 31);
-      const float bn = bl[n];
+    for (int t = 0; t < NT; ++t) a[t] = g.wf[((n0 / 32 + t) * (g.kp / 16) + kc) * 64 + lane];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      const bf16x8 b = *reinterpret_cast<const bf16x8*>(act + (m0 + m * 32 + col) * lx + kc * 16 +
+                                                        8 * half);
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        acc[m][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[t], b, acc[m][t], 0, 0, 0);
+    }
+  }
+  if constexpr (TRAIN) transpose_out(act, lx, g.kp / 32, g.xT);
+  activate(0);
+  const int64_t lstride = nchunk * (W / 32) * 64;  // one layer of hT / dzT
+  for (int l = 1; l < g.depth; ++l) {
+    if constexpr (TRAIN) transpose_out(act, LD, W / 32, g.hT + (l - 1) * lstride);
+    product(whid + (l - 1) * frags_hidden(W) * 64);
+    if (l + 1 < g.depth) prefetch(whid + l * frags_hidden(W) * 64);
+    activate(l);
+  }
+  // Last layer: wave w takes the rows 32 w .. 32 w + 31 (4 waves, 4 tiles).
+  f32x16 out;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) out[r] = 0.0f;
+  const bf16x8* wo = whid + (g.depth - 1) * frags_hidden(W) * 64;
+  const int orow = wave * 32 + col;
+#pragma unroll 4
+  for (int kc = 0; kc < KC; ++kc)
+    out = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+        wo[kc * 64 + lane],
+        *reinterpret_cast<const bf16x8*>(act + orow * LD + kc * 16 + 8 * half), out, 0, 0, 0);
+  const float* bo = g.bias + g.boff[g.depth];
+  if constexpr (!TRAIN) {
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {  // n_out <= 16
+      const int o = 8 * (r >> 2) + 4 * half + (r & 3);
+      if (o < g.nout && orow < rows) g.Y[(r0 + orow) * g.nout + o] = out[r] + bo[o];
+    }
+    return;
+  } else {
+    float* dys = reinterpret_cast<float*>(lds + g.dy_lds);
+    double sq[1] = {0.0};
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const int o = 8 * (r >> 2) + 4 * half + (r & 3);
+      if (o >= g.nout) continue;
+      float d = 0.0f;
+      if (orow < rows) d = out[r] + bo[o] - g.T[(r0 + orow) * g.nout + o];
+      dys[orow * g.nout + o] = 2.0f * d * g.scale;
+      sq[0] += double(d) * double(d);
+    }
+    transpose_out(act, LD, W / 32, g.hT + (g.depth - 1) * lstride);
+    const bf16x8* wback = g.wb + (g.depth - 2) * frags_hidden(W) * 64;
+    if (g.depth > 1) prefetch(wback);
+    __shared__ double wsum[16];
+    block_sum<1>(sq, wsum);  // its barriers also publish dys and end the reads of h
+    if (tid == 0) g.loss[blk] = sq[0];
+    {
+      const int tiles = (3 * g.nout + 31) / 32;
+      for (int f = wave; f < tiles * (kRows / 16); f += 4) {
+        const int mc = f / tiles, i = (f - mc * tiles) * 32 + col;
+        const int part = i / g.nout, o = i - part * g.nout;
+        bf16x8 v;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          v[j] = part < 3 ? split_part(dys[(mc * 16 + 8 * half + j) * g.nout + o], part)
+                          : __bf16(0.0f);
+        g.dyT[((blk * (kRows / 16) + mc) * tiles + (f - mc * tiles)) * 64 + lane] = v;
+      }
+    }
+    // dz of the last hidden layer: (dy W_out) gelu'(z).
+    each([&](int i, int r, int n, float4) {
+      float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+      for (int o = 0; o < g.nout; ++o) {
+        const float d = dys[r * g.nout + o];
+        const __bf16* w = g.wlast + int64_t(o) * W + n;
+        s.x += d * float(w[0]);
+        s.y += d * float(w[1]);
+        s.z += d * float(w[2]);
+        s.w += d * float(w[3]);
+      }
+      const float4 z = g.z[zslot(g.depth - 1, i)];
+      put(r, n, s.x * dgelu(z.x), s.y * dgelu(z.y), s.z * dgelu(z.z), s.w * dgelu(z.w));
+    });
+    __syncthreads();
+    for (int l = g.depth - 1; l >= 1; --l) {
+      transpose_out(act, LD, W / 32, g.dzT + l * lstride);
+      product(g.wb + (l - 1) * frags_hidden(W) * 64);
+      if (l > 1) prefetch(g.wb + (l - 2) * frags_hidden(W) * 64);
+      __syncthreads();
+      each([&](int i, int r, int n, float4 v) {
+        const float4 z = g.z[zslot(l - 1, i)];
+        put(r, n, v.x * dgelu(z.x), v.y * dgelu(z.y), v.z * dgelu(z.z), v.w * dgelu(z.w));
+      });
+      __syncthreads();
+    }
+    transpose_out(act, LD, W / 32, g.dzT);
+  }
+}
+
+// Operand fragments of the BF16 weights (see k_mlp_fused): element j of lane
+// l in fragment (t, c) of a matrix A is A[32 t + l % 32][16 c + 8 (l / 32) + j].
+// Layer 0 repeats its columns for the three input parts.
+struct FragArgs {
+  const __bf16* w;
+  int nin, kp, width, depth, nout;
+  int64_t woff[kMaxLayers];
+  bf16x8 *wf, *wb;
+};
+__global__ void k_make_fragments(FragArgs g) {
+  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  const int64_t f = i >> 6;
+  const int lane = int(i & 63), row = lane & 31, k8 = 8 * (lane >> 5);
+  const int W = g.width;
+  const int64_t n0 = frags_first(W, g.kp), nh = frags_hidden(W);
+  const int64_t nf = n0 + (g.depth - 1) * nh + W / 16;
+  bf16x8 v;
+  if (f < n0) {
+    const int t = int(f / (g.kp / 16)), c = int(f - int64_t(t) * (g.kp / 16));
+    const __bf16* w = g.w + g.woff[0] + int64_t(32 * t + row) * g.nin;
+    for (int j = 0; j < 8; ++j) {
+      const int k = 16 * c + k8 + j;
+      v[j] = k < 3 * g.nin ? w[k % g.nin] : __bf16(0.0f);
+    }
+    g.wf[i] = v;
+  } else if (f < nf - W / 16) {
+    const int l = int((f - n0) / nh) + 1;
+    const int q = int((f - n0) - (l - 1) * nh), t = q / (W / 16), c = q - t * (W / 16);
+    const __bf16* w = g.w + g.woff[l];
+    g.wf[i] = *reinterpret_cast<const bf16x8*>(w + int64_t(32 * t + row) * W + 16 * c + k8);
+    for (int j = 0; j < 8; ++j) v[j] = w[int64_t(16 * c + k8 + j) * W + 32 * t + row];
+    g.wb[i - n0 * 64] = v;
+  } else if (f < nf) {
+    const int c = int(f - (nf - W / 16));
+    const __bf16* w = g.w + g.woff[g.depth] + int64_t(row) * W + 16 * c + k8;
+    for (int j = 0; j < 8; ++j) v[j] = row < g.nout ? w[j] : __bf16(0.0f);
+    g.wf[i] = v;
+  }
+}
+
+// All weight and bias gradients of a minibatch: products over the rows of the
+// fragments k_mlp_fused wrote (each 1 KB load feeds an MFMA operand, nothing
+// goes through LDS). One wave per output tile and row split:
+//   64 x 64 tiles of dz_l^T h_{l-1} (hidden layers), then 32 x 32 tiles of
+//   dz_l^T [x | 1] (layer 0's weights; the column of ones gives every
+//   layer's bias gradient) and of dy^T [h | 1] (last layer).
+// Split sums go to hpart / spart and are added in order by k_grad_sum. Splits
+// of 512 rows: 16 k rows at width 256 and depth 4 give 2848 waves.
+struct WgradArgs {
+  int width, depth, kp, nin, nout, ptiles;  // ptiles: 32-column tiles of dyT
+  int64_t nchunk, per_split;                // 16-row chunks, chunks per split
+  const bf16x8 *hT, *dzT, *xT, *dyT;
+  float* hpart;  // [split][l - 1][width][width]
+  float* spart;  // [split][small tile][32][32]
+};
+__host__ __device__ inline int wgrad_big(int width, int depth) {
+  return (depth - 1) * (width / 64) * (width / 64);
+}
+// Small tiles: (l = 0: width/32 x kp/32), (l >= 1: width/32), (dy: ptiles x
+// width/32), (dy bias: ptiles).
+__host__ __device__ inline int wgrad_small(int width, int depth, int kp, int ptiles) {
+  return (width / 32) * (kp / 32) + (depth - 1) * (width / 32) + ptiles * (width / 32) + ptiles;
+}
+
+template <int TA, int TB>
+__device__ __forceinline__ void wgrad_tile(const bf16x8* __restrict__ A, int64_t sa,
+                                           const bf16x8* __restrict__ B, int64_t sb, int64_t c0,
+                                           int64_t c1, int lane, float* __restrict__ out, int ld) {
+  f32x16 acc[TA][TB];
+#pragma unroll
+  for (int a = 0; a < TA; ++a)
+#pragma unroll
+    for (int b = 0; b < TB; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.0f;
+  for (int64_t c = c0; c < c1; ++c) {
+    bf16x8 av[TA], bv[TB];
+#pragma unroll
+    for (int a = 0; a < TA; ++a) av[a] = A[(c * sa + a) * 64 + lane];
+#pragma unroll
+    for (int b = 0; b < TB; ++b) bv[b] = B[(c * sb + b) * 64 + lane];
+#pragma unroll
+    for (int a = 0; a < TA; ++a)
+#pragma unroll
+      for (int b = 0; b < TB; ++b)
+        acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[a], bv[b], acc[a][b], 0, 0, 0);
+  }
+#pragma unroll
+  for (int a = 0; a < TA; ++a)
+#pragma unroll
+    for (int b = 0; b < TB; ++b)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int i = 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        act[wave * 32 + i][n] = __bf16(gelu(acc[t][r] + bn));
+        const int i = 32 * a + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+        out[int64_t(i) * ld + 32 * b + (lane & 31)] = acc[a][b][r];
+      }
+}
+
+__global__ __launch_bounds__(256) void k_wgrad(WgradArgs g) {
+  const int lane = threadIdx.x & 63;
+  int job = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int W = g.width, wt = W / 32;
+  const int big = wgrad_big(W, g.depth), small = wgrad_small(W, g.depth, g.kp, g.ptiles);
+  if (job >= big + small) return;
+  const int64_t split = blockIdx.y;
+  const int64_t c0 = split * g.per_split, c1 = min(g.nchunk, c0 + g.per_split);
+  const int64_t ls = g.nchunk * wt * 64;
+  if (job < big) {
+    const int per = (W / 64) * (W / 64);
+    const int l = job / per + 1, q = job - (l - 1) * per, ti = q / (W / 64), tj = q - ti * (W / 64);
+    float* out = g.hpart + ((split * (g.depth - 1) + l - 1) * W + 64 * ti) * W + 64 * tj;
+    wgrad_tile<2, 2>(g.dzT + l * ls + 2 * ti * 64, wt, g.hT + (l - 1) * ls + 2 * tj * 64, wt, c0,
+                     c1, lane, out, W);
+    return;
+  }
+  job -= big;
+  float* out = g.spart + (split * small + job) * 1024;
+  const int xt = g.kp / 32, ones = 3 * g.nin / 32;
+  const bf16x8 *A, *B;
+  int64_t sa, sb;
+  if (job < wt * xt) {
+    A = g.dzT + (job / xt) * 64, sa = wt;
+    B = g.xT + (job % xt) * 64, sb = xt;
+  } else if ((job -= wt * xt) < (g.depth - 1) * wt) {
+    A = g.dzT + (1 + job / wt) * ls + (job % wt) * 64, sa = wt;
+    B = g.xT + ones * 64, sb = xt;
+  } else if ((job -= (g.depth - 1) * wt) < g.ptiles * wt) {
+    A = g.dyT + (job / wt) * 64, sa = g.ptiles;
+    B = g.hT + (g.depth - 1) * ls + (job % wt) * 64, sb = wt;
+  } else {
+    job -= g.ptiles * wt;
+    A = g.dyT + job * 64, sa = g.ptiles;
+    B = g.xT + ones * 64, sb = xt;
+  }
+  wgrad_tile<1, 1>(A, sa, B, sb, c0, c1, lane, out, 32);
+}
+
+// Gradient of parameter i (layout of the parameter vector): the split sums
+// of its tile in split order, the three parts of a split operand together.
+struct GradSumArgs {
+  WgradArgs w;
+  int splits;
+  int64_t nweights, nparams;
+  int64_t woff[kMaxLayers], boff[kMaxLayers];
+  float* grad;
+};
+__global__ void k_grad_sum(GradSumArgs g) {
+  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= g.nparams) return;
+  const int W = g.w.width, D = g.w.depth, wt = W / 32, xt = g.w.kp / 32, nin = g.w.nin,
+            nout = g.w.nout, pt = g.w.ptiles;
+  const int small = wgrad_small(W, D, g.w.kp, pt);
+  const int j1 = wt * xt, j2 = j1 + (D - 1) * wt, j3 = j2 + pt * wt;
+  const int ones = 3 * nin;
+  const bool is_bias = i >= g.nweights;
+  const int64_t q = is_bias ? i - g.nweights : i;
+  const int64_t* off = is_bias ? g.boff : g.woff;
+  int l = 0;
+  while (l < D && q >= off[l + 1]) ++l;
+  const int64_t e = q - off[l];
+  float s = 0.0f;
+  if (!is_bias && l > 0 && l < D) {
+    const float* p = g.w.hpart + int64_t(l - 1) * W * W + e;
+    const int64_t st = int64_t(D - 1) * W * W;
+#pragma unroll 8
+    for (int z = 0; z < g.splits; ++z) s += p[z * st];
+  } else {
+    // Up to three entries of the small tiles.
+    int64_t at[3];
+    int parts = 3;
+    if (!is_bias && l == 0) {
+      const int n = int(e / nin), c = int(e - int64_t(n) * nin);
+      for (int p = 0; p < 3; ++p) {
+        const int k = p * nin + c;
+        at[p] = int64_t((n / 32) * xt + k / 32) * 1024 + (n % 32) * 32 + k % 32;
+      }
+    } else if (!is_bias) {
+      const int o = int(e / W), k = int(e - int64_t(o) * W);
+      for (int p = 0; p < 3; ++p) {
+        const int r = p * nout + o;
+        at[p] = int64_t(j2 + (r / 32) * wt + k / 32) * 1024 + (r % 32) * 32 + k % 32;
+      }
+    } else if (l < D) {
+      const int n = int(e);
+      const int job = l == 0 ? (n / 32) * xt + ones / 32 : j1 + (l - 1) * wt + n / 32;
+      at[0] = int64_t(job) * 1024 + (n % 32) * 32 + ones % 32;
+      parts = 1;
+    } else {
+      for (int p = 0; p < 3; ++p) {
+        const int r = p * nout + int(e);
+        at[p] = int64_t(j3 + r / 32) * 1024 + (r % 32) * 32 + ones % 32;
       }
     }
-  }
-  __syncthreads();
-  // Last layer: W -> n_out, FP32 dot products over k in order (16-byte loads
-  // of activations and weights).
-  const int L = g.depth;
-  for (int i = tid; i < kInferRows * g.nout; i += 256) {
-    const int r = i / g.nout, o = i - r * g.nout;
-    if (r >= rows) continue;
-    const __bf16* wo = g.w + g.woff[L] + int64_t(o) * W;
-    float s = g.bias[g.boff[L] + o];
-    for (int k8 = 0; k8 < W / 8; ++k8) {
-      const bf16x8 av = *reinterpret_cast<const bf16x8*>(&act[r][k8 * 8]);
-      const bf16x8 wv = *reinterpret_cast<const bf16x8*>(wo + k8 * 8);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) s += float(av[e]) * float(wv[e]);
+    for (int z = 0; z < g.splits; ++z) {
+      const float* p = g.w.spart + int64_t(z) * small * 1024;
+      float v = p[at[0]];
+      if (parts == 3) v += p[at[1]] + p[at[2]];
+      s += v;
     }
-    g.Y[(r0 + r) * g.nout + o] = s;
   }
+  g.grad[i] = s;
 }
 
 unsigned g1(int64_t n, int b = 256) { return grid_for(n, b); }
@@ -502,7 +861,7 @@ void Mlp::init(int nin_, int width_, int depth_, int nout_, uint64_t seed) {
   m2.alloc(nparams);
   m2.zero(s);
   wbf.alloc(nweights);
-  k_f32_to_bf16<<<g1(nweights), 256, 0, s>>>(master.p, nweights, wbf.p);
+  sync_bf16(s);
   steps = 0;
   NOSH_HIP(hipStreamSynchronize(s));
 }
@@ -552,7 +911,152 @@ void Mlp::gemm(const __bf16* A, int64_t sam, int64_t sak, const __bf16* B, int64
   k_gemm_bf16<<<grid, 256, 0, s>>>(g);
 }
 
+// ------------------------------------------------ fused path (host side)
+bool Mlp::fused() const {
+  return (width == 64 || width == 128 || width == 256) && nin <= kFusedMaxIn;
+}
+
+namespace {
+
+int split_cols(int nin) { return (3 * nin + 1 + 31) / 32 * 32; }
+
+template <int W>
+size_t fused_lds(int kp, int nout, bool train, int* dy_off) {
+  const size_t a = size_t(kRows) * Tiling<W>::LD * 2, x = size_t(kRows) * (kp + 8) * 2;
+  const size_t top = std::max(a, x);
+  *dy_off = int(top);
+  return top + (train ? size_t(kRows) * nout * 4 : 0);
+}
+
+template <int W, bool TRAIN>
+void launch_fused(FusedArgs g, hipStream_t s) {
+  const size_t lds = fused_lds<W>(g.kp, g.nout, TRAIN, &g.dy_lds);
+  // More than the 64 KB a kernel may use by default at width 256.
+  static const hipError_t attr = hipFuncSetAttribute(
+      reinterpret_cast<const void*>(k_mlp_fused<W, TRAIN>),
+      hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
+  NOSH_HIP(attr);
+  const unsigned nb = unsigned((g.M + kRows - 1) / kRows);
+  k_mlp_fused<W, TRAIN><<<nb, 256, lds, s>>>(g);
+}
+
+template <bool TRAIN>
+void launch_fused_width(int width, const FusedArgs& g, hipStream_t s) {
+  if (width == 256)
+    launch_fused<256, TRAIN>(g, s);
+  else if (width == 128)
+    launch_fused<128, TRAIN>(g, s);
+  else
+    launch_fused<64, TRAIN>(g, s);
+}
+
+FusedArgs fused_args(const Mlp& n, const float* X, int64_t M) {
+  FusedArgs g{};
+  g.X = X;
+  g.M = M;
+  g.nin = n.nin;
+  g.kp = split_cols(n.nin);
+  g.depth = n.depth;
+  g.nout = n.nout;
+  g.wf = reinterpret_cast<const bf16x8*>(n.wfrag.p);
+  g.wb = reinterpret_cast<const bf16x8*>(n.wfrag_t.p);
+  g.wlast = n.wbf.p + n.woff[n.depth];
+  g.bias = n.master.p + n.nweights;
+  for (int l = 0; l <= n.depth; ++l) g.boff[l] = n.boff[l];
+  return g;
+}
+
+}  // namespace
+
+void Mlp::make_fragments(hipStream_t s) {
+  if (!fused()) return;
+  const int kp = split_cols(nin);
+  const int64_t nf = frags_first(width, kp) + (depth - 1) * frags_hidden(width) + width / 16;
+  if (!wfrag.p) {
+    wfrag.alloc(nf * kFrag);
+    wfrag_t.alloc(std::max<int64_t>(1, (depth - 1) * frags_hidden(width)) * kFrag);
+  }
+  FragArgs g{};
+  g.w = wbf.p;
+  g.nin = nin;
+  g.kp = kp;
+  g.width = width;
+  g.depth = depth;
+  g.nout = nout;
+  for (int l = 0; l <= depth; ++l) g.woff[l] = woff[l];
+  g.wf = reinterpret_cast<bf16x8*>(wfrag.p);
+  g.wb = reinterpret_cast<bf16x8*>(wfrag_t.p);
+  k_make_fragments<<<g1(nf * 64), 256, 0, s>>>(g);
+}
+
+void Mlp::ensure_fused(int64_t M) {
+  if (M <= fcap) return;
+  fcap = M;
+  const int64_t nb = (M + kRows - 1) / kRows, mp = nb * kRows;
+  const int64_t pt = (3 * nout + 31) / 32;
+  zs.alloc(mp * width * depth);
+  hT.alloc(mp * width * depth);
+  dzT.alloc(mp * width * depth);
+  xT.alloc(mp * split_cols(nin));
+  dyT.alloc(mp * pt * 32);
+  partials.alloc(nb + 64);
+  if (!loss.p) loss.alloc(1);
+}
+
+void Mlp::gradients_fused(const float* X, const float* T, int64_t M, hipStream_t s) {
+  ensure_fused(M);
+  const unsigned nb = unsigned((M + kRows - 1) / kRows);
+  FusedArgs g = fused_args(*this, X, M);
+  g.T = T;
+  g.scale = 1.0f / float(M * nout);
+  g.z = reinterpret_cast<float4*>(zs.p);
+  g.hT = reinterpret_cast<bf16x8*>(hT.p);
+  g.dzT = reinterpret_cast<bf16x8*>(dzT.p);
+  g.xT = reinterpret_cast<bf16x8*>(xT.p);
+  g.dyT = reinterpret_cast<bf16x8*>(dyT.p);
+  g.loss = partials.p;
+  launch_fused_width<true>(width, g, s);
+  k_finalize1<<<1, 256, 0, s>>>(partials.p, int(nb), 1.0 / double(M * nout), loss.p);
+  GradSumArgs r{};
+  WgradArgs& w = r.w;
+  w.width = width;
+  w.depth = depth;
+  w.kp = g.kp;
+  w.nin = nin;
+  w.nout = nout;
+  w.ptiles = (3 * nout + 31) / 32;
+  w.nchunk = int64_t(nb) * (kRows / 16);
+  // 512 rows a split, at most 64 splits.
+  w.per_split = std::max<int64_t>(32, (w.nchunk + 63) / 64);
+  r.splits = int((w.nchunk + w.per_split - 1) / w.per_split);
+  const int big = wgrad_big(width, depth), small = wgrad_small(width, depth, w.kp, w.ptiles);
+  const size_t nh = size_t(r.splits) * (depth - 1) * width * width;
+  const size_t need = nh + size_t(r.splits) * small * 1024;
+  if (red.n < need) red.alloc(need);
+  w.hT = g.hT;
+  w.dzT = g.dzT;
+  w.xT = g.xT;
+  w.dyT = g.dyT;
+  w.hpart = red.p;
+  w.spart = red.p + nh;
+  k_wgrad<<<dim3(unsigned((big + small + 3) / 4), unsigned(r.splits)), 256, 0, s>>>(w);
+  r.nweights = nweights;
+  r.nparams = nparams;
+  for (int l = 0; l <= depth; ++l) {
+    r.woff[l] = woff[l];
+    r.boff[l] = boff[l];
+  }
+  r.grad = grad.p;
+  k_grad_sum<<<g1(nparams), 256, 0, s>>>(r);
+}
+
 void Mlp::forward(const float* X, int64_t M, float* Y, hipStream_t s, bool keep_pre) {
+  if (fused() && !keep_pre) {
+    FusedArgs g = fused_args(*this, X, M);
+    g.Y = Y;
+    launch_fused_width<false>(width, g, s);
+    return;
+  }
   ensure(M);
   const int L = int(dims.size()) - 1;
   k_layer_in<<<g1(M * dims[1]), 256, 0, s>>>(X, M, nin, wbf.p + woff[0], bias(0), dims[1],
@@ -567,35 +1071,13 @@ void Mlp::forward(const float* X, int64_t M, float* Y, hipStream_t s, bool keep_
 }
 
 void Mlp::infer(const float* X, int64_t M, float* Y, hipStream_t s) {
-  const int nt = width / 32;
-  if (width % 32 != 0 || (nt != 2 && nt != 4 && nt != 8) || nin > kInferMaxIn ||
-      depth + 1 > kInferMaxLayers) {
-    constexpr int64_t kChunk = 1 << 19;
-    for (int64_t r0 = 0; r0 < M; r0 += kChunk)
-      forward(X + r0 * nin, std::min(kChunk, M - r0), Y + r0 * nout, s, false);
+  if (fused()) {
+    forward(X, M, Y, s, false);
     return;
   }
-  InferArgs g{};
-  g.X = X;
-  g.M = M;
-  g.nin = nin;
-  g.width = width;
-  g.depth = depth;
-  g.nout = nout;
-  g.w = wbf.p;
-  g.bias = master.p + nweights;
-  for (int l = 0; l <= depth; ++l) {
-    g.woff[l] = woff[l];
-    g.boff[l] = boff[l];
-  }
-  g.Y = Y;
-  const unsigned nb = unsigned((M + kInferRows - 1) / kInferRows);
-  if (nt == 8)
-    k_mlp_infer<8><<<nb, 256, 0, s>>>(g);
-  else if (nt == 4)
-    k_mlp_infer<4><<<nb, 256, 0, s>>>(g);
-  else
-    k_mlp_infer<2><<<nb, 256, 0, s>>>(g);
+  constexpr int64_t kChunk = 1 << 19;
+  for (int64_t r0 = 0; r0 < M; r0 += kChunk)
+    forward(X + r0 * nin, std::min(kChunk, M - r0), Y + r0 * nout, s, false);
 }
 
 double Mlp::last_loss(hipStream_t s) {
@@ -606,6 +1088,10 @@ double Mlp::last_loss(hipStream_t s) {
 }
 
 double Mlp::gradients(const float* X, const float* T, int64_t M, hipStream_t s, bool read_loss) {
+  if (fused()) {
+    gradients_fused(X, T, M, s);
+    return read_loss ? last_loss(s) : std::numeric_limits<double>::quiet_NaN();
+  }
   ensure(M);
   forward(X, M, y.p, s);
   const int L = int(dims.size()) - 1;
@@ -687,10 +1173,12 @@ void Mlp::adam(float lr, hipStream_t s) {
   k_adam<<<g1(nparams - nweights), 256, 0, s>>>(master.p + nweights, grad.p + nweights,
                                                 m1.p + nweights, m2.p + nweights, nullptr,
                                                 nparams - nweights, lr, b1, b2, eps, c1, c2);
+  make_fragments(s);
 }
 
 void Mlp::sync_bf16(hipStream_t s) {
   k_f32_to_bf16<<<g1(nweights), 256, 0, s>>>(master.p, nweights, wbf.p);
+  make_fragments(s);
 }
 
 namespace {

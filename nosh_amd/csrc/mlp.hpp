@@ -24,6 +24,13 @@ struct Mlp {
   DBuf<__bf16> dzb, dza;
   DBuf<float> y, dy, red;
   DBuf<double> partials, loss;
+  // Fused path: operand fragments of the weights (and of the transposed
+  // hidden ones), and one minibatch's pre-activations and row fragments
+  // (capacity fcap rows).
+  DBuf<__bf16> wfrag, wfrag_t;
+  int64_t fcap = 0;
+  DBuf<float> zs;
+  DBuf<__bf16> hT, dzT, xT, dyT;
 
   void init(int nin, int width, int depth, int nout, uint64_t seed);
   void ensure(int64_t M);
@@ -31,7 +38,13 @@ struct Mlp {
   void gemm(const __bf16* A, int64_t sam, int64_t sak, const __bf16* B, int64_t sbk, int64_t sbn,
             int64_t M, int64_t N, int64_t K, int epi, const float* bias, const float* zin,
             float* outf, __bf16* outb, int splits, hipStream_t s);
-  // keep_pre: store the hidden pre-activations (needed by gradients()).
+  // Whether this shape takes the fused kernels.
+  bool fused() const;
+  void make_fragments(hipStream_t s);
+  void ensure_fused(int64_t M);
+  void gradients_fused(const float* X, const float* T, int64_t M, hipStream_t s);
+  // keep_pre: layer by layer, storing the hidden pre-activations (needed by
+  // gradients() of the shapes that are not fused).
   void forward(const float* X, int64_t M, float* Y, hipStream_t s, bool keep_pre = true);
   // Inference only (no stored activations): the fused one-kernel network for
   // width 64, 128 or 256 and n_in <= 32, else forward() in row chunks.

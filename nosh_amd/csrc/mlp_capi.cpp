@@ -70,7 +70,7 @@ int nosh_mlp_set_params(nosh_mlp_t mlp, const float* params) {
 int nosh_mlp_forward_device(nosh_mlp_t mlp, const float* X, int64_t M, float* Y, void* stream) {
   return mguard([&] {
     NOSH_CHECK(mlp && X && Y && M >= 1, kInvalid, "invalid argument");
-    mlp->net.forward(X, M, Y, stream ? static_cast<hipStream_t>(stream) : default_stream());
+    mlp->net.forward(X, M, Y, stream ? static_cast<hipStream_t>(stream) : default_stream(), false);
   });
 }
 
@@ -82,7 +82,7 @@ int nosh_mlp_forward(nosh_mlp_t mlp, const float* X, int64_t M, float* Y) {
     if (mlp->x.n < size_t(M * n.nin)) mlp->x.alloc(M * n.nin);
     if (mlp->y.n < size_t(M * n.nout)) mlp->y.alloc(M * n.nout);
     mlp->x.upload(X, M * n.nin, s);
-    n.forward(mlp->x.p, M, mlp->y.p, s);
+    n.forward(mlp->x.p, M, mlp->y.p, s, false);
     mlp->y.download(Y, M * n.nout, s);
     NOSH_HIP(hipStreamSynchronize(s));
   });

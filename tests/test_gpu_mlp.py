@@ -119,3 +119,30 @@ def test_first_adam_step_closed_form():
     big = np.abs(g) > 1e-5
     assert big.sum() > 0.9 * g.size
     np.testing.assert_allclose(d[big], -lr * np.sign(g[big]), rtol=0, atol=2e-3 * lr + 1e-6)
+
+
+@pytest.mark.parametrize("nin,width,depth,nout,M", [
+    (1, 64, 1, 1, 1), (7, 64, 2, 2, 127), (10, 128, 3, 2, 128), (11, 128, 2, 3, 129),
+    (21, 256, 2, 11, 257), (32, 256, 3, 16, 500), (9, 256, 4, 2, 40000)])
+def test_fused_network_shapes(nin, width, depth, nout, M):
+    """The fused kernels at the edges of their tiles: rows around the 128-row
+    workgroups and the 512-row gradient splits, inputs around the 32-column
+    tiles of their three-part split (3 n_in + 1 = 31, 34, 64, 97), one hidden
+    layer, and outputs on both sides of one 32-row tile of 3 n_out."""
+    net = _net(nin=nin, width=width, depth=depth, nout=nout, seed=9)
+    rng = np.random.default_rng(12)
+    p = net.get_params()
+    p[net.nweights:] = rng.uniform(-0.2, 0.2, net.nparams - net.nweights)
+    net.set_params(p)
+    X = rng.normal(0, 1, (M, nin)).astype(np.float32)
+    T = rng.normal(0, 1, (M, nout)).astype(np.float32)
+    y_bf, _, _ = MO.forward(p, X, net.dims, bf=True)
+    assert np.linalg.norm(net.infer(X) - y_bf) / np.linalg.norm(y_bf) < 5e-3
+    loss, g = net.gradients(X, T)
+    loss_ref, g_ref = MO.loss_and_grad(p, X, T, net.dims, bf=True)
+    assert abs(loss - loss_ref) / loss_ref < 5e-3
+    off = 0
+    for size in [a * b for a, b in zip(net.dims[:-1], net.dims[1:])] + net.dims[1:]:
+        s = slice(off, off + size)
+        assert np.linalg.norm(g[s] - g_ref[s]) / np.linalg.norm(g_ref[s]) < 2e-2
+        off += size
