@@ -281,8 +281,8 @@ __global__ void k_bf16_to_f32(const __bf16* __restrict__ a, int64_t n, float* __
 }
 
 __global__ void k_adam(float* __restrict__ w, const float* __restrict__ gr, float* __restrict__ m,
-                       float* __restrict__ v, __bf16* __restrict__ wb, int64_t n, float lr,
-                       float b1, float b2, float eps, float c1, float c2) {
+                       float* __restrict__ v, __bf16* __restrict__ wb, int64_t nwb, int64_t n,
+                       float lr, float b1, float b2, float eps, float c1, float c2) {
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const float g = gr[i];
@@ -292,7 +292,7 @@ __global__ void k_adam(float* __restrict__ w, const float* __restrict__ gr, floa
   v[i] = vi;
   const float wi = w[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
   w[i] = wi;
-  if (wb) wb[i] = __bf16(wi);
+  if (i < nwb) wb[i] = __bf16(wi);  // the weights; biases stay FP32
 }
 
 __global__ void k_f32_to_bf16(const float* __restrict__ a, int64_t n, __bf16* __restrict__ b) {
@@ -301,8 +301,8 @@ __global__ void k_f32_to_bf16(const float* __restrict__ a, int64_t n, __bf16* __
 }
 
 // ------------------------------------------------------- fused network
-// Widths 64, 128 and 256 with n_in <= 32: the whole network for 128 rows in
-// one workgroup of 4 waves, the activations (BF16) in LDS between layers,
+// Widths 64, 128 and 256 with n_in <= 32: the whole network for R = 128, 64 or
+// 32 rows in one workgroup of 4 waves, the activations (BF16) in LDS between layers,
 // every layer on MFMA with FP32 accumulation; in training the same kernel
 // goes on to the loss and back through the layers.
 //
@@ -326,7 +326,6 @@ __global__ void k_f32_to_bf16(const float* __restrict__ a, int64_t n, __bf16* __
 // (x = x1 + x2 + x3 exactly), times the same BF16 weight: exact products,
 // FP32 sums, as the scalar form. The same split serves dy and x in the
 // weight gradients.
-constexpr int kRows = 128;
 constexpr int kFusedMaxIn = 32;
 constexpr int kMaxLayers = 18;
 constexpr int kFrag = 512;  // bf16 per operand fragment
@@ -382,20 +381,23 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {
   return v.u;
 }
 
-template <int W>
+template <int W, int R>
 struct Tiling {
   static constexpr int NT = W >= 256 ? 2 : 1;   // 32-column tiles per wave
   static constexpr int WN = W / (32 * NT);      // waves along the columns
-  static constexpr int MT = 4 / (4 / WN);       // 32-row tiles per wave
+  static constexpr int MT = R * WN / 128;       // 32-row tiles per wave
   static constexpr int LD = W + 8;              // padded LDS row (bf16): no bank conflicts
   static constexpr int KC = W / 16;             // k-steps of a hidden layer
   static constexpr int Q = MT * NT * 4;         // groups of 4 outputs per thread
+  static_assert(MT >= 1, "a wave needs a row tile");
 };
 
-// Workgroups a CU holds by LDS: 2 at width 256, 4 below.
-template <int W, bool TRAIN>
-__global__ __launch_bounds__(256, W >= 256 ? 2 : TRAIN && W >= 128 ? 3 : 4) void k_mlp_fused(FusedArgs g) {
-  using C = Tiling<W>;
+// Workgroups a CU holds by LDS: 2 at 128 rows of width 256, 4 below.
+template <int W, int R, bool TRAIN>
+__global__ __launch_bounds__(256, W * R >= 256 * 128 ? 2 : TRAIN && W * R >= 128 * 128 ? 3 : 4) void
+k_mlp_fused(FusedArgs g) {
+  using C = Tiling<W, R>;
+  constexpr int kRows = R;
   constexpr int NT = C::NT, MT = C::MT, LD = C::LD, KC = C::KC, G = 4;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   __bf16* act = reinterpret_cast<__bf16*>(lds);  // [kRows][LD]; first the split inputs
@@ -523,23 +525,26 @@ __global__ __launch_bounds__(256, W >= 256 ? 2 : TRAIN && W >= 128 ? 3 : 4) void
     if (l + 1 < g.depth) prefetch(whid + l * frags_hidden(W) * 64);
     activate(l);
   }
-  // Last layer: wave w takes the rows 32 w .. 32 w + 31 (4 waves, 4 tiles).
+  // Last layer: wave w takes the rows 32 w .. 32 w + 31 while there are any.
+  const bool owave = wave < kRows / 32;
   f32x16 out;
 #pragma unroll
   for (int r = 0; r < 16; ++r) out[r] = 0.0f;
   const bf16x8* wo = whid + (g.depth - 1) * frags_hidden(W) * 64;
   const int orow = wave * 32 + col;
+  if (owave) {
 #pragma unroll 4
-  for (int kc = 0; kc < KC; ++kc)
-    out = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-        wo[kc * 64 + lane],
-        *reinterpret_cast<const bf16x8*>(act + orow * LD + kc * 16 + 8 * half), out, 0, 0, 0);
+    for (int kc = 0; kc < KC; ++kc)
+      out = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+          wo[kc * 64 + lane],
+          *reinterpret_cast<const bf16x8*>(act + orow * LD + kc * 16 + 8 * half), out, 0, 0, 0);
+  }
   const float* bo = g.bias + g.boff[g.depth];
   if constexpr (!TRAIN) {
 #pragma unroll
     for (int r = 0; r < 8; ++r) {  // n_out <= 16
       const int o = 8 * (r >> 2) + 4 * half + (r & 3);
-      if (o < g.nout && orow < rows) g.Y[(r0 + orow) * g.nout + o] = out[r] + bo[o];
+      if (o < g.nout && orow < rows && owave) g.Y[(r0 + orow) * g.nout + o] = out[r] + bo[o];
     }
     return;
   } else {
@@ -548,7 +553,7 @@ __global__ __launch_bounds__(256, W >= 256 ? 2 : TRAIN && W >= 128 ? 3 : 4) void
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
       const int o = 8 * (r >> 2) + 4 * half + (r & 3);
-      if (o >= g.nout) continue;
+      if (o >= g.nout || !owave) continue;
       float d = 0.0f;
       if (orow < rows) d = out[r] + bo[o] - g.T[(r0 + orow) * g.nout + o];
       dys[orow * g.nout + o] = 2.0f * d * g.scale;
@@ -703,11 +708,16 @@ __device__ __forceinline__ void wgrad_tile(const bf16x8* __restrict__ A, int64_t
 
 __global__ __launch_bounds__(256) void k_wgrad(WgradArgs g) {
   const int lane = threadIdx.x & 63;
-  int job = blockIdx.x * 4 + (threadIdx.x >> 6);
   const int W = g.width, wt = W / 32;
   const int big = wgrad_big(W, g.depth), small = wgrad_small(W, g.depth, g.kp, g.ptiles);
+  // One split's workgroups run on one XCD, whose L2 then reads its rows once
+  // (spread over all eight, 16 k rows took 32 us; now 20). Loading four
+  // chunks ahead measured slower (26 us, 202 registers).
+  const int per_split_blocks = (big + small + 3) / 4;
+  const int64_t logical = xcd_block(true);
+  const int64_t split = logical / per_split_blocks;
+  int job = int(logical - split * per_split_blocks) * 4 + (threadIdx.x >> 6);
   if (job >= big + small) return;
-  const int64_t split = blockIdx.y;
   const int64_t c0 = split * g.per_split, c1 = min(g.nchunk, c0 + g.per_split);
   const int64_t ls = g.nchunk * wt * 64;
   if (job < big) {
@@ -748,8 +758,18 @@ struct GradSumArgs {
   int64_t nweights, nparams;
   int64_t woff[kMaxLayers], boff[kMaxLayers];
   float* grad;
+  const double* loss_part;  // nloss partial sums; the last workgroup adds them
+  int nloss;
+  double loss_scale;
+  double* loss;
 };
 __global__ void k_grad_sum(GradSumArgs g) {
+  if (blockIdx.x + 1 == gridDim.x) {
+    double v[1];
+    finalize_sum<1>(v, g.loss_part, g.nloss);
+    if (threadIdx.x == 0) *g.loss = v[0] * g.loss_scale;
+    return;
+  }
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= g.nparams) return;
   const int W = g.w.width, D = g.w.depth, wt = W / 32, xt = g.w.kp / 32, nin = g.w.nin,
@@ -767,7 +787,7 @@ __global__ void k_grad_sum(GradSumArgs g) {
   if (!is_bias && l > 0 && l < D) {
     const float* p = g.w.hpart + int64_t(l - 1) * W * W + e;
     const int64_t st = int64_t(D - 1) * W * W;
-#pragma unroll 8
+#pragma unroll 16
     for (int z = 0; z < g.splits; ++z) s += p[z * st];
   } else {
     // Up to three entries of the small tiles.
@@ -796,11 +816,12 @@ __global__ void k_grad_sum(GradSumArgs g) {
         at[p] = int64_t(j3 + r / 32) * 1024 + (r % 32) * 32 + ones % 32;
       }
     }
+    if (parts == 1) at[1] = at[2] = at[0];
+#pragma unroll 8
     for (int z = 0; z < g.splits; ++z) {
       const float* p = g.w.spart + int64_t(z) * small * 1024;
-      float v = p[at[0]];
-      if (parts == 3) v += p[at[1]] + p[at[2]];
-      s += v;
+      const float v1 = p[at[0]], v2 = p[at[1]], v3 = p[at[2]];
+      s += parts == 1 ? v1 : v1 + (v2 + v3);
     }
   }
   g.grad[i] = s;
@@ -920,34 +941,49 @@ namespace {
 
 int split_cols(int nin) { return (3 * nin + 1 + 31) / 32 * 32; }
 
-template <int W>
-size_t fused_lds(int kp, int nout, bool train, int* dy_off) {
-  const size_t a = size_t(kRows) * Tiling<W>::LD * 2, x = size_t(kRows) * (kp + 8) * 2;
-  const size_t top = std::max(a, x);
-  *dy_off = int(top);
-  return top + (train ? size_t(kRows) * nout * 4 : 0);
+template <int W, int R, bool TRAIN>
+void launch_fused(FusedArgs g, hipStream_t s) {
+  const size_t top = std::max(size_t(R) * Tiling<W, R>::LD * 2, size_t(R) * (g.kp + 8) * 2);
+  const size_t lds = top + (TRAIN ? size_t(R) * g.nout * 4 : 0);
+  g.dy_lds = int(top);
+  // More than the 64 KB a kernel may use by default at 128 rows of width 256.
+  static const hipError_t attr = hipFuncSetAttribute(
+      reinterpret_cast<const void*>(k_mlp_fused<W, R, TRAIN>),
+      hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
+  NOSH_HIP(attr);
+  k_mlp_fused<W, R, TRAIN><<<unsigned((g.M + R - 1) / R), 256, lds, s>>>(g);
+}
+
+// Rows per workgroup: the largest that still gives every CU of the chip a
+// workgroup (128-row ones read each weight half as often as 64-row ones, but
+// leave CUs idle below 32 k rows: a training pass over 16,384 rows of width
+// 256 took 146 us with 128 of them and 84 us with 256). A wave needs a
+// 32-row tile of its own, which sets the least at width 64.
+int fused_rows(int width, int64_t M) {
+  const int64_t cus = 256;
+  if ((M + 127) / 128 >= cus) return 128;
+  if (width == 64 || (M + 63) / 64 >= cus) return 64;
+  return 32;
 }
 
 template <int W, bool TRAIN>
-void launch_fused(FusedArgs g, hipStream_t s) {
-  const size_t lds = fused_lds<W>(g.kp, g.nout, TRAIN, &g.dy_lds);
-  // More than the 64 KB a kernel may use by default at width 256.
-  static const hipError_t attr = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(k_mlp_fused<W, TRAIN>),
-      hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
-  NOSH_HIP(attr);
-  const unsigned nb = unsigned((g.M + kRows - 1) / kRows);
-  k_mlp_fused<W, TRAIN><<<nb, 256, lds, s>>>(g);
+void launch_fused_rows(int rows, const FusedArgs& g, hipStream_t s) {
+  if (rows == 128)
+    launch_fused<W, 128, TRAIN>(g, s);
+  else if (rows == 64)
+    launch_fused<W, 64, TRAIN>(g, s);
+  else if constexpr (W > 64)
+    launch_fused<W, 32, TRAIN>(g, s);
 }
 
 template <bool TRAIN>
-void launch_fused_width(int width, const FusedArgs& g, hipStream_t s) {
+void launch_fused_width(int width, int rows, const FusedArgs& g, hipStream_t s) {
   if (width == 256)
-    launch_fused<256, TRAIN>(g, s);
+    launch_fused_rows<256, TRAIN>(rows, g, s);
   else if (width == 128)
-    launch_fused<128, TRAIN>(g, s);
+    launch_fused_rows<128, TRAIN>(rows, g, s);
   else
-    launch_fused<64, TRAIN>(g, s);
+    launch_fused_rows<64, TRAIN>(rows, g, s);
 }
 
 FusedArgs fused_args(const Mlp& n, const float* X, int64_t M) {
@@ -992,20 +1028,21 @@ void Mlp::make_fragments(hipStream_t s) {
 void Mlp::ensure_fused(int64_t M) {
   if (M <= fcap) return;
   fcap = M;
-  const int64_t nb = (M + kRows - 1) / kRows, mp = nb * kRows;
+  const int64_t mp = (M + 127) / 128 * 128;  // covers every rows-per-workgroup choice below M too
   const int64_t pt = (3 * nout + 31) / 32;
   zs.alloc(mp * width * depth);
   hT.alloc(mp * width * depth);
   dzT.alloc(mp * width * depth);
   xT.alloc(mp * split_cols(nin));
   dyT.alloc(mp * pt * 32);
-  partials.alloc(nb + 64);
+  partials.alloc(mp / 32 + 64);
   if (!loss.p) loss.alloc(1);
 }
 
 void Mlp::gradients_fused(const float* X, const float* T, int64_t M, hipStream_t s) {
   ensure_fused(M);
-  const unsigned nb = unsigned((M + kRows - 1) / kRows);
+  const int rows = fused_rows(width, M);
+  const unsigned nb = unsigned((M + rows - 1) / rows);
   FusedArgs g = fused_args(*this, X, M);
   g.T = T;
   g.scale = 1.0f / float(M * nout);
@@ -1015,8 +1052,7 @@ void Mlp::gradients_fused(const float* X, const float* T, int64_t M, hipStream_t
   g.xT = reinterpret_cast<bf16x8*>(xT.p);
   g.dyT = reinterpret_cast<bf16x8*>(dyT.p);
   g.loss = partials.p;
-  launch_fused_width<true>(width, g, s);
-  k_finalize1<<<1, 256, 0, s>>>(partials.p, int(nb), 1.0 / double(M * nout), loss.p);
+  launch_fused_width<true>(width, rows, g, s);
   GradSumArgs r{};
   WgradArgs& w = r.w;
   w.width = width;
@@ -1025,7 +1061,7 @@ void Mlp::gradients_fused(const float* X, const float* T, int64_t M, hipStream_t
   w.nin = nin;
   w.nout = nout;
   w.ptiles = (3 * nout + 31) / 32;
-  w.nchunk = int64_t(nb) * (kRows / 16);
+  w.nchunk = int64_t(nb) * (rows / 16);
   // 512 rows a split, at most 64 splits.
   w.per_split = std::max<int64_t>(32, (w.nchunk + 63) / 64);
   r.splits = int((w.nchunk + w.per_split - 1) / w.per_split);
@@ -1039,7 +1075,7 @@ void Mlp::gradients_fused(const float* X, const float* T, int64_t M, hipStream_t
   w.dyT = g.dyT;
   w.hpart = red.p;
   w.spart = red.p + nh;
-  k_wgrad<<<dim3(unsigned((big + small + 3) / 4), unsigned(r.splits)), 256, 0, s>>>(w);
+  k_wgrad<<<unsigned((big + small + 3) / 4 * r.splits), 256, 0, s>>>(w);
   r.nweights = nweights;
   r.nparams = nparams;
   for (int l = 0; l <= depth; ++l) {
@@ -1047,14 +1083,18 @@ void Mlp::gradients_fused(const float* X, const float* T, int64_t M, hipStream_t
     r.boff[l] = boff[l];
   }
   r.grad = grad.p;
-  k_grad_sum<<<g1(nparams), 256, 0, s>>>(r);
+  r.loss_part = partials.p;
+  r.nloss = int(nb);
+  r.loss_scale = 1.0 / double(M * nout);
+  r.loss = loss.p;
+  k_grad_sum<<<g1(nparams) + 1, 256, 0, s>>>(r);
 }
 
 void Mlp::forward(const float* X, int64_t M, float* Y, hipStream_t s, bool keep_pre) {
   if (fused() && !keep_pre) {
     FusedArgs g = fused_args(*this, X, M);
     g.Y = Y;
-    launch_fused_width<false>(width, g, s);
+    launch_fused_width<false>(width, fused_rows(width, M), g, s);
     return;
   }
   ensure(M);
@@ -1168,11 +1208,8 @@ void Mlp::adam(float lr, hipStream_t s) {
   ++steps;
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   const float c1 = 1.0f - std::pow(b1, float(steps)), c2 = 1.0f - std::pow(b2, float(steps));
-  k_adam<<<g1(nweights), 256, 0, s>>>(master.p, grad.p, m1.p, m2.p, wbf.p, nweights, lr, b1, b2,
-                                      eps, c1, c2);
-  k_adam<<<g1(nparams - nweights), 256, 0, s>>>(master.p + nweights, grad.p + nweights,
-                                                m1.p + nweights, m2.p + nweights, nullptr,
-                                                nparams - nweights, lr, b1, b2, eps, c1, c2);
+  k_adam<<<g1(nparams), 256, 0, s>>>(master.p, grad.p, m1.p, m2.p, wbf.p, nweights, nparams, lr,
+                                     b1, b2, eps, c1, c2);
   make_fragments(s);
 }
 
