@@ -61,6 +61,41 @@ double gibbs_dev(nosh_nls_s* nls, ContWork& w, const double* psi_int, hipStream_
   return e;
 }
 
+// r -= <i psi, r> / <psi, psi> i psi. At a solution J (i psi) = i F = 0 and dF/dp
+// is orthogonal to i psi except for rounding. Where dF/dp itself is rounding
+// (the field's gauge makes dK/dmu psi vanish at mu = 0) that rounding made the
+// singular system inconsistent: MINRES ran to its iteration limit and the
+// tangent grew along i psi by whatever its last bits were.
+__global__ __launch_bounds__(256) void k_phase_dots(int64_t n, const double2* __restrict__ psi,
+                                                    const double2* __restrict__ r,
+                                                    double* __restrict__ partials) {
+  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  double v[2] = {0.0, 0.0};
+  if (i < n) {
+    const double2 p = psi[i], q = r[i];
+    v[0] = p.x * q.y - p.y * q.x;
+    v[1] = p.x * p.x + p.y * p.y;
+  }
+  block_partials<2>(v, partials);
+}
+
+__global__ __launch_bounds__(256) void k_phase_project(int64_t n, const double2* __restrict__ psi,
+                                                       const double* __restrict__ partials,
+                                                       double2* __restrict__ r) {
+  __shared__ double c;
+  double v[2];
+  finalize_sum<2>(v, partials, int(gridDim.x));
+  if (threadIdx.x == 0) c = v[1] > 0.0 ? v[0] / v[1] : 0.0;
+  __syncthreads();
+  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const double2 p = psi[i];
+  double2 q = r[i];
+  q.x += c * p.y;
+  q.y -= c * p.x;
+  r[i] = q;
+}
+
 // Tangent t with J(psi) t = -dF/dp(psi); returns MINRES iterations.
 int tangent(nosh_nls_s* nls, ContWork& w, const std::string& param, double* psi_int,
             const std::map<std::string, double>& p, const nosh_newton_options& o,
@@ -75,6 +110,12 @@ int tangent(nosh_nls_s* nls, ContWork& w, const std::string& param, double* psi_
   // dF/dp: dK/dp psi + (p == "g" ? ct |psi|^2 psi : ct dV/dp psi).
   launch_dfdp(m, w.dk->kv, nls->ct.p, psi_int, param == "g", nls->V->sf.dvdp_constant(param),
               nls->V->sf.dvdp_values(param, s), w.rhs.p, s);
+  const unsigned gn = grid_for(n, 256);
+  if (w.partials.n < 2 * size_t(gn)) w.partials.alloc(2 * size_t(gn));
+  const auto psi2 = reinterpret_cast<const double2*>(psi_int);
+  const auto rhs2 = reinterpret_cast<double2*>(w.rhs.p);
+  k_phase_dots<<<gn, 256, 0, s>>>(n, psi2, rhs2, w.partials.p);
+  k_phase_project<<<gn, 256, 0, s>>>(n, psi2, w.partials.p, rhs2);
   if (nls->jblk.n != size_t(3 * n)) {
     nls->jblk.alloc(3 * n);
     nls->pblk.alloc(3 * n);
