@@ -10,6 +10,11 @@ namespace nosh {
 template <class T>
 using V2 = typename Vec2<T>::type;
 
+// Meshes up to this many rows use P = 4, larger ones P = 2 (see RowBlock): at
+// 69 k rows (40^3) P = 4 takes 787 us where P = 2 takes 866, at 118 k 1126
+// against 1010.
+constexpr int64_t kSplitRows = 90000;
+
 // MI355X dispatches consecutive workgroups round-robin over its 8 XCDs.
 // Remap so that XCD x processes one contiguous range of workgroup indices,
 // keeping each XCD's gathers of x within its own L2.
@@ -35,44 +40,56 @@ __device__ __forceinline__ int32_t ld_uniform(const int32_t* p) {
 #endif
 }
 
-// Off-diagonal product of one internal row over the split layout: the upper
-// part reads its values in place, sum val_k x[col_k]; the lower part reads
-// each value at its position in the upper part (a gather that the
-// neighbouring rows' waves have just brought into L2) and uses its
-// conjugate, sum conj(val_pos_k) x[col_k]. Upper slots first, each part in
-// slot order. The columns come as 16-bit offsets from the row when the
-// layout has them (2 bytes a slot instead of 4), else as 32-bit indices;
-// the same columns in the same order either way.
-template <class T, bool OFF16>
-__device__ __forceinline__ V2<T> sell_row_cols(int64_t row, const SellView& S,
-                                               const V2<T>* __restrict__ val,
-                                               const V2<T>* __restrict__ x) {
+// Row products of one workgroup of 256 threads. P waves share a 64-row slice:
+// P = 4: two take its upper slots and two its lower ones (every other slot
+// each); P = 2: one takes the upper slots, one the lower ones. The first of
+// them adds the sums through LDS and owns the slice's rows. One wave a slice
+// walks a chain of some twelve dependent loads (slot pointer, columns,
+// gathers, first above then below the diagonal); P waves are P times as many,
+// with a part of the chain each. A Newton step of 16 MINRES iterations (112
+// products) with one, two and four waves a slice: 20^3 cube 878 / 746 / 664 us,
+// 48^3 1310 / 1010 / 1126 us, 96^3 5997 / 5025 / 5597 us in FP64 (3994 /
+// 3321 / 3878 us in FP32). Columns and positions are ordinary loads: as
+// non-temporal ones they miss the Infinity Cache when the next product reads
+// them again (96^3: 5219 us). Eight slots at a time instead of four: 6126 us.
+template <int P>
+struct RowBlock {
+  static constexpr int kSlices = 4 / P;  // per workgroup
+  int64_t row;
+  int part;    // of the slice, wave-uniform
+  bool owner;  // this thread owns `row`
+  __device__ __forceinline__ RowBlock(int64_t n) {
+    const int w = uniform(int(threadIdx.x >> 6));
+    part = w % P;
+    row = (xcd_block(true) * kSlices + w / P) * kSliceH + (threadIdx.x & 63);
+    owner = row < n && part == 0;
+  }
+};
+
+template <class T, bool OFF16, int P>
+__device__ __forceinline__ V2<T> sell_part(int64_t row, int part, const SellView& S,
+                                           const V2<T>* __restrict__ val,
+                                           const V2<T>* __restrict__ x) {
+  constexpr int H = P / 2;  // waves per half
   const int32_t s = uniform(int32_t(row >> 6));
-  const int lane = int(row & 63);
-  const int32_t r32 = int32_t(row);
+  const int32_t first = kSliceH * (part % H) + int32_t(row & 63), r32 = int32_t(row);
   T ar = T(0), ai = T(0);
-  {
-    const int32_t b = uniform(S.uptr[s]);
-    const int32_t e = uniform(S.uptr[s + 1]);
+  if (part < H) {
+    const int32_t b = uniform(S.uptr[s]), e = uniform(S.uptr[s + 1]);
 #pragma unroll 4
-    for (int32_t j = b + lane; j < e; j += kSliceH) {
-      const int32_t c = OFF16 ? r32 + int32_t(__builtin_nontemporal_load(S.uoff + j))
-                              : __builtin_nontemporal_load(S.ucol + j);
+    for (int32_t j = b + first; j < e; j += H * kSliceH) {
+      const int32_t c = OFF16 ? r32 + int32_t(S.uoff[j]) : S.ucol[j];
       const V2<T> v = val[j];
       const V2<T> xv = x[c];
       ar += v.x * xv.x - v.y * xv.y;
       ai += v.x * xv.y + v.y * xv.x;
     }
-  }
-  {
-    const int32_t b = uniform(S.lptr[s]);
-    const int32_t e = uniform(S.lptr[s + 1]);
+  } else {
+    const int32_t b = uniform(S.lptr[s]), e = uniform(S.lptr[s + 1]);
 #pragma unroll 4
-    for (int32_t j = b + lane; j < e; j += kSliceH) {
-      const int32_t c = OFF16 ? r32 + int32_t(__builtin_nontemporal_load(S.loff + j))
-                              : __builtin_nontemporal_load(S.lcol + j);
-      const int32_t p = __builtin_nontemporal_load(S.lpos + j);
-      const V2<T> v = val[p];
+    for (int32_t j = b + first; j < e; j += H * kSliceH) {
+      const int32_t c = OFF16 ? r32 + int32_t(S.loff[j]) : S.lcol[j];
+      const V2<T> v = val[S.lpos[j]];
       const V2<T> xv = x[c];
       ar += v.x * xv.x + v.y * xv.y;
       ai += v.x * xv.y - v.y * xv.x;
@@ -84,12 +101,45 @@ __device__ __forceinline__ V2<T> sell_row_cols(int64_t row, const SellView& S,
   return r;
 }
 
-template <class T>
-__device__ __forceinline__ V2<T> sell_row(int64_t row, const SellView& S,
-                                          const V2<T>* __restrict__ val,
-                                          const V2<T>* __restrict__ x) {
-  return S.uoff ? sell_row_cols<T, true>(row, S, val, x) : sell_row_cols<T, false>(row, S, val, x);
+// Off-diagonal row product of rb.row, valid where rb.owner: upper slots, then
+// lower slots conjugated at their mirrored positions (a gather that the
+// neighbouring rows' waves have just brought into L2). The columns come as
+// 16-bit offsets from the row when the layout has them (2 bytes a slot
+// instead of 4), else as 32-bit indices. Every thread of the workgroup calls
+// it (there is a barrier).
+template <class T, int P>
+__device__ __forceinline__ V2<T> row_product(const RowBlock<P>& rb, int64_t n, const SellView& S,
+                                             const V2<T>* __restrict__ val,
+                                             const V2<T>* __restrict__ x) {
+  __shared__ V2<T> sums[4][kSliceH];
+  const int w = uniform(int(threadIdx.x >> 6)), lane = int(threadIdx.x & 63);
+  V2<T> acc;
+  acc.x = acc.y = T(0);
+  if (rb.row < n)
+    acc = S.uoff ? sell_part<T, true, P>(rb.row, rb.part, S, val, x)
+                 : sell_part<T, false, P>(rb.row, rb.part, S, val, x);
+  if (rb.part > 0) sums[w][lane] = acc;
+  __syncthreads();
+  if (rb.part == 0) {
+    if constexpr (P == 4) {
+      const V2<T> a = sums[1][lane], b = sums[2][lane], c = sums[3][lane];
+      acc.x = (acc.x + a.x) + (b.x + c.x);
+      acc.y = (acc.y + a.y) + (b.y + c.y);
+    } else {
+      const V2<T> b = sums[w + 1][lane];
+      acc.x += b.x;
+      acc.y += b.y;
+    }
+  }
+  return acc;
 }
+
+// P of a mesh, and its number of workgroups and of slices they cover.
+inline int row_split(const MeshCache& m) { return m.n <= kSplitRows ? 4 : 2; }
+inline unsigned row_blocks(const MeshCache& m) {
+  return grid_for(m.n, kSliceH * (4 / row_split(m)));
+}
+inline unsigned row_slices(const MeshCache& m) { return row_blocks(m) * (4 / row_split(m)); }
 
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
@@ -101,6 +151,17 @@ __device__ __forceinline__ double wave_max(double v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
   return v;
+}
+
+// Sum of v over each slice's rows (lanes of its owning wave; v = 0 where no row
+// is owned) to partials[slice].
+template <int P>
+__device__ __forceinline__ void slice_partials(const RowBlock<P>& rb, double v,
+                                               double* __restrict__ partials) {
+  if (rb.part != 0) return;
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0)
+    partials[blockIdx.x * RowBlock<P>::kSlices + (threadIdx.x >> 6) / P] = v;
 }
 
 // Block-wide sums of NV values; the totals end up in every lane of wave 0.
@@ -165,6 +226,23 @@ __device__ __forceinline__ void finalize_sum(double (&v)[NV], const double* __re
     for (int q = 0; q < NV; ++q) v[q] = wave_sum(lane < kVw ? lds[q * 16 + lane] : 0.0);
   }
   __syncthreads();
+}
+
+// Sum of nb partials by one workgroup of kFinThreads (valid in thread 0, fixed
+// order). 1024 threads: a solve on 10^6 rows leaves 14 k partials, 14 loads
+// a thread, all in flight.
+constexpr int kFinThreads = 1024;
+__device__ __forceinline__ double fin_sum(const double* __restrict__ partials, int nb) {
+  __shared__ double w[kFinThreads / 64];
+  double v = 0.0;
+#pragma unroll 16
+  for (int i = threadIdx.x; i < nb; i += kFinThreads) v += partials[i];
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) w[threadIdx.x >> 6] = v;
+  __syncthreads();
+  v = 0.0;
+  if (threadIdx.x < 64) v = wave_sum(threadIdx.x < kFinThreads / 64 ? w[threadIdx.x] : 0.0);
+  return v;
 }
 
 }  // namespace nosh

@@ -121,53 +121,58 @@ __global__ void k_gather(int64_t n, const int32_t* __restrict__ perm,
   if (i < n) vi[i] = vr[perm[i]];
 }
 
+template <int P>
 __global__ __launch_bounds__(kBlock) void k_keo_apply(
     int64_t n, SellView S,
     const double2* __restrict__ val, const double* __restrict__ diag,
     const double2* __restrict__ x, double2* __restrict__ y) {
-  const int64_t row = xcd_block(true) * kBlock + threadIdx.x;
-  if (row >= n) return;
-  const double2 acc = sell_row<double>(row, S, val, x);
+  const RowBlock<P> rb(n);
+  const int64_t row = rb.row;
+  const double2 acc = row_product<double, P>(rb, n, S, val, x);
+  if (!rb.owner) return;
   const double2 xi = x[row];
   const double d = diag[row];
   y[row] = make_double2(acc.x + d * xi.x, acc.y + d * xi.y);
 }
 
 // f = K x + ct (V + g |x|^2) x  and  sum |f|^2 (when nrm2 != nullptr).
+template <int P>
 __global__ __launch_bounds__(kBlock) void k_compute_f(
     int64_t n, SellView S,
     const double2* __restrict__ val, const double* __restrict__ diag,
     const double* __restrict__ ct, const double* __restrict__ V, double g,
     const double2* __restrict__ x, double2* __restrict__ f, double* __restrict__ partials) {
-  const int64_t row = xcd_block(true) * kBlock + threadIdx.x;
-  double s2[1] = {0.0};
-  if (row < n) {
-    const double2 acc = sell_row<double>(row, S, val, x);
+  const RowBlock<P> rb(n);
+  const int64_t row = rb.row;
+  double s2 = 0.0;
+  const double2 acc = row_product<double, P>(rb, n, S, val, x);
+  if (rb.owner) {
     const double2 xi = x[row];
     const double a = ct[row] * (V[row] + g * (xi.x * xi.x + xi.y * xi.y));
     const double d = diag[row];
     const double2 r = make_double2(acc.x + d * xi.x + a * xi.x, acc.y + d * xi.y + a * xi.y);
     f[row] = r;
-    s2[0] = r.x * r.x + r.y * r.y;
+    s2 = r.x * r.x + r.y * r.y;
   }
-  if (partials) block_partials<1>(s2, partials);
+  if (partials) slice_partials<P>(rb, s2, partials);
 }
 
-__global__ void k_finalize_store(const double* __restrict__ partials, int nb,
-                                 double* __restrict__ out) {
-  double v[1];
-  finalize_sum<1>(v, partials, nb);
-  if (threadIdx.x == 0) *out = v[0];
+__global__ __launch_bounds__(kFinThreads) void k_finalize_store(
+    const double* __restrict__ partials, int nb, double* __restrict__ out) {
+  const double v = fin_sum(partials, nb);
+  if (threadIdx.x == 0) *out = v;
 }
 
 // dF/dp column: dK x + ct |x|^2 x (parameter "g") or ct dV/dp x.
+template <int P>
 __global__ __launch_bounds__(kBlock) void k_dfdp(
     int64_t n, SellView S,
     const double2* __restrict__ dval, const double* __restrict__ ct, int is_g, double dvdp,
     const double* __restrict__ dvdp_vec, const double2* __restrict__ x, double2* __restrict__ y) {
-  const int64_t row = xcd_block(true) * kBlock + threadIdx.x;
-  if (row >= n) return;
-  const double2 acc = sell_row<double>(row, S, dval, x);
+  const RowBlock<P> rb(n);
+  const int64_t row = rb.row;
+  const double2 acc = row_product<double, P>(rb, n, S, dval, x);
+  if (!rb.owner) return;
   const double2 xi = x[row];
   const double dv = dvdp_vec ? dvdp + dvdp_vec[row] : dvdp;
   const double a = is_g ? ct[row] * (xi.x * xi.x + xi.y * xi.y) : ct[row] * dv;
@@ -228,14 +233,15 @@ __global__ __launch_bounds__(kBlock) void k_rebuild_blocks(
   }
 }
 
-template <class T>
+template <class T, int P>
 __global__ __launch_bounds__(kBlock) void k_block_apply(
     int64_t n, SellView S,
     const V2<T>* __restrict__ val, const T* __restrict__ blk, const V2<T>* __restrict__ x,
     V2<T>* __restrict__ y) {
-  const int64_t row = xcd_block(true) * kBlock + threadIdx.x;
-  if (row >= n) return;
-  const V2<T> acc = sell_row<T>(row, S, val, x);
+  const RowBlock<P> rb(n);
+  const int64_t row = rb.row;
+  const V2<T> acc = row_product<T, P>(rb, n, S, val, x);
+  if (!rb.owner) return;
   const V2<T> xi = x[row];
   const T b0 = blk[row], b1 = blk[n + row], b2 = blk[2 * n + row];
   V2<T> r;
@@ -299,14 +305,16 @@ void launch_gather_ref(int64_t n, const int32_t* perm, const double* v_ref, doub
 
 void launch_keo_apply(const MeshCache& m, const KeoValues& kv, const double* x, double* y,
                       hipStream_t s) {
-  k_keo_apply<<<grid_for(m.n, kBlock), kBlock, 0, s>>>(
+  const auto k = row_split(m) == 4 ? k_keo_apply<4> : k_keo_apply<2>;
+  k<<<row_blocks(m), kBlock, 0, s>>>(
       m.n, sell_view(m), kv.val.p, kv.diag.p, reinterpret_cast<const double2*>(x),
       reinterpret_cast<double2*>(y));
 }
 
 void launch_dfdp(const MeshCache& m, const KeoValues& kv, const double* ct, const double* x,
                  bool is_g, double dvdp, const double* dvdp_vec, double* y, hipStream_t s) {
-  k_dfdp<<<grid_for(m.n, kBlock), kBlock, 0, s>>>(
+  const auto k = row_split(m) == 4 ? k_dfdp<4> : k_dfdp<2>;
+  k<<<row_blocks(m), kBlock, 0, s>>>(
       m.n, sell_view(m), kv.dval.p, ct, is_g ? 1 : 0, dvdp, dvdp_vec,
       reinterpret_cast<const double2*>(x), reinterpret_cast<double2*>(y));
 }
@@ -326,12 +334,13 @@ DBuf<double>& fscratch(int64_t nblocks) {
 void launch_compute_f(const MeshCache& m, const KeoValues& kv, const double* ct,
                       const double* V, double g, const double* x, double* f, double* nrm2,
                       hipStream_t s) {
-  const unsigned nb = grid_for(m.n, kBlock);
-  double* partials = nrm2 ? fscratch(nb).p : nullptr;
-  k_compute_f<<<nb, kBlock, 0, s>>>(m.n, sell_view(m), kv.val.p, kv.diag.p, ct, V, g,
-                                    reinterpret_cast<const double2*>(x),
-                                    reinterpret_cast<double2*>(f), partials);
-  if (nrm2) k_finalize_store<<<1, kFinalizeThreads, 0, s>>>(partials, int(nb), nrm2);
+  const unsigned nb = row_blocks(m), ns = row_slices(m);
+  double* partials = nrm2 ? fscratch(ns).p : nullptr;
+  const auto k = row_split(m) == 4 ? k_compute_f<4> : k_compute_f<2>;
+  k<<<nb, kBlock, 0, s>>>(m.n, sell_view(m), kv.val.p, kv.diag.p, ct, V, g,
+                          reinterpret_cast<const double2*>(x), reinterpret_cast<double2*>(f),
+                          partials);
+  if (nrm2) k_finalize_store<<<1, kFinThreads, 0, s>>>(partials, int(ns), nrm2);
 }
 
 void launch_rebuild_blocks(const MeshCache& m, const KeoValues& kv, const double* ct,
@@ -343,17 +352,25 @@ void launch_rebuild_blocks(const MeshCache& m, const KeoValues& kv, const double
       reinterpret_cast<unsigned long long*>(bound));
 }
 
+namespace {
+template <class T>
+void launch_blocks(const MeshCache& m, const V2<T>* val, const T* blk, const V2<T>* x, V2<T>* y,
+                   hipStream_t s, hipEvent_t t0, hipEvent_t t1) {
+  const auto k = row_split(m) == 4 ? k_block_apply<T, 4> : k_block_apply<T, 2>;
+  const dim3 grid(row_blocks(m));
+  if (t0 || t1)
+    hipExtLaunchKernelGGL(k, grid, dim3(kBlock), 0, s, t0, t1, 0, m.n, sell_view(m), val, blk, x,
+                          y);
+  else
+    k<<<grid, kBlock, 0, s>>>(m.n, sell_view(m), val, blk, x, y);
+}
+}  // namespace
+
 void launch_block_apply(const MeshCache& m, const KeoValues& kv, const double* blk,
                         const double* x, double* y, hipStream_t s, hipEvent_t t0,
                         hipEvent_t t1) {
-  const auto xv = reinterpret_cast<const double2*>(x);
-  const auto yv = reinterpret_cast<double2*>(y);
-  if (t0 || t1)
-    hipExtLaunchKernelGGL(k_block_apply<double>, dim3(grid_for(m.n, kBlock)), dim3(kBlock), 0, s,
-                          t0, t1, 0, m.n, sell_view(m), static_cast<const double2*>(kv.val.p), blk, xv, yv);
-  else
-    k_block_apply<double><<<grid_for(m.n, kBlock), kBlock, 0, s>>>(m.n, sell_view(m), kv.val.p,
-                                                                   blk, xv, yv);
+  launch_blocks<double>(m, kv.val.p, blk, reinterpret_cast<const double2*>(x),
+                        reinterpret_cast<double2*>(y), s, t0, t1);
 }
 
 namespace {
@@ -388,14 +405,8 @@ void launch_mul(const double* a, const double* b, double* c, int64_t n, hipStrea
 void launch_block_apply32(const MeshCache& m, const KeoValues& kv, const float* blk,
                           const float* x, float* y, hipStream_t s, hipEvent_t t0,
                           hipEvent_t t1) {
-  const auto xv = reinterpret_cast<const float2*>(x);
-  const auto yv = reinterpret_cast<float2*>(y);
-  if (t0 || t1)
-    hipExtLaunchKernelGGL(k_block_apply<float>, dim3(grid_for(m.n, kBlock)), dim3(kBlock), 0, s,
-                          t0, t1, 0, m.n, sell_view(m), kv.val32.p, blk, xv, yv);
-  else
-    k_block_apply<float><<<grid_for(m.n, kBlock), kBlock, 0, s>>>(m.n, sell_view(m),
-                                                                  kv.val32.p, blk, xv, yv);
+  launch_blocks<float>(m, kv.val32.p, blk, reinterpret_cast<const float2*>(x),
+                       reinterpret_cast<float2*>(y), s, t0, t1);
 }
 
 }  // namespace nosh

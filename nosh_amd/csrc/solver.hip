@@ -8,19 +8,25 @@
 //
 // MINRES runs as a fixed sequence of fused kernels per iteration with every
 // scalar of the Lanczos/Givens recurrences kept on the device:
-//   A  one Jacobian product v = y/beta, u = J v - (beta/beta_old) r1, the
-//      partial sums of alpha = <v,u>, and the previous iteration's update of
-//      the direction vectors w and the solution x;
-//   B  r_new = u - (alpha/beta) r2 and the first Chebyshev step on r_new;
+//   A  the Givens step of the previous iteration, one Jacobian product
+//      v = y/beta, u = J v - (beta/beta_old) r1, the partial sums of
+//      alpha = <v,u>, and the previous iteration's update of the direction
+//      vectors w and the solution x;
+//   B  alpha, r_new = u - (alfa/beta) r2 and the first Chebyshev step on r_new;
 //   C  the remaining Chebyshev steps, each one product with P; the last one
-//      also sums beta^2 = <r_new, z> and advances the Givens rotation.
-// Reductions are deterministic: partial sums per block, then a one-block
-// kernel adds them in block order and evaluates the scalar recurrences. The host only
-// polls the `done` flag every few iterations, so iterations issued after
-// convergence are no-ops. Buffer rotations (r1/r2, w) are indexed by the
-// device iteration counter, so every iteration launches identical kernels.
+//      also forms the partial sums of beta^2 = <r_new, z>.
+// Reductions are deterministic: partial sums per block, added in a fixed order
+// by every block of the next kernel (A and B) while there are few of them
+// (kFoldMax), else by a one-block kernel in between. The Givens state is then
+// written by A's first block to the other of two records, since the other
+// blocks still read the old one. The host only polls the `done` flag every
+// few iterations, so iterations issued after convergence write nothing; it
+// counts the iterations it issues, which fixes every buffer rotation (r1/r2,
+// w) until then.
 // Vectors are FP64 or FP32 (template T); inner products, norms, recurrence
 // scalars and the solution accumulator are always FP64.
+
+#include <algorithm>
 
 #include "kernels.hpp"
 #include "minres_device.hpp"
@@ -31,7 +37,33 @@ namespace {
 
 constexpr int kBlock = 256;
 
-// mode: 0 standalone preconditioner, 1 MINRES initialisation, 2 MINRES iteration.
+// Most partial sums that the consuming kernel adds itself: 16 loads a thread,
+// issued ahead of the row product. A separate one-block kernel costs 2.5-6 us
+// and a launch. Newton step of 16 iterations with the line at 1000 / 2048 /
+// 4096 sums: 300^2 square (1416 sums) 856 / 800 / 803 us, 400^2 (2513)
+// 961 / 967 / 893 us, 60^3 cube (3547) 1687 / 1685 / 1651 us. At 96^3 (14 k
+// sums) both ways take 5.65 ms, and every block's own sum reads 200 MB.
+constexpr unsigned kFoldMax = 4096;
+
+// Sum of v over the 256 threads of a block, in every thread (fixed order).
+__device__ __forceinline__ double block_total(double v) {
+  __shared__ double w[kBlock / 64];
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) w[threadIdx.x >> 6] = v;
+  __syncthreads();
+  return (w[0] + w[1]) + (w[2] + w[3]);
+}
+
+__device__ __forceinline__ double thread_sum(const double* __restrict__ partials, int nb) {
+  double v = 0.0;
+#pragma unroll 8
+  for (int i = threadIdx.x; i < nb; i += kBlock) v += partials[i];
+  return v;
+}
+
+// Chebyshev coefficients of one solve: theta, then (c1, c2) of steps 1, 2, ...
+// Worked out once by the first kernel of a chain (some ten dependent FP64
+// divisions, 0.5 us, that every thread of every step used to do).
 template <class T>
 struct ChebArgs {
   int64_t n;
@@ -41,111 +73,140 @@ struct ChebArgs {
   const double* bound; // max ratio from the rebuild
   double upper, ratio;
   int iters;           // Chebyshev iterations (0 = identity)
-  V2<T>* R0;           // r buffers (mode 0/1: the input, R0 == R1)
-  V2<T>* R1;
-  V2<T>* D;            // Chebyshev direction
+  V2<T>* r;            // residual (written by mode 2's first step)
+  const V2<T>* r2;     // mode 2: the previous residual
   const V2<T>* u;      // mode 2: J v - (beta/oldb) r1
   MinresScalars* S;
-  double* partials;
+  double* coef;
+  const double* pa;    // partial sums of alfa, na of them (mode 2)
+  int na, fold;        // fold: the first step adds them, else S->alfa holds the sum
+  double* pb;          // partial sums of beta^2
 };
 
 // Chebyshev step 0 (z = D^{-1} r / theta), producing r first in mode 2.
+// mode: 0 standalone preconditioner, 1 MINRES initialisation, 2 MINRES iteration.
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_cheb_first(ChebArgs<T> a, int mode, V2<T>* zout) {
   MinresScalars* S = a.S;
-  if (mode != 0 && S->done) return;
   const int64_t row = int64_t(blockIdx.x) * kBlock + threadIdx.x;
-  const int it = mode == 2 ? S->it : 0;
-  V2<T>* r = (mode == 2) ? ((it & 1) ? a.R1 : a.R0) : a.R0;
+  double alfa = 0.0;
+  if (mode == 2) {
+    alfa = a.fold ? block_total(thread_sum(a.pa, a.na)) : S->alfa;
+    if (S->done) return;
+    if (a.fold && blockIdx.x == 0 && threadIdx.x == 0) {
+      S->alfa = alfa;
+      S->pending = 0;
+    }
+  } else {
+    if (mode == 1 && S->done) return;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      const double hi = cheb_hi(a.bound, a.upper);
+      a.coef[0] = 0.5 * (hi + hi / a.ratio);
+      for (int j = 1; j < a.iters; ++j) {
+        const Cheb c = cheb_coef(hi, a.ratio, j);
+        a.coef[2 * j - 1] = c.c1;
+        a.coef[2 * j] = c.c2;
+      }
+    }
+  }
   double s2[1] = {0.0};
   if (row < a.n) {
     V2<T> rv;
     if (mode == 2) {
-      const V2<T>* r2 = (it & 1) ? a.R0 : a.R1;
-      const T c = T(S->alfa / S->beta);
-      const V2<T> uu = a.u[row], r2v = r2[row];
+      const T c = T(alfa / S->beta);
+      const V2<T> uu = a.u[row], r2v = a.r2[row];
       rv.x = uu.x - c * r2v.x;
       rv.y = uu.y - c * r2v.y;
-      r[row] = rv;
+      a.r[row] = rv;
     } else {
-      rv = r[row];
+      rv = a.r[row];
     }
     V2<T> z;
     if (a.iters == 0) {
       z = rv;
     } else {
-      const double hi = cheb_hi(a.bound, a.upper);
-      const T th = T(0.5 * (hi + hi / a.ratio));
+      double th = 0.0;
+      if (mode == 2) {
+        th = a.coef[0];
+      } else {
+        const double hi = cheb_hi(a.bound, a.upper);
+        th = 0.5 * (hi + hi / a.ratio);
+      }
       T o0, o1;
       dinv<T>(a.pblk[row], a.pblk[a.n + row], a.pblk[2 * a.n + row], rv.x, rv.y, &o0, &o1);
-      z.x = o0 / th;
-      z.y = o1 / th;
-      if (a.iters > 1) a.D[row] = z;
+      z.x = o0 / T(th);
+      z.y = o1 / T(th);
     }
     zout[row] = z;
     s2[0] = double(rv.x) * double(z.x) + double(rv.y) * double(z.y);
   }
   if (mode == 0 || a.iters > 1) return;
-  block_partials<1>(s2, a.partials);
+  block_partials<1>(s2, a.pb);
 }
 
-// Chebyshev step j >= 1: z_out = z_in + d, d = c1 d + c2 D^{-1}(r - P z_in).
-template <class T>
+// Chebyshev step j >= 1 in three-term form,
+//   z_j = z_{j-1} + c1 (z_{j-1} - z_{j-2}) + c2 D^{-1} (r - P z_{j-1}),
+// z_{-1} = 0; z_{j-2} sits in z_j's buffer and is overwritten by its own
+// thread, so no direction vector is stored.
+template <class T, int P>
 __global__ __launch_bounds__(kBlock) void k_cheb_step(ChebArgs<T> a, int mode, int j,
                                                      const V2<T>* __restrict__ zin,
                                                      V2<T>* __restrict__ zout) {
-  MinresScalars* S = a.S;
-  if (mode != 0 && S->done) return;
-  const int64_t row = xcd_block(true) * kBlock + threadIdx.x;
-  const int it = mode == 2 ? S->it : 0;
-  const V2<T>* r = (mode == 2) ? ((it & 1) ? a.R1 : a.R0) : a.R0;
-  const bool last = (j == a.iters - 1);
-  double s2[1] = {0.0};
-  if (row < a.n) {
-    const Cheb c = cheb_coef(cheb_hi(a.bound, a.upper), a.ratio, j);
-    const V2<T> acc = sell_row<T>(row, a.sv, a.pval, zin);
-    const V2<T> zi = zin[row];
-    const T b0 = a.pblk[row], b1 = a.pblk[a.n + row], b2 = a.pblk[2 * a.n + row];
-    const V2<T> rv = r[row];
+  const MinresScalars* S = a.S;
+  // Read here, used after the row product: one load less in front of it (a
+  // no-op launch then costs as much as a real one; see minres_solve's poll).
+  const int done = mode != 0 ? S->done : 0;
+  const RowBlock<P> rb(a.n);
+  const int64_t row = rb.row;
+  V2<T> zi{}, rv{}, zpp{};
+  T b0 = T(1), b1 = T(1), b2 = T(0);
+  if (rb.owner) {
+    zi = zin[row];
+    rv = a.r[row];
+    if (j > 1) zpp = zout[row];
+    b0 = a.pblk[row], b1 = a.pblk[a.n + row], b2 = a.pblk[2 * a.n + row];
+  }
+  const T c1 = T(a.coef[2 * j - 1]), c2 = T(a.coef[2 * j]);
+  const V2<T> acc = row_product<T, P>(rb, a.n, a.sv, a.pval, zin);
+  if (done) return;
+  double s2 = 0.0;
+  if (rb.owner) {
     const T res0 = rv.x - (acc.x + b0 * zi.x + b2 * zi.y);
     const T res1 = rv.y - (acc.y + b2 * zi.x + b1 * zi.y);
     T u0, u1;
     dinv<T>(b0, b1, b2, res0, res1, &u0, &u1);
-    V2<T> d = a.D[row];
-    d.x = T(c.c1) * d.x + T(c.c2) * u0;
-    d.y = T(c.c1) * d.y + T(c.c2) * u1;
     V2<T> z;
-    z.x = zi.x + d.x;
-    z.y = zi.y + d.y;
-    if (!last) a.D[row] = d;
+    z.x = zi.x + (c1 * (zi.x - zpp.x) + c2 * u0);
+    z.y = zi.y + (c1 * (zi.y - zpp.y) + c2 * u1);
     zout[row] = z;
-    s2[0] = double(rv.x) * double(z.x) + double(rv.y) * double(z.y);
+    s2 = double(rv.x) * double(z.x) + double(rv.y) * double(z.y);
   }
-  if (mode == 0 || !last) return;
-  block_partials<1>(s2, a.partials);
+  if (mode == 0 || j != a.iters - 1) return;
+  slice_partials<P>(rb, s2, a.pb);
 }
 
 // beta^2 = sum of the partials of <r, z>: MINRES initialisation (mode 1) or
 // the Givens step of the current iteration (mode 2).
-__global__ void k_fin_beta(MinresScalars* S, const double* __restrict__ partials, int nb,
-                           int mode) {
+__global__ __launch_bounds__(kFinThreads) void k_fin_beta(MinresScalars* S,
+                                                          const double* __restrict__ partials,
+                                                          int nb, int mode) {
   if (mode == 2 && S->done) return;
-  double v[1];
-  finalize_sum<1>(v, partials, nb);
+  const double v = fin_sum(partials, nb);
   if (threadIdx.x == 0) {
     if (mode == 1)
-      init_update(S, v[0]);
+      init_update(S, v);
     else
-      givens_update(S, v[0]);
+      givens_update(S, v);
   }
 }
 
-__global__ void k_fin_alfa(MinresScalars* S, const double* __restrict__ partials, int nb) {
+__global__ __launch_bounds__(kFinThreads) void k_fin_alfa(MinresScalars* S,
+                                                          const double* __restrict__ partials,
+                                                          int nb) {
   if (S->done) return;
-  double v[1];
-  finalize_sum<1>(v, partials, nb);
+  const double v = fin_sum(partials, nb);
   if (threadIdx.x == 0) {
-    S->alfa = v[0];
+    S->alfa = v;
     S->pending = 0;
   }
 }
@@ -159,62 +220,61 @@ struct MinresArgs {
   const V2<T>* y;  // preconditioned residual of the previous iteration
   V2<T>* v;
   V2<T>* u;
-  const V2<T>* R0;
-  const V2<T>* R1;
-  V2<T>* W0;
-  V2<T>* W1;
-  V2<T>* W2;
+  V2<T>* W[3];     // direction vector k in W[k % 3]
   double2* x;
-  MinresScalars* S;
-  double* partials;
 };
-
-template <class T>
-__device__ __forceinline__ V2<T>* wbuf(const MinresArgs<T>& a, int k) {
-  const int q = ((k % 3) + 3) % 3;
-  return q == 0 ? a.W0 : (q == 1 ? a.W1 : a.W2);
-}
 
 // Pending update of iteration k: w_k = (v_k - oldeps w_{k-2} - delta w_{k-1}) / gamma,
 // x += phi w_k.
 template <class T>
-__device__ __forceinline__ void w_update(const MinresArgs<T>& a, const MinresScalars* S, int k,
-                                         int64_t row, V2<T> vk) {
-  V2<T>* wk = wbuf(a, k);
-  const V2<T> w1 = wbuf(a, k - 2)[row], w2 = wbuf(a, k - 1)[row];
-  const T oe = T(S->p_oldeps), de = T(S->p_delta), dn = T(S->p_denom);
+__device__ __forceinline__ void w_update(const V2<T>* w1p, const V2<T>* w2p, V2<T>* wk, double2* x,
+                                         const MinresScalars& S, int64_t row, V2<T> vk) {
+  const V2<T> w1 = w1p[row], w2 = w2p[row];
+  const T oe = T(S.p_oldeps), de = T(S.p_delta), dn = T(S.p_denom);
   V2<T> w;
   w.x = (vk.x - oe * w1.x - de * w2.x) * dn;
   w.y = (vk.y - oe * w1.y - de * w2.y) * dn;
   wk[row] = w;
-  const double phi = S->p_phi;
-  double2 xv = a.x[row];
-  xv.x += phi * double(w.x);
-  xv.y += phi * double(w.y);
-  a.x[row] = xv;
+  double2 xv = x[row];
+  xv.x += S.p_phi * double(w.x);
+  xv.y += S.p_phi * double(w.y);
+  x[row] = xv;
 }
 
-template <class T>
-__global__ __launch_bounds__(kBlock) void k_minres_a(MinresArgs<T> a) {
-  MinresScalars* S = a.S;
-  if (S->done) return;
-  const int64_t row = xcd_block(true) * kBlock + threadIdx.x;
-  const int it = S->it;
-  const double beta = S->beta;
-  double s[1] = {0.0};
-  if (row < a.n) {
-    const V2<T> vold = a.v[row];
-    if (S->pending) w_update<T>(a, S, it, row, vold);
-    const V2<T> acc = sell_row<T>(row, a.sv, a.jval, a.y);
+// Iteration `it` (from 0). Sin: the state of this iteration's start, or with
+// nb > 0 the one before the Givens step whose nb partial sums are in pb, which
+// is then taken here and stored in Sout.
+template <class T, int P>
+__global__ __launch_bounds__(kBlock) void k_minres_a(MinresArgs<T> a, int it, const V2<T>* r1,
+                                                     const MinresScalars* Sin, MinresScalars* Sout,
+                                                     const double* pb, int nb, double* pa) {
+  __shared__ MinresScalars S;
+  double sum = nb > 0 ? thread_sum(pb, nb) : 0.0;
+  const RowBlock<P> rb(a.n);
+  const int64_t row = rb.row;
+  const V2<T> acc = row_product<T, P>(rb, a.n, a.sv, a.jval, a.y);
+  if (nb > 0) sum = block_total(sum);
+  if (threadIdx.x == 0) {
+    S = *Sin;
+    if (nb > 0) {
+      if (!S.done) givens_update(&S, sum);
+      if (blockIdx.x == 0) *Sout = S;
+    }
+  }
+  __syncthreads();
+  if (S.done) return;
+  double s = 0.0;
+  if (rb.owner) {
+    if (it >= 1)
+      w_update<T>(a.W[(it + 1) % 3], a.W[(it + 2) % 3], a.W[it % 3], a.x, S, row, a.v[row]);
     const V2<T> yi = a.y[row];
     const T b0 = a.jblk[row], b1 = a.jblk[a.n + row], b2 = a.jblk[2 * a.n + row];
-    const T ib = T(1.0 / beta);
+    const T ib = T(1.0 / S.beta);
     V2<T> uu;
     uu.x = (acc.x + b0 * yi.x + b2 * yi.y) * ib;
     uu.y = (acc.y + b2 * yi.x + b1 * yi.y) * ib;
     if (it >= 1) {
-      const V2<T>* r1 = (it & 1) ? a.R1 : a.R0;  // r1 of iteration it+1: R[it % 2]
-      const T c = T(beta / S->oldb);
+      const T c = T(S.beta / S.oldb);
       const V2<T> rv = r1[row];
       uu.x -= c * rv.x;
       uu.y -= c * rv.y;
@@ -224,18 +284,21 @@ __global__ __launch_bounds__(kBlock) void k_minres_a(MinresArgs<T> a) {
     vn.y = yi.y * ib;
     a.v[row] = vn;
     a.u[row] = uu;
-    s[0] = double(vn.x) * double(uu.x) + double(vn.y) * double(uu.y);
+    s = double(vn.x) * double(uu.x) + double(vn.y) * double(uu.y);
   }
-  block_partials<1>(s, a.partials);
+  slice_partials<P>(rb, s, pa);
 }
 
 // Applies the last pending w/x update, then psi += x when psi != nullptr.
 template <class T>
-__global__ __launch_bounds__(kBlock) void k_minres_flush(MinresArgs<T> a, double2* psi) {
-  const MinresScalars* S = a.S;
+__global__ __launch_bounds__(kBlock) void k_minres_flush(MinresArgs<T> a, const MinresScalars* S,
+                                                         double2* psi) {
   const int64_t row = int64_t(blockIdx.x) * kBlock + threadIdx.x;
   if (row >= a.n) return;
-  if (S->pending) w_update<T>(a, S, S->it, row, a.v[row]);
+  if (S->pending) {
+    const int k = S->it;
+    w_update<T>(a.W[(k + 1) % 3], a.W[(k + 2) % 3], a.W[k % 3], a.x, *S, row, a.v[row]);
+  }
   if (psi) {
     const double2 d = a.x[row];
     double2 p = psi[row];
@@ -245,11 +308,21 @@ __global__ __launch_bounds__(kBlock) void k_minres_flush(MinresArgs<T> a, double
   }
 }
 
-// r0 = r1 = scale * b (converted to T), x = 0, w_{-1} = w_0 = 0.
+// r0 = r1 = scale * b (converted to T), x = 0, w_{-1} = w_0 = 0, and the state
+// of a solve about to start.
 template <class T>
 __global__ void k_minres_setup(int64_t n, const double2* __restrict__ b, double scale,
-                               V2<T>* R0, V2<T>* R1, V2<T>* W0, V2<T>* W2, double2* x) {
+                               V2<T>* R0, V2<T>* R1, V2<T>* W0, V2<T>* W2, double2* x,
+                               MinresScalars* S, double rtol, int maxit) {
   const int64_t row = int64_t(blockIdx.x) * kBlock + threadIdx.x;
+  if (row == 0) {
+    S->done = 0;
+    S->it = 0;
+    S->pending = 0;
+    S->rtol = rtol;
+    S->maxit = maxit;
+    S->relres = 1.0;
+  }
   if (row >= n) return;
   const double2 bv = b[row];
   V2<T> r;
@@ -265,15 +338,6 @@ __global__ void k_minres_setup(int64_t n, const double2* __restrict__ b, double 
   x[row] = make_double2(0.0, 0.0);
 }
 
-__global__ void k_scalars_reset(MinresScalars* S, double rtol, int maxit) {
-  S->done = 0;
-  S->it = 0;
-  S->pending = 0;
-  S->rtol = rtol;
-  S->maxit = maxit;
-  S->relres = 1.0;
-}
-
 template <class T>
 __global__ void k_to_t(int64_t m, const double* __restrict__ a, T* __restrict__ b) {
   const int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x;
@@ -286,11 +350,10 @@ template <class T>
 void MinresWork<T>::ensure(int64_t n_) {
   if (n == n_) return;
   n = n_;
-  for (auto* b : {&Y, &Z2, &v, &u, &R0, &R1, &D, &W0, &W1, &W2}) b->alloc(n);
+  for (auto* b : {&Y, &Z2, &v, &u, &R0, &R1, &W0, &W1, &W2}) b->alloc(n);
   x.alloc(n);
-  const int64_t nb = grid_for(n, kBlock);
-  partials.alloc(4 * nb + 64);
-  if (!S.p) S.alloc(1);
+  partials.alloc(2 * size_t(grid_for(n, kSliceH) + 4));  // one per slice, whatever its waves
+  if (!S.p) S.alloc(2);
   if (!Sh) NOSH_HIP(hipHostMalloc(reinterpret_cast<void**>(&Sh), sizeof(MinresScalars)));
   NOSH_HIP(hipStreamSynchronize(default_stream()));
 }
@@ -301,9 +364,10 @@ MinresWork<T>::~MinresWork() {
 }
 
 template <class T>
-static ChebArgs<T> cheb_args(const MeshCache& m, const PrecView<T>& P, MinresWork<T>& w,
-                             V2<T>* R0, V2<T>* R1) {
-  ChebArgs<T> a;
+static ChebArgs<T> cheb_args(const MeshCache& m, const PrecView<T>& P, MinresWork<T>& w) {
+  const size_t nc = 2 * size_t(std::max(P.iters, 64));
+  if (w.coef.n < nc) w.coef.alloc(nc);
+  ChebArgs<T> a{};
   a.n = m.n;
   a.sv = sell_view(m);
   a.pval = P.val;
@@ -312,35 +376,37 @@ static ChebArgs<T> cheb_args(const MeshCache& m, const PrecView<T>& P, MinresWor
   a.upper = P.upper;
   a.ratio = P.ratio;
   a.iters = P.iters;
-  a.R0 = R0;
-  a.R1 = R1;
-  a.D = w.D.p;
   a.u = w.u.p;
   a.S = w.S.p;
-  a.partials = w.partials.p;
+  a.coef = w.coef.p;
+  a.pa = w.partials.p;
+  a.pb = w.partials.p + w.partials.n / 2;
   return a;
 }
 
-// Launches the Chebyshev chain so that the final z lands in `out`.
+// Launches the Chebyshev chain so that the final z lands in `out`; returns
+// the number of partial sums of beta^2 (modes 1 and 2).
 template <class T>
-static void cheb_chain(const MeshCache& m, ChebArgs<T> a, int mode, V2<T>* out, V2<T>* tmp,
-                       hipStream_t s) {
-  const unsigned nb = grid_for(m.n, kBlock);
+static unsigned cheb_chain(const MeshCache& m, const ChebArgs<T>& a, int mode, V2<T>* out,
+                           V2<T>* tmp, hipStream_t s) {
+  const unsigned n1 = grid_for(m.n, kBlock), nb = row_blocks(m);
+  const auto step = row_split(m) == 4 ? k_cheb_step<T, 4> : k_cheb_step<T, 2>;
   const int steps = a.iters < 1 ? 1 : a.iters;
   V2<T>* zb[2] = {out, tmp};
   int cur = (steps - 1) % 2;
-  k_cheb_first<T><<<nb, kBlock, 0, s>>>(a, mode, zb[cur]);
+  k_cheb_first<T><<<n1, kBlock, 0, s>>>(a, mode, zb[cur]);
   for (int j = 1; j < steps; ++j) {
-    k_cheb_step<T><<<nb, kBlock, 0, s>>>(a, mode, j, zb[cur], zb[1 - cur]);
+    step<<<nb, kBlock, 0, s>>>(a, mode, j, zb[cur], zb[1 - cur]);
     cur = 1 - cur;
   }
-  if (mode != 0) k_fin_beta<<<1, kFinalizeThreads, 0, s>>>(a.S, a.partials, int(nb), mode);
+  return steps > 1 ? row_slices(m) : n1;
 }
 
 template <class T>
 void prec_apply(const MeshCache& m, const PrecView<T>& P, MinresWork<T>& w, const V2<T>* r,
                 V2<T>* z, hipStream_t s) {
-  ChebArgs<T> a = cheb_args(m, P, w, const_cast<V2<T>*>(r), const_cast<V2<T>*>(r));
+  ChebArgs<T> a = cheb_args(m, P, w);
+  a.r = const_cast<V2<T>*>(r);  // read only in mode 0
   cheb_chain<T>(m, a, 0, z, w.Z2.p, s);
 }
 
@@ -349,43 +415,45 @@ int minres_solve(const MeshCache& m, const JacView<T>& J, const PrecView<T>& P,
                  MinresWork<T>& w, const double* b, double b_scale, double rtol, int maxit,
                  double* psi_update, hipStream_t s, double* relres_out, int poll) {
   w.ensure(m.n);
-  const unsigned nb = grid_for(m.n, kBlock);
-  k_scalars_reset<<<1, 1, 0, s>>>(w.S.p, rtol, maxit);
-  k_minres_setup<T><<<nb, kBlock, 0, s>>>(m.n, reinterpret_cast<const double2*>(b), b_scale,
-                                          w.R0.p, w.R1.p, w.W0.p, w.W2.p, w.x.p);
-  ChebArgs<T> ca = cheb_args(m, P, w, w.R0.p, w.R1.p);
+  const unsigned n1 = grid_for(m.n, kBlock), nb = row_blocks(m), ns = row_slices(m);
+  MinresScalars* S[2] = {w.S.p, w.S.p + 1};
+  int cur = 0;  // the current state's record
+  k_minres_setup<T><<<n1, kBlock, 0, s>>>(m.n, reinterpret_cast<const double2*>(b), b_scale,
+                                          w.R0.p, w.R1.p, w.W0.p, w.W2.p, w.x.p, S[0], rtol,
+                                          maxit);
+  V2<T>* R[2] = {w.R0.p, w.R1.p};
+  ChebArgs<T> ca = cheb_args(m, P, w);
+  double* const pa = w.partials.p;
+  ca.na = int(ns);
+  ca.fold = ns <= kFoldMax;
   // y = M^{-1} b and beta1.
-  cheb_chain<T>(m, ca, 1, w.Y.p, w.Z2.p, s);
-  MinresArgs<T> ma;
-  ma.n = m.n;
-  ma.sv = sell_view(m);
-  ma.jval = J.val;
-  ma.jblk = J.blk;
-  ma.y = w.Y.p;
-  ma.v = w.v.p;
-  ma.u = w.u.p;
-  ma.R0 = w.R0.p;
-  ma.R1 = w.R1.p;
-  ma.W0 = w.W0.p;
-  ma.W1 = w.W1.p;
-  ma.W2 = w.W2.p;
-  ma.x = w.x.p;
-  ma.S = w.S.p;
-  ma.partials = w.partials.p;
+  ca.r = R[0];
+  const unsigned nbeta = cheb_chain<T>(m, ca, 1, w.Y.p, w.Z2.p, s);
+  k_fin_beta<<<1, kFinThreads, 0, s>>>(S[0], ca.pb, int(nbeta), 1);
+  MinresArgs<T> ma{m.n, sell_view(m), J.val, J.blk, w.Y.p, w.v.p, w.u.p,
+                   {w.W0.p, w.W1.p, w.W2.p}, w.x.p};
+  const bool fold_beta = nbeta <= kFoldMax;
+  const auto iter = row_split(m) == 4 ? k_minres_a<T, 4> : k_minres_a<T, 2>;
   int issued = 0;
   for (;;) {
+    bool owed = false;  // the last iteration's Givens step is still to be taken
     for (int q = 0; q < poll && issued < maxit; ++q, ++issued) {
-      k_minres_a<T><<<nb, kBlock, 0, s>>>(ma);
-      k_fin_alfa<<<1, kFinalizeThreads, 0, s>>>(w.S.p, w.partials.p, int(nb));
+      iter<<<nb, kBlock, 0, s>>>(ma, issued, R[issued & 1], S[cur], S[1 - cur], ca.pb,
+                                 owed ? int(nbeta) : 0, pa);
+      if (owed) cur = 1 - cur;
+      ca.S = S[cur];
+      ca.r = R[issued & 1];
+      ca.r2 = R[1 - (issued & 1)];
+      if (!ca.fold) k_fin_alfa<<<1, kFinThreads, 0, s>>>(S[cur], pa, int(ns));
       cheb_chain<T>(m, ca, 2, w.Y.p, w.Z2.p, s);
+      owed = fold_beta && q + 1 < poll && issued + 1 < maxit;
+      if (!owed) k_fin_beta<<<1, kFinThreads, 0, s>>>(S[cur], ca.pb, int(nbeta), 2);
     }
-    NOSH_HIP(hipMemcpyAsync(w.Sh, w.S.p, sizeof(MinresScalars), hipMemcpyDeviceToHost, s));
+    NOSH_HIP(hipMemcpyAsync(w.Sh, S[cur], sizeof(MinresScalars), hipMemcpyDeviceToHost, s));
     NOSH_HIP(hipStreamSynchronize(s));
     if (w.Sh->done || issued >= maxit) break;
   }
-  k_minres_flush<T><<<nb, kBlock, 0, s>>>(ma, reinterpret_cast<double2*>(psi_update));
-  NOSH_HIP(hipMemcpyAsync(w.Sh, w.S.p, sizeof(MinresScalars), hipMemcpyDeviceToHost, s));
-  NOSH_HIP(hipStreamSynchronize(s));
+  k_minres_flush<T><<<n1, kBlock, 0, s>>>(ma, S[cur], reinterpret_cast<double2*>(psi_update));
   if (relres_out) *relres_out = w.Sh->relres;
   return w.Sh->it;
 }
