@@ -333,7 +333,7 @@ int nosh_batch_create(int ngroups, const nosh_nls_t* models, const int* counts, 
       launch_slot_fields(m, md->keo->alpha.p, md->mvp->vf.atilde.p, G.s32.p, G.a64.p,
                          G.t64.p, G.diag.p, G.rowabs.p, s);
       G.ct.alloc(m.n);
-      compute_ct(m, md->thickness, G.ct, p0, s);
+      launch_mul(m.cv_int.p, md->thickness->sf.get_v(p0, s), G.ct.p, m.n, s);
       G.V.alloc(m.n);
       NOSH_HIP(hipMemcpyAsync(G.V.p, md->V->sf.get_v(p0, s), sizeof(double) * m.n,
                               hipMemcpyDeviceToDevice, s));

@@ -56,6 +56,7 @@ const double* ScalarField::get_v(const std::map<std::string, double>& p, hipStre
       launch_fill(dev.p, mesh->n, v, s);
       dev_value = v;
       dev_valid = true;
+      ++version;
     }
   } else {
     // vals.scale(params.at("beta")) (src/scalar_field_explicit_values.cpp:36-43).
@@ -65,6 +66,7 @@ const double* ScalarField::get_v(const std::map<std::string, double>& p, hipStre
       launch_scale(base.p, beta, dev.p, mesh->n, s);
       dev_value = beta;
       dev_valid = true;
+      ++version;
     }
   }
   return dev.p;
@@ -130,7 +132,8 @@ void check_apply_mode(int mode, double alpha, double beta) {
 
 hipStream_t stream_of(void* s) { return s ? static_cast<hipStream_t>(s) : default_stream(); }
 
-// Host columns -> device (internal order) -> op -> host columns.
+// Host columns -> device (internal order) -> op -> host columns. The op takes
+// internal order and writes reference order.
 template <class Op>
 void host_apply(MeshCache& m, Staging& st, const double* x, double* y, int ncols, int64_t ld,
                 Op op) {
@@ -143,8 +146,7 @@ void host_apply(MeshCache& m, Staging& st, const double* x, double* y, int ncols
   for (int c = 0; c < ncols; ++c) {
     st.a.upload(x + c * ld, len, s);
     launch_permute_in(m.n, m.perm.p, st.a.p, st.b.p, s);
-    op(st.b.p, st.c.p, s);
-    launch_permute_out(m.n, m.perm.p, st.c.p, st.d.p, s);
+    op(st.b.p, st.d.p, s);
     st.d.download(y + c * ld, len, s);
   }
   NOSH_HIP(hipStreamSynchronize(s));
@@ -155,8 +157,7 @@ void device_apply(MeshCache& m, Staging& st, const double* x, double* y, hipStre
   NOSH_CHECK(x && y, kInvalid, "null vector");
   st.ensure(2 * m.n);
   launch_permute_in(m.n, m.perm.p, x, st.b.p, s);
-  op(st.b.p, st.c.p, s);
-  launch_permute_out(m.n, m.perm.p, st.c.p, y, s);
+  op(st.b.p, y, s);
 }
 
 void upload_internal(MeshCache& m, Staging& st, const double* x_host, double* dst,
@@ -202,10 +203,13 @@ double need(const std::map<std::string, double>& p, const char* key) {
   return it->second;
 }
 
-void compute_ct(MeshCache& m, nosh_sfield_s* t, DBuf<double>& ct,
+void compute_ct(MeshCache& m, nosh_sfield_s* t, CtBuf& ct,
                 const std::map<std::string, double>& p, hipStream_t s) {
+  const double* v = t->sf.get_v(p, s);
+  if (ct.n == size_t(m.n) && ct.version == t->sf.version) return;
   if (ct.n != size_t(m.n)) ct.alloc(m.n);
-  launch_mul(m.cv_int.p, t->sf.get_v(p, s), ct.p, m.n, s);
+  launch_mul(m.cv_int.p, v, ct.p, m.n, s);
+  ct.version = t->sf.version;
 }
 
 }  // namespace nosh
@@ -437,7 +441,8 @@ int nosh_keo_set_parameters(nosh_keo_t keo, int np, const char* const* names,
   });
 }
 
-static void keo_op(nosh_keo_s* keo, const double* x, double* y, hipStream_t s) {
+static void keo_op(nosh_keo_s* keo, const double* x, double* y, hipStream_t s,
+                   const int32_t* perm = nullptr) {
   MeshCache& m = *keo->mesh->m;
   if (keo->dkeo) {
     // dK/dp alone: the dF/dp kernel with a zero vertex term.
@@ -446,9 +451,9 @@ static void keo_op(nosh_keo_s* keo, const double* x, double* y, hipStream_t s) {
       zero.alloc(m.n);
       zero.zero(s);
     }
-    launch_dfdp(m, keo->kv, zero.p, x, false, 0.0, nullptr, y, s);
+    launch_dfdp(m, keo->kv, zero.p, x, false, 0.0, nullptr, y, s, perm);
   } else {
-    launch_keo_apply(m, keo->kv, x, y, s);
+    launch_keo_apply(m, keo->kv, x, y, s, perm);
   }
 }
 
@@ -458,8 +463,10 @@ int nosh_keo_apply(nosh_keo_t keo, const double* x, double* y, int ncols, int64_
     NOSH_CHECK(keo, kInvalid, "null keo");
     check_apply_mode(mode, alpha, beta);
     NOSH_CHECK(keo->kv.valid, kNotBuilt, "keo: set_parameters has not been called");
-    host_apply(*keo->mesh->m, keo->st, x, y, ncols, ld,
-               [&](const double* a, double* b, hipStream_t s) { keo_op(keo, a, b, s); });
+    MeshCache& m = *keo->mesh->m;
+    host_apply(m, keo->st, x, y, ncols, ld, [&](const double* a, double* b, hipStream_t s) {
+      keo_op(keo, a, b, s, m.perm.p);
+    });
   });
 }
 
@@ -467,8 +474,11 @@ int nosh_keo_apply_device(nosh_keo_t keo, const double* x, double* y, void* stre
   return guard([&] {
     NOSH_CHECK(keo, kInvalid, "null keo");
     NOSH_CHECK(keo->kv.valid, kNotBuilt, "keo: set_parameters has not been called");
-    device_apply(*keo->mesh->m, keo->st, x, y, stream_of(stream),
-                 [&](const double* a, double* b, hipStream_t s) { keo_op(keo, a, b, s); });
+    MeshCache& m = *keo->mesh->m;
+    device_apply(m, keo->st, x, y, stream_of(stream),
+                 [&](const double* a, double* b, hipStream_t s) {
+                   keo_op(keo, a, b, s, m.perm.p);
+                 });
   });
 }
 
@@ -534,7 +544,7 @@ int nosh_jac_apply(nosh_jac_t jac, const double* x, double* y, int ncols, int64_
     NOSH_CHECK(jac->built, kNotBuilt, "jacobian_operator: rebuild has not been called");
     MeshCache& m = *jac->mesh->m;
     host_apply(m, jac->st, x, y, ncols, ld, [&](const double* a, double* b, hipStream_t s) {
-      launch_block_apply(m, jac->keo->kv, jac->blk.p, a, b, s);
+      launch_block_apply(m, jac->keo->kv, jac->blk.p, a, b, s, nullptr, nullptr, m.perm.p);
     });
   });
 }
@@ -546,7 +556,7 @@ int nosh_jac_apply_device(nosh_jac_t jac, const double* x, double* y, void* stre
     MeshCache& m = *jac->mesh->m;
     device_apply(m, jac->st, x, y, stream_of(stream),
                  [&](const double* a, double* b, hipStream_t s) {
-                   launch_block_apply(m, jac->keo->kv, jac->blk.p, a, b, s);
+                   launch_block_apply(m, jac->keo->kv, jac->blk.p, a, b, s, nullptr, nullptr, m.perm.p);
                  });
   });
 }
@@ -719,8 +729,11 @@ int nosh_prec_apply(nosh_prec_t prec, const double* x, double* y, int ncols, int
     NOSH_CHECK(prec, kInvalid, "null preconditioner");
     check_apply_mode(mode, alpha, beta);
     NOSH_CHECK(prec->built, kNotBuilt, "keo_regularized: rebuild has not been called");
-    host_apply(*prec->mesh->m, prec->st, x, y, ncols, ld,
-               [&](const double* a, double* b, hipStream_t s) { prec_op(prec, a, b, s); });
+    MeshCache& m = *prec->mesh->m;
+    host_apply(m, prec->st, x, y, ncols, ld, [&](const double* a, double* b, hipStream_t s) {
+      prec_op(prec, a, prec->st.c.p, s);
+      launch_permute_out(m.n, m.perm.p, prec->st.c.p, b, s);
+    });
   });
 }
 
@@ -728,8 +741,12 @@ int nosh_prec_apply_device(nosh_prec_t prec, const double* x, double* y, void* s
   return guard([&] {
     NOSH_CHECK(prec, kInvalid, "null preconditioner");
     NOSH_CHECK(prec->built, kNotBuilt, "keo_regularized: rebuild has not been called");
-    device_apply(*prec->mesh->m, prec->st, x, y, stream_of(stream),
-                 [&](const double* a, double* b, hipStream_t s) { prec_op(prec, a, b, s); });
+    MeshCache& m = *prec->mesh->m;
+    device_apply(m, prec->st, x, y, stream_of(stream),
+                 [&](const double* a, double* b, hipStream_t s) {
+                   prec_op(prec, a, prec->st.c.p, s);
+                   launch_permute_out(m.n, m.perm.p, prec->st.c.p, b, s);
+                 });
   });
 }
 
@@ -739,7 +756,7 @@ int nosh_prec_apply_operator(nosh_prec_t prec, const double* x, double* y) {
     NOSH_CHECK(prec->built, kNotBuilt, "keo_regularized: rebuild has not been called");
     MeshCache& m = *prec->mesh->m;
     host_apply(m, prec->st, x, y, 1, 2 * m.n, [&](const double* a, double* b, hipStream_t s) {
-      launch_block_apply(m, prec->keo->kv, prec->blk.p, a, b, s);
+      launch_block_apply(m, prec->keo->kv, prec->blk.p, a, b, s, nullptr, nullptr, m.perm.p);
     });
   });
 }
@@ -826,13 +843,13 @@ int nosh_nls_param_nominal(nosh_nls_t nls, int index, double* value) {
 }
 
 static void nls_f_dev(nosh_nls_s* nls, const std::map<std::string, double>& p, const double* x,
-                      double* f, double* nrm2, hipStream_t s) {
+                      double* f, double* nrm2, hipStream_t s, const int32_t* perm = nullptr) {
   MeshCache& m = *nls->mesh->m;
   nls->keo->set_parameters(p, s);
   const double g = need(p, "g");
   compute_ct(m, nls->thickness, nls->ct, p, s);
   const double* V = nls->V->sf.get_v(p, s);
-  launch_compute_f(m, nls->keo->kv, nls->ct.p, V, g, x, f, nrm2, s);
+  launch_compute_f(m, nls->keo->kv, nls->ct.p, V, g, x, f, nrm2, s, perm);
 }
 
 }  // extern "C"
@@ -862,8 +879,9 @@ int nosh_nls_eval_f(nosh_nls_t nls, const double* x, int np, const char* const* 
     hipStream_t s = default_stream();
     nls->st.ensure(2 * m.n);
     upload_internal(m, nls->st, x, nls->st.b.p, s);
-    nls_f_dev(nls, p, nls->st.b.p, nls->st.c.p, nullptr, s);
-    download_internal(m, nls->st, nls->st.c.p, f, s);
+    nls_f_dev(nls, p, nls->st.b.p, nls->st.d.p, nullptr, s, m.perm.p);
+    nls->st.d.download(f, 2 * m.n, s);
+    NOSH_HIP(hipStreamSynchronize(s));
   });
 }
 
@@ -876,8 +894,7 @@ int nosh_nls_eval_f_device(nosh_nls_t nls, const double* x, int np, const char* 
     hipStream_t s = stream_of(stream);
     nls->st.ensure(2 * m.n);
     launch_permute_in(m.n, m.perm.p, x, nls->st.b.p, s);
-    nls_f_dev(nls, p, nls->st.b.p, nls->st.c.p, nullptr, s);
-    launch_permute_out(m.n, m.perm.p, nls->st.c.p, f, s);
+    nls_f_dev(nls, p, nls->st.b.p, f, nullptr, s, m.perm.p);
   });
 }
 
@@ -905,9 +922,10 @@ int nosh_nls_eval_dfdp(nosh_nls_t nls, const double* x, int np, const char* cons
     nls->st.ensure(2 * m.n);
     upload_internal(m, nls->st, x, nls->st.b.p, s);
     launch_dfdp(m, nls->dkeo->kv, nls->ct.p, nls->st.b.p, name == "g",
-                nls->V->sf.dvdp_constant(name), nls->V->sf.dvdp_values(name, s), nls->st.c.p,
-                s);
-    download_internal(m, nls->st, nls->st.c.p, dfdp, s);
+                nls->V->sf.dvdp_constant(name), nls->V->sf.dvdp_values(name, s), nls->st.d.p, s,
+                m.perm.p);
+    nls->st.d.download(dfdp, 2 * m.n, s);
+    NOSH_HIP(hipStreamSynchronize(s));
   });
 }
 

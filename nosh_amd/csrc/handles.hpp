@@ -45,6 +45,12 @@ struct Staging {
   }
 };
 
+// Control volume x thickness per row, with the fill of the thickness field it
+// was made from (compute_ct).
+struct CtBuf : DBuf<double> {
+  int64_t version = -1;
+};
+
 struct nosh_keo_s {
   nosh_mesh_s* mesh;
   nosh_sfield_s* thickness;
@@ -63,7 +69,8 @@ struct nosh_jac_s {
   nosh_sfield_s* V;
   nosh_sfield_s* thickness;
   nosh_keo_s* keo;
-  DBuf<double> ct, blk, psi;
+  CtBuf ct;
+  DBuf<double> blk, psi;
   DBuf<float> blk32;
   bool built = false;
   bool blk32_valid = false;  // blk32 holds the FP32 copy of the current blk
@@ -74,7 +81,8 @@ struct nosh_prec_s {
   nosh_mesh_s* mesh;
   nosh_sfield_s* thickness;
   std::unique_ptr<nosh_keo_s> keo;
-  DBuf<double> ct, blk, psi, bound;
+  CtBuf ct;
+  DBuf<double> blk, psi, bound;
   int iters = 6;
   double ratio = 300.0, upper = 0.0;
   bool built = false;
@@ -93,7 +101,8 @@ struct nosh_nls_s {
   std::unique_ptr<nosh_keo_s> keo, dkeo;
   std::vector<std::string> p_names;
   std::vector<double> p_nominal;
-  DBuf<double> ct, x, f, nrm2;
+  CtBuf ct;
+  DBuf<double> x, f, nrm2;
   Staging st;
   // Newton work.
   DBuf<double> jblk, pblk, bound;
@@ -110,7 +119,8 @@ double need(const std::map<std::string, double>& p, const char* key);
 // ||F(x)|| at the parameters p, x in internal order (uses nls->f, nls->nrm2).
 double residual_norm(nosh_nls_s* nls, const double* x_int,
                      const std::map<std::string, double>& p, hipStream_t s);
-void compute_ct(MeshCache& m, nosh_sfield_s* t, DBuf<double>& ct,
+// ct := control volume x thickness, unless it already is.
+void compute_ct(MeshCache& m, nosh_sfield_s* t, CtBuf& ct,
                 const std::map<std::string, double>& p, hipStream_t s);
 void newton_run(nosh_nls_s* nls, double* psi_int, const std::map<std::string, double>& p,
                 const nosh_newton_options& o, nosh_newton_stats* st, hipStream_t s);

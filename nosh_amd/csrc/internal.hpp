@@ -92,6 +92,7 @@ struct ScalarField {
   DBuf<double> dev;            // internal order, current parameters
   double dev_value = 0.0;      // constant (or beta) currently applied in dev
   bool dev_valid = false;
+  int64_t version = 0;         // counts the fills of dev
   std::map<std::string, double> scalar_parameters() const;
   // Value at the given parameters, written to dev (internal order).
   const double* get_v(const std::map<std::string, double>& p, hipStream_t s);
@@ -150,17 +151,19 @@ void launch_permute_out(int64_t n, const int32_t* perm, const double* x_int, dou
 void launch_gather_ref(int64_t n, const int32_t* perm, const double* v_ref, double* v_int,
                        hipStream_t s);
 
-// y = K x (internal order).
+// y = K x: x in internal order, y too, or in reference order when perm (the
+// mesh's) is given; the same below.
 void launch_keo_apply(const MeshCache& m, const KeoValues& kv, const double* x, double* y,
-                      hipStream_t s);
+                      hipStream_t s, const int32_t* perm = nullptr);
 // y = dK x + (is_g ? ct |x|^2 x : ct dvdp x)   (dF/dp column).
 // y = dK/dp x + ct (is_g ? |x|^2 : dvdp + dvdp_vec[k]) x; dvdp_vec may be null.
 void launch_dfdp(const MeshCache& m, const KeoValues& kv, const double* ct, const double* x,
-                 bool is_g, double dvdp, const double* dvdp_vec, double* y, hipStream_t s);
+                 bool is_g, double dvdp, const double* dvdp_vec, double* y, hipStream_t s,
+                 const int32_t* perm = nullptr);
 // f = K x + ct (V + g |x|^2) x; optional ||f||^2 into *nrm2 (device scalar).
 void launch_compute_f(const MeshCache& m, const KeoValues& kv, const double* ct,
                       const double* V, double g, const double* x, double* f, double* nrm2,
-                      hipStream_t s);
+                      hipStream_t s, const int32_t* perm = nullptr);
 // Per-vertex 2x2 blocks: J (with V) and P (keo_regularized), and the
 // Chebyshev bound into *bound (device).
 void launch_rebuild_blocks(const MeshCache& m, const KeoValues& kv, const double* ct,
@@ -170,7 +173,7 @@ void launch_rebuild_blocks(const MeshCache& m, const KeoValues& kv, const double
 // runtime stamps the kernel's own start and end into those events.
 void launch_block_apply(const MeshCache& m, const KeoValues& kv, const double* blk,
                         const double* x, double* y, hipStream_t s, hipEvent_t t0 = nullptr,
-                        hipEvent_t t1 = nullptr);
+                        hipEvent_t t1 = nullptr, const int32_t* perm = nullptr);
 
 // Elementwise helpers.
 void launch_fill(double* a, int64_t n, double v, hipStream_t s);

@@ -103,15 +103,21 @@ __global__ void k_to_fp32(const double2* __restrict__ a, int64_t nnz, float2* __
   b[j] = make_float2(float(v.x), float(v.y));
 }
 
+// Between reference and internal order. A 128-byte line of the reference side
+// holds 8 vertices that lie in 8 consecutive levels of the internal order, so
+// the workgroups of one XCD take a contiguous range of internal rows and its
+// L2 reads (or completes, before writing back) each line once; dealt round
+// the XCDs, every one of them fetched every line (912,673 rows: about 15 -> 10 us
+// against 6.5 us for the bytes at copy speed).
 __global__ void k_permute_in(int64_t n, const int32_t* __restrict__ perm,
                              const double2* __restrict__ xr, double2* __restrict__ xi) {
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  const int64_t i = xcd_block(true) * blockDim.x + threadIdx.x;
   if (i < n) xi[i] = xr[perm[i]];
 }
 
 __global__ void k_permute_out(int64_t n, const int32_t* __restrict__ perm,
                               const double2* __restrict__ xi, double2* __restrict__ xr) {
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  const int64_t i = xcd_block(true) * blockDim.x + threadIdx.x;
   if (i < n) xr[perm[i]] = xi[i];
 }
 
@@ -121,18 +127,23 @@ __global__ void k_gather(int64_t n, const int32_t* __restrict__ perm,
   if (i < n) vi[i] = vr[perm[i]];
 }
 
+// The operator kernels write row r of their result to perm[r] when perm is
+// given (reference order out), else to r. At 96^3 the scattered store adds
+// 11 us to the kernel, where the separate permutation took 15 and a second
+// vector; on small meshes it is one launch in three.
 template <int P>
 __global__ __launch_bounds__(kBlock) void k_keo_apply(
     int64_t n, SellView S,
     const double2* __restrict__ val, const double* __restrict__ diag,
-    const double2* __restrict__ x, double2* __restrict__ y) {
+    const double2* __restrict__ x, double2* __restrict__ y, const int32_t* __restrict__ perm) {
   const RowBlock<P> rb(n);
   const int64_t row = rb.row;
+  const int64_t out = perm && rb.owner ? perm[row] : row;
   const double2 acc = row_product<double, P>(rb, n, S, val, x);
   if (!rb.owner) return;
   const double2 xi = x[row];
   const double d = diag[row];
-  y[row] = make_double2(acc.x + d * xi.x, acc.y + d * xi.y);
+  y[out] = make_double2(acc.x + d * xi.x, acc.y + d * xi.y);
 }
 
 // f = K x + ct (V + g |x|^2) x  and  sum |f|^2 (when nrm2 != nullptr).
@@ -141,9 +152,11 @@ __global__ __launch_bounds__(kBlock) void k_compute_f(
     int64_t n, SellView S,
     const double2* __restrict__ val, const double* __restrict__ diag,
     const double* __restrict__ ct, const double* __restrict__ V, double g,
-    const double2* __restrict__ x, double2* __restrict__ f, double* __restrict__ partials) {
+    const double2* __restrict__ x, double2* __restrict__ f, double* __restrict__ partials,
+    const int32_t* __restrict__ perm) {
   const RowBlock<P> rb(n);
   const int64_t row = rb.row;
+  const int64_t out = perm && rb.owner ? perm[row] : row;
   double s2 = 0.0;
   const double2 acc = row_product<double, P>(rb, n, S, val, x);
   if (rb.owner) {
@@ -151,7 +164,7 @@ __global__ __launch_bounds__(kBlock) void k_compute_f(
     const double a = ct[row] * (V[row] + g * (xi.x * xi.x + xi.y * xi.y));
     const double d = diag[row];
     const double2 r = make_double2(acc.x + d * xi.x + a * xi.x, acc.y + d * xi.y + a * xi.y);
-    f[row] = r;
+    f[out] = r;
     s2 = r.x * r.x + r.y * r.y;
   }
   if (partials) slice_partials<P>(rb, s2, partials);
@@ -168,15 +181,17 @@ template <int P>
 __global__ __launch_bounds__(kBlock) void k_dfdp(
     int64_t n, SellView S,
     const double2* __restrict__ dval, const double* __restrict__ ct, int is_g, double dvdp,
-    const double* __restrict__ dvdp_vec, const double2* __restrict__ x, double2* __restrict__ y) {
+    const double* __restrict__ dvdp_vec, const double2* __restrict__ x, double2* __restrict__ y,
+    const int32_t* __restrict__ perm) {
   const RowBlock<P> rb(n);
   const int64_t row = rb.row;
+  const int64_t out = perm && rb.owner ? perm[row] : row;
   const double2 acc = row_product<double, P>(rb, n, S, dval, x);
   if (!rb.owner) return;
   const double2 xi = x[row];
   const double dv = dvdp_vec ? dvdp + dvdp_vec[row] : dvdp;
   const double a = is_g ? ct[row] * (xi.x * xi.x + xi.y * xi.y) : ct[row] * dv;
-  y[row] = make_double2(acc.x + a * xi.x, acc.y + a * xi.y);
+  y[out] = make_double2(acc.x + a * xi.x, acc.y + a * xi.y);
 }
 
 // Jacobian and keo_regularized 2x2 blocks, each stored as three arrays
@@ -237,9 +252,10 @@ template <class T, int P>
 __global__ __launch_bounds__(kBlock) void k_block_apply(
     int64_t n, SellView S,
     const V2<T>* __restrict__ val, const T* __restrict__ blk, const V2<T>* __restrict__ x,
-    V2<T>* __restrict__ y) {
+    V2<T>* __restrict__ y, const int32_t* __restrict__ perm) {
   const RowBlock<P> rb(n);
   const int64_t row = rb.row;
+  const int64_t out = perm && rb.owner ? perm[row] : row;
   const V2<T> acc = row_product<T, P>(rb, n, S, val, x);
   if (!rb.owner) return;
   const V2<T> xi = x[row];
@@ -247,7 +263,7 @@ __global__ __launch_bounds__(kBlock) void k_block_apply(
   V2<T> r;
   r.x = acc.x + b0 * xi.x + b2 * xi.y;
   r.y = acc.y + b2 * xi.x + b1 * xi.y;
-  y[row] = r;
+  y[out] = r;
 }
 
 }  // namespace
@@ -304,19 +320,20 @@ void launch_gather_ref(int64_t n, const int32_t* perm, const double* v_ref, doub
 }
 
 void launch_keo_apply(const MeshCache& m, const KeoValues& kv, const double* x, double* y,
-                      hipStream_t s) {
+                      hipStream_t s, const int32_t* perm) {
   const auto k = row_split(m) == 4 ? k_keo_apply<4> : k_keo_apply<2>;
   k<<<row_blocks(m), kBlock, 0, s>>>(
       m.n, sell_view(m), kv.val.p, kv.diag.p, reinterpret_cast<const double2*>(x),
-      reinterpret_cast<double2*>(y));
+      reinterpret_cast<double2*>(y), perm);
 }
 
 void launch_dfdp(const MeshCache& m, const KeoValues& kv, const double* ct, const double* x,
-                 bool is_g, double dvdp, const double* dvdp_vec, double* y, hipStream_t s) {
+                 bool is_g, double dvdp, const double* dvdp_vec, double* y, hipStream_t s,
+                 const int32_t* perm) {
   const auto k = row_split(m) == 4 ? k_dfdp<4> : k_dfdp<2>;
   k<<<row_blocks(m), kBlock, 0, s>>>(
       m.n, sell_view(m), kv.dval.p, ct, is_g ? 1 : 0, dvdp, dvdp_vec,
-      reinterpret_cast<const double2*>(x), reinterpret_cast<double2*>(y));
+      reinterpret_cast<const double2*>(x), reinterpret_cast<double2*>(y), perm);
 }
 
 // Reduction scratch for k_compute_f (one per process; calls on the library
@@ -333,13 +350,13 @@ DBuf<double>& fscratch(int64_t nblocks) {
 
 void launch_compute_f(const MeshCache& m, const KeoValues& kv, const double* ct,
                       const double* V, double g, const double* x, double* f, double* nrm2,
-                      hipStream_t s) {
+                      hipStream_t s, const int32_t* perm) {
   const unsigned nb = row_blocks(m), ns = row_slices(m);
   double* partials = nrm2 ? fscratch(ns).p : nullptr;
   const auto k = row_split(m) == 4 ? k_compute_f<4> : k_compute_f<2>;
   k<<<nb, kBlock, 0, s>>>(m.n, sell_view(m), kv.val.p, kv.diag.p, ct, V, g,
                           reinterpret_cast<const double2*>(x), reinterpret_cast<double2*>(f),
-                          partials);
+                          partials, perm);
   if (nrm2) k_finalize_store<<<1, kFinThreads, 0, s>>>(partials, int(ns), nrm2);
 }
 
@@ -355,22 +372,22 @@ void launch_rebuild_blocks(const MeshCache& m, const KeoValues& kv, const double
 namespace {
 template <class T>
 void launch_blocks(const MeshCache& m, const V2<T>* val, const T* blk, const V2<T>* x, V2<T>* y,
-                   hipStream_t s, hipEvent_t t0, hipEvent_t t1) {
+                   hipStream_t s, hipEvent_t t0, hipEvent_t t1, const int32_t* perm) {
   const auto k = row_split(m) == 4 ? k_block_apply<T, 4> : k_block_apply<T, 2>;
   const dim3 grid(row_blocks(m));
   if (t0 || t1)
     hipExtLaunchKernelGGL(k, grid, dim3(kBlock), 0, s, t0, t1, 0, m.n, sell_view(m), val, blk, x,
-                          y);
+                          y, perm);
   else
-    k<<<grid, kBlock, 0, s>>>(m.n, sell_view(m), val, blk, x, y);
+    k<<<grid, kBlock, 0, s>>>(m.n, sell_view(m), val, blk, x, y, perm);
 }
 }  // namespace
 
 void launch_block_apply(const MeshCache& m, const KeoValues& kv, const double* blk,
                         const double* x, double* y, hipStream_t s, hipEvent_t t0,
-                        hipEvent_t t1) {
+                        hipEvent_t t1, const int32_t* perm) {
   launch_blocks<double>(m, kv.val.p, blk, reinterpret_cast<const double2*>(x),
-                        reinterpret_cast<double2*>(y), s, t0, t1);
+                        reinterpret_cast<double2*>(y), s, t0, t1, perm);
 }
 
 namespace {
@@ -406,7 +423,7 @@ void launch_block_apply32(const MeshCache& m, const KeoValues& kv, const float* 
                           const float* x, float* y, hipStream_t s, hipEvent_t t0,
                           hipEvent_t t1) {
   launch_blocks<float>(m, kv.val32.p, blk, reinterpret_cast<const float2*>(x),
-                       reinterpret_cast<float2*>(y), s, t0, t1);
+                       reinterpret_cast<float2*>(y), s, t0, t1, nullptr);
 }
 
 }  // namespace nosh
