@@ -93,22 +93,18 @@ namespace nosh {
 void scatter_all(nosh_batch_s* h, const double* src_dev, hipStream_t s) {
   int64_t off = 0;
   for (auto& G : h->b.ghost) {
-    for (int b = 0; b < G.B; ++b) {
-      launch_scatter_lane(G.mesh->n, G.dev.bp, b, G.mesh->perm.p, src_dev + off,
-                          reinterpret_cast<double*>(G.psi.p), s);
-      off += 2 * G.mesh->n;
-    }
+    launch_scatter_lanes(G.mesh->n, G.dev.bp, G.B, G.mesh->perm.p, src_dev + off,
+                         reinterpret_cast<double*>(G.psi.p), s);
+    off += int64_t(G.B) * 2 * G.mesh->n;
   }
 }
 
 void gather_all(nosh_batch_s* h, double* dst_dev, hipStream_t s) {
   int64_t off = 0;
   for (auto& G : h->b.ghost) {
-    for (int b = 0; b < G.B; ++b) {
-      launch_gather_lane(G.mesh->n, G.dev.bp, b, G.mesh->perm.p,
-                         reinterpret_cast<const double*>(G.psi.p), dst_dev + off, s);
-      off += 2 * G.mesh->n;
-    }
+    launch_gather_lanes(G.mesh->n, G.dev.bp, G.B, G.mesh->perm.p,
+                        reinterpret_cast<const double*>(G.psi.p), dst_dev + off, s);
+    off += int64_t(G.B) * 2 * G.mesh->n;
   }
 }
 
@@ -121,11 +117,7 @@ int newton_batch(nosh_batch_s* h, const nosh_newton_options& o, nosh_batch_insta
                  const double* ptc0, int stall) {
   Batch& B = h->b;
   const int ni = B.args.ninst;
-  B.args.iters = o.cheb_iters;
-  B.args.ratio = o.cheb_ratio;
-  B.args.upper = 0.0;
-  B.args.z0 = std::max(o.cheb_iters - 1, 0) % 2;
-  B.drop_graph();
+  B.set_chebyshev(o.cheb_iters, o.cheb_ratio);
   std::vector<double> nf, nf_prev(ni, -1.0), eta_prev(ni, o.forcing_max), rt(ni);
   std::vector<int> done(ni, 0), newton(ni, 0), mres(ni, 0), last_gain(ni, 0);
   std::vector<double> best(ni, -1.0), f1(ni, -1.0), f2(ni, -1.0);
@@ -237,11 +229,7 @@ int tangent_batch(nosh_batch_s* h, const nosh_newton_options& o, double scale, d
                   hipStream_t s) {
   Batch& B = h->b;
   const int ni = B.args.ninst;
-  B.args.iters = o.cheb_iters;
-  B.args.ratio = o.cheb_ratio;
-  B.args.upper = 0.0;
-  B.args.z0 = std::max(o.cheb_iters - 1, 0) % 2;
-  B.drop_graph();
+  B.set_chebyshev(o.cheb_iters, o.cheb_ratio);
   B.active_h.assign(ni, 1);
   const std::vector<double> rt(ni, rtol);
   NOSH_HIP(hipMemcpyAsync(B.active.p, B.active_h.data(), sizeof(int) * ni, hipMemcpyHostToDevice,
@@ -301,7 +289,7 @@ extern "C" {
 int nosh_batch_create(int ngroups, const nosh_nls_t* models, const int* counts, const double* mu,
                       const double* g, nosh_batch_t* out) {
   return bguard([&] {
-    NOSH_CHECK(ngroups >= 1 && ngroups <= 16 && models && counts && mu && g && out, kInvalid,
+    NOSH_CHECK(ngroups >= 1 && ngroups <= kMaxGroups && models && counts && mu && g && out, kInvalid,
                "invalid batch description");
     auto h = std::make_unique<nosh_batch_s>();
     Batch& B = h->b;
@@ -341,6 +329,7 @@ int nosh_batch_create(int ngroups, const nosh_nls_t* models, const int* counts, 
       d.n = m.n;
       d.B = counts[k];
       d.bp = next_pow2(counts[k]);
+      d.lb = __builtin_ctz(unsigned(d.bp));
       d.inst0 = inst;
       d.slice_ptr = m.slice_ptr.p;
       d.scol = m.scol.p;
@@ -493,7 +482,7 @@ void solve_compacting(nosh_batch_s* h, const nosh_newton_options& o, const int* 
     subcaps.push_back((caps ? caps[i] : o.max_iters) - loc[i].newton_iters);
   }
   nosh_batch_t sub = nullptr;
-  if (models.size() > 16 ||
+  if (models.size() > size_t(kMaxGroups) ||
       nosh_batch_create(int(models.size()), models.data(), counts.data(), mu.data(), g.data(),
                         &sub) != NOSH_OK) {
     // Not expressible as a batch: finish in this one.

@@ -712,8 +712,8 @@ int nosh_batch_continuation_run(nosh_batch_t bt, double* psi, double span, int s
           }
           if (!ok[i]) {
             fb_h.resize(2 * n);
-            launch_gather_lane(n, G.dev.bp, b, G.mesh->perm.p,
-                               reinterpret_cast<const double*>(gc[g].cur.p), fb.p, s);
+            launch_gather_lanes(n, G.dev.bp, 1, G.mesh->perm.p,
+                                reinterpret_cast<const double*>(gc[g].cur.p + b), fb.p, s);
             fb.download(fb_h.data(), 2 * n, s);
             NOSH_HIP(hipStreamSynchronize(s));
             nosh_continuation_options co;
@@ -747,8 +747,8 @@ int nosh_batch_continuation_run(nosh_batch_t bt, double* psi, double span, int s
               r.halvings = std::max(r.halvings, fhalv);
               st[i].final_norm_f = crec[1].norm_f;
               fb.upload(fb_h.data(), 2 * n, s);
-              launch_scatter_lane(n, G.dev.bp, b, G.mesh->perm.p, fb.p,
-                                  reinterpret_cast<double*>(G.psi.p), s);
+              launch_scatter_lanes(n, G.dev.bp, 1, G.mesh->perm.p, fb.p,
+                                   reinterpret_cast<double*>(G.psi.p + b), s);
             }
           }
           if (ok[i]) st[i].converged = 1;

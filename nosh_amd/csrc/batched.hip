@@ -39,27 +39,18 @@
 namespace nosh {
 namespace {
 
-struct Lane {
-  BGroup G;  // in registers (see load_group)
-  int64_t row;
-  int b;
-  int inst;
-  int64_t idx;  // row * bp + b
-  bool valid;
-};
-
-__device__ __forceinline__ int group_of(const BatchArgs& a, int64_t vb) {
+// Group of launched block rb.
+__device__ __forceinline__ int group_of(const BatchArgs& a, unsigned rb) {
   int gi = 0;
-  while (gi + 1 < a.ngroups && vb >= a.groups[gi + 1].block0) ++gi;
+  while (gi + 1 < a.ngroups && rb >= a.gl[gi + 1]) ++gi;
   return gi;
 }
 
-// The record of the group holding virtual block v0, read through the
-// constant address space at a wave-uniform index: the record is never
-// written by a kernel, and pointers loaded from constant memory are known to
-// address global memory, so the row loops use global (not flat) loads.
-__device__ __forceinline__ BGroup load_group(const BatchArgs& a, int64_t v0) {
-  const int gi = __builtin_amdgcn_readfirstlane(group_of(a, v0));
+// A group's record, read through the constant address space at a
+// wave-uniform index: the record is never written by a kernel, and pointers
+// loaded from constant memory are known to address global memory, so the row
+// loops use global (not flat) loads.
+__device__ __forceinline__ BGroup load_group(const BatchArgs& a, int gi) {
 #if __HIP_DEVICE_COMPILE__
   typedef const __attribute__((address_space(4))) BGroup* ConstGroups;
   return ((ConstGroups)a.groups)[gi];
@@ -68,34 +59,120 @@ __device__ __forceinline__ BGroup load_group(const BatchArgs& a, int64_t v0) {
 #endif
 }
 
-__device__ __forceinline__ Lane lane_ctx(const BatchArgs& a, int64_t vb) {
-  Lane L;
-  L.G = load_group(a, vb);
-  const int bp = L.G.bp;
-  L.b = threadIdx.x & (bp - 1);
-  L.row = (vb - L.G.block0) * (blockDim.x / bp) + threadIdx.x / bp;
-  L.inst = L.G.inst0 + L.b;
-  L.idx = L.row * bp + L.b;
-  L.valid = L.row < L.G.n && L.b < L.G.B;
-  return L;
+// Per-thread context of a launched block. All fold row tiles of a block
+// belong to one group and a thread keeps its lane (instance) in all of them,
+// so the group record and the instance's MINRES scalars are read once per
+// thread, not once per tile. The record is copied into registers by scalar
+// loads at kernel entry (its index made wave-uniform): read through a pointer
+// it would be reloaded by vector loads after every store of a row tile, which
+// the compiler cannot prove does not alias it, with a wait on each reload.
+struct Ctx {
+  BGroup G;
+  unsigned part;    // the block's number in its group: the slot of its partial sums
+  int b, inst;
+  int64_t row0;     // the thread's row in the block's first tile
+  int64_t tstride;  // rows from one of the block's tiles to the next
+  bool lane_ok;  // a real instance (b < B)
+};
+
+// Row tiles of launched blocks. The launched blocks form 8 contiguous ranges,
+// one per XCD (the order xcd_block gives them), and within a group each
+// range's blocks take the range's own contiguous share of the group's tiles,
+// strided by their count (block j of a range of c blocks: tiles s + j,
+// s + j + c, s + j + 2c, ...). The blocks resident on one XCD then sweep
+// one band of rows through their own stretch of the mesh, so the halo their
+// gathers read beyond the band was mostly read by that XCD's previous band
+// and is still in its L2 (each XCD's stretch has two ends, where the
+// neighbouring XCD's rows are read again). Before, the eight XCDs took
+// adjacent bands of one sweep of the whole group (block k: tiles k, k + nl,
+// ...), and every band's halo was the neighbouring XCDs' rows, read again
+// (96^3 x 8 lanes: ~2x the gathered vector's bytes). The mapping is a
+// function of the logical block index alone (the persistent kernel, which
+// does not remap, takes the same tiles and partial-sum slots).
+struct TileMap {
+  unsigned first;   // the block's first tile in its group
+  unsigned stride;  // tiles from one of its tiles to the next
+};
+__device__ __forceinline__ TileMap tile_map(const BatchArgs& a, int gi, unsigned rb) {
+  const unsigned nb = a.gl[a.ngroups], q = nb / 8, r = nb % 8;
+  unsigned xs, xc;
+  if (rb < r * (q + 1)) {
+    xs = rb / (q + 1) * (q + 1);
+    xc = q + 1;
+  } else {
+    xs = r * (q + 1) + (rb - r * (q + 1)) / q * q;
+    xc = q;
+  }
+  const unsigned g0 = a.gl[gi], g1 = a.gl[gi + 1];
+  const unsigned s0 = max(g0, xs), s1 = min(g1, xs + xc);
+  TileMap m;
+  m.first = (s0 - g0) * unsigned(a.fold) + (rb - s0);
+  m.stride = s1 - s0;
+  return m;
 }
 
-// Per-instance partial sums of one launched block, which covers the virtual
-// blocks v0 .. v0 + fold - 1 of one group; v is the thread's sum over them
-// (0 for padding lanes). Rows are reduced in order for every lane b, giving
-// partial (v0 - block0) / fold of the instance.
-__device__ __forceinline__ void lane_partials(const BatchArgs& a, int64_t v0, double v) {
-  __shared__ double lds[1024];
-  const BGroup& G = a.groups[group_of(a, v0)];
-  lds[threadIdx.x] = v;
+__device__ __forceinline__ Ctx make_ctx(const BatchArgs& a, unsigned rb) {
+  Ctx c;
+  rb = unsigned(uniform(int32_t(rb)));
+  const int gi = group_of(a, rb);
+  c.G = load_group(a, gi);
+  c.part = rb - a.gl[gi];
+  c.b = threadIdx.x & (c.G.bp - 1);
+  c.inst = c.G.inst0 + c.b;
+  const TileMap m = tile_map(a, gi, rb);
+  const int rows = int(blockDim.x >> c.G.lb);
+  c.row0 = int64_t(m.first) * rows + (threadIdx.x >> c.G.lb);
+  c.tstride = int64_t(m.stride) * rows;
+  c.lane_ok = c.b < c.G.B;
+  return c;
+}
+
+// f(row) for every row of the thread in the block.
+template <class F>
+__device__ __forceinline__ void each_row(const BatchArgs& a, const Ctx& c, F f) {
+  int64_t row = c.row0;
+  for (int t = 0; t < a.fold && row < c.G.n; ++t, row += c.tstride) f(row);
+}
+
+// Per-instance partial sums of one launched block; v is the thread's sum over
+// its rows (0 for padding lanes), giving partial c.part of the instance.
+// The sums of a lane's R rows sit in lds[r * bp + b]; they are added as
+// at most 8 runs of consecutive rows, then the runs in order: the same order
+// whichever threads hold the rows, and a chain of R / 8 + 8 additions instead
+// of R (64 at 8 lanes and 512 threads), which every reducing block waits for.
+__device__ __forceinline__ void sum_rows(const BatchArgs& a, const BGroup& G, unsigned part,
+                                         double* lds, int R) {
+  const int bp = G.bp, runs = min(8, R), len = (R + runs - 1) / runs, nt = int(blockDim.x);
   __syncthreads();
-  const int bp = G.bp;
-  if (threadIdx.x < bp && threadIdx.x < G.B) {
-    double s = 0.0;
-    for (int r = 0; r < int(blockDim.x) / bp; ++r) s += lds[r * bp + threadIdx.x];
-    a.partials[int64_t(G.inst0 + threadIdx.x) * a.maxblocks + (v0 - G.block0) / a.fold] = s;
+  // runs bp <= R bp entries: at most two per thread (the two-lane kernels have
+  // R bp / 2 threads).
+  double s[2] = {0.0, 0.0};
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int i = int(threadIdx.x) + q * nt;
+    if (i < runs * bp) {
+      const int g = i >> G.lb, b = i & (bp - 1);
+      for (int r = g * len; r < min(R, (g + 1) * len); ++r) s[q] += lds[r * bp + b];
+    }
   }
   __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {  // run g of lane b to lds[g bp + b]
+    const int i = int(threadIdx.x) + q * nt;
+    if (i < runs * bp) lds[i] = s[q];
+  }
+  __syncthreads();
+  for (int b = int(threadIdx.x); b < G.B; b += nt) {
+    double t = 0.0;
+    for (int g = 0; g < runs; ++g) t += lds[g * bp + b];
+    a.partials[int64_t(G.inst0 + b) * a.maxblocks + part] = t;
+  }
+  __syncthreads();
+}
+__device__ __forceinline__ void lane_partials(const BatchArgs& a, const Ctx& c, double v) {
+  __shared__ double lds[1024];
+  lds[threadIdx.x] = v;
+  sum_rows(a, c.G, c.part, lds, int(blockDim.x >> c.G.lb));
 }
 
 template <class T>
@@ -279,94 +356,111 @@ __device__ __forceinline__ void brow_slots(const BGroup& G, int32_t j, int b, T 
 
 constexpr int kSlotBatch = 4;
 
-#ifndef NOSH_META_SHFL
-#define NOSH_META_SHFL 1
-#endif
+// Groups whose rows share their slot records over the quads of a wave: at
+// least 4 lanes per row. The callers keep every lane of a row in the row
+// product (lanes of converged instances and padding lanes compute and discard).
+__device__ __forceinline__ bool quad_rows(const BGroup& G) { return G.bp >= 4; }
 
-// Groups whose rows take their slot metadata by lane shuffles: every lane is
-// a real instance and the callers keep all lanes of a row in brow (lanes of
-// converged instances compute and discard).
-__device__ __forceinline__ bool meta_shfl(const BGroup& G) {
-  return NOSH_META_SHFL && G.B == G.bp && G.bp >= 4;
+// Lane i's value of v in every lane of its quad (DPP quad_perm [i,i,i,i]).
+template <int I>
+__device__ __forceinline__ int32_t quad_bcast(int32_t v) {
+  return __builtin_amdgcn_mov_dpp(v, I * 0x55, 0xf, 0xf, false);
+}
+template <int I>
+__device__ __forceinline__ float quad_bcast(float v) {
+  return __int_as_float(quad_bcast<I>(__float_as_int(v)));
+}
+template <int I>
+__device__ __forceinline__ double quad_bcast(double v) {
+  return __hiloint2double(quad_bcast<I>(__double2hiint(v)), quad_bcast<I>(__double2loint(v)));
 }
 
-// FP32 rows of a full group (B == bp >= 4 lanes, all lanes computing): the
-// shuffled row product over a whole row, NS slots per batch. Lane q < NS of
-// the row's lanes loads the metadata of slot k + q once and the others take
-// it by a lane shuffle, instead of every lane loading the same 12 bytes
-// (NS <= bp; 8 measured slower than 4 at 96^3 x 8 lanes: 178 vs 164 us,
-// occupancy 6 instead of 8). Software-pipelined: the metadata load of the
-// next batch is issued right after the x gathers of the current one, so the
-// two dependent memory latencies of consecutive batches overlap (169 -> 164
-// us against the unpipelined loop, same arithmetic in the same order).
-template <int NS>
-__device__ __forceinline__ void brow_shfl_row(const BGroup& G, int32_t j, int32_t w, int b,
-                                              float mu, const float2* __restrict__ x, float& ar,
-                                              float& ai) {
-  const int lane = int(threadIdx.x & 63);
-  const int g0 = lane & ~(G.bp - 1);
-  const int bp = G.bp;
-  SlotMeta mine = {0, 0.0f, 0.0f};
-  if (b < NS && b < w) mine = G.s32[j + b * kSliceH];
-  for (int32_t k = 0; k < w; k += NS, j += NS * kSliceH) {
-    int32_t c[NS];
-    float av[NS], tv[NS];
+// A slot's record as (column, p, q): its value p + i q at the mu all lanes share
+// (DIRECT), or (alpha, a~) from which every lane rebuilds it at its own.
+struct RecF32V {
+  static constexpr bool kDirect = true;
+  const SlotVal* r;
+  __device__ __forceinline__ void get(int32_t j, int32_t& c, float& p, float& q) const {
+    const SlotVal m = r[j];
+    c = m.col, p = m.vr, q = m.vi;
+  }
+};
+struct RecF32M {
+  static constexpr bool kDirect = false;
+  const SlotMeta* r;
+  __device__ __forceinline__ void get(int32_t j, int32_t& c, float& p, float& q) const {
+    const SlotMeta m = r[j];
+    c = m.col, p = m.alpha, q = m.at;
+  }
+};
+struct RecF64V {
+  static constexpr bool kDirect = true;
+  const int32_t* col;
+  const double2* v;
+  __device__ __forceinline__ void get(int32_t j, int32_t& c, double& p, double& q) const {
+    const double2 m = v[j];
+    c = col[j], p = m.x, q = m.y;
+  }
+};
+struct RecF64M {
+  static constexpr bool kDirect = false;
+  const int32_t* col;
+  const double *al, *at;
+  __device__ __forceinline__ void get(int32_t j, int32_t& c, double& p, double& q) const {
+    c = col[j], p = al[j], q = at[j];
+  }
+};
+
+// Row product of one lane, 4 D slots at a time: lane i of the quad loads the
+// records of slots k + i, k + 4 + i, ... and the quad shares them by DPP, so a
+// record costs one load a quad instead of one a lane (and no LDS traffic, as
+// lane shuffles would). The next records are loaded right after the gathers
+// of the current ones. The slots past the row's end gather from clamped
+// records and add x = 0, which leaves an accumulator that started at +0
+// unchanged, bit for bit. Slot order and arithmetic are brow_slots's.
+template <int D, class T, class Rec>
+__device__ __forceinline__ void brow_quad(const Rec& rec, int32_t j0, int32_t w, int bp, int b,
+                                          T mu, const typename Vt<T>::v2* __restrict__ x, T& ar,
+                                          T& ai) {
+  if (w <= 0) return;
+  const int i = int(threadIdx.x & 3);
+  int32_t c[D];
+  T p[D], q[D];
 #pragma unroll
-    for (int q = 0; q < NS; ++q) {
-      c[q] = __shfl(mine.col, g0 + q, 64);
-      av[q] = __shfl(mine.alpha, g0 + q, 64);
-      tv[q] = __shfl(mine.at, g0 + q, 64);
+  for (int d = 0; d < D; ++d) rec.get(j0 + min(4 * d + i, w - 1) * kSliceH, c[d], p[d], q[d]);
+  for (int32_t k = 0; k < w; k += 4 * D) {
+    int32_t cc[4 * D];
+    T pp[4 * D], qq[4 * D];
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      cc[4 * d] = quad_bcast<0>(c[d]), cc[4 * d + 1] = quad_bcast<1>(c[d]);
+      cc[4 * d + 2] = quad_bcast<2>(c[d]), cc[4 * d + 3] = quad_bcast<3>(c[d]);
+      pp[4 * d] = quad_bcast<0>(p[d]), pp[4 * d + 1] = quad_bcast<1>(p[d]);
+      pp[4 * d + 2] = quad_bcast<2>(p[d]), pp[4 * d + 3] = quad_bcast<3>(p[d]);
+      qq[4 * d] = quad_bcast<0>(q[d]), qq[4 * d + 1] = quad_bcast<1>(q[d]);
+      qq[4 * d + 2] = quad_bcast<2>(q[d]), qq[4 * d + 3] = quad_bcast<3>(q[d]);
     }
-    float2 xv[NS];
+    typename Vt<T>::v2 xv[4 * D];
 #pragma unroll
-    for (int q = 0; q < NS; ++q)
-      if (k + q < w) xv[q] = x[int64_t(c[q]) * bp + b];
-    if (b < NS && k + NS + b < w) mine = G.s32[j + (NS + b) * kSliceH];
+    for (int s = 0; s < 4 * D; ++s) xv[s] = x[int64_t(cc[s]) * bp + b];
+    if (k + 4 * D < w) {
 #pragma unroll
-    for (int q = 0; q < NS; ++q) {
-      if (k + q < w) {
-        float vr, vi;
-        slot_value(av[q], tv[q], mu, vr, vi);
-        cmac(ar, ai, vr, vi, xv[q]);
-      }
+      for (int d = 0; d < D; ++d)
+        rec.get(j0 + min(k + 4 * D + 4 * d + i, w - 1) * kSliceH, c[d], p[d], q[d]);
+    }
+#pragma unroll
+    for (int s = 0; s < 4 * D; ++s) {
+      const bool in = k + s < w;
+      xv[s].x = in ? xv[s].x : T(0);
+      xv[s].y = in ? xv[s].y : T(0);
+      T vr = pp[s], vi = qq[s];
+      if constexpr (!Rec::kDirect) slot_value(pp[s], qq[s], mu, vr, vi);
+      cmac(ar, ai, vr, vi, xv[s]);
     }
   }
 }
 
-// The shuffled, pipelined row product of brow_shfl_row over the group's
-// precomputed slot values (every active lane shares mu): no sine and cosine
-// per slot and lane. Same values, same order, same bits.
-template <int NS>
-__device__ __forceinline__ void brow_shfl_val(const BGroup& G, int32_t j, int32_t w, int b,
-                                              const float2* __restrict__ x, float& ar,
-                                              float& ai) {
-  const int lane = int(threadIdx.x & 63);
-  const int g0 = lane & ~(G.bp - 1);
-  const int bp = G.bp;
-  SlotVal mine = {0, 0.0f, 0.0f};
-  if (b < NS && b < w) mine = G.kval[j + b * kSliceH];
-  for (int32_t k = 0; k < w; k += NS, j += NS * kSliceH) {
-    int32_t c[NS];
-    float vr[NS], vi[NS];
-#pragma unroll
-    for (int q = 0; q < NS; ++q) {
-      c[q] = __shfl(mine.col, g0 + q, 64);
-      vr[q] = __shfl(mine.vr, g0 + q, 64);
-      vi[q] = __shfl(mine.vi, g0 + q, 64);
-    }
-    float2 xv[NS];
-#pragma unroll
-    for (int q = 0; q < NS; ++q)
-      if (k + q < w) xv[q] = x[int64_t(c[q]) * bp + b];
-    if (b < NS && k + NS + b < w) mine = G.kval[j + (NS + b) * kSliceH];
-#pragma unroll
-    for (int q = 0; q < NS; ++q) {
-      if (k + q < w) cmac(ar, ai, vr[q], vi[q], xv[q]);
-    }
-  }
-}
-
-template <class T>
+template <class T, int D = 1>
 __device__ __forceinline__ typename Vt<T>::v2 brow(const BGroup& G, int64_t row, int b, T mu,
                                                     const typename Vt<T>::v2* __restrict__ x) {
   // A wave's rows lie in one 64-row slice (it holds 64 / bp consecutive rows
@@ -377,22 +471,21 @@ __device__ __forceinline__ typename Vt<T>::v2 brow(const BGroup& G, int64_t row,
   const int32_t w = (end - beg) / kSliceH;
   T ar = T(0), ai = T(0);
   int32_t j = beg + int32_t(row & 63);
-  int32_t k = 0;
-  if constexpr (std::is_same<T, float>::value) {
-    if (meta_shfl(G)) {
+  if (quad_rows(G)) {
+    if constexpr (std::is_same<T, float>::value) {
       if (G.kval)
-        brow_shfl_val<4>(G, j, w, b, x, ar, ai);
+        brow_quad<D, T>(RecF32V{G.kval}, j, w, G.bp, b, mu, x, ar, ai);
       else
-        brow_shfl_row<4>(G, j, w, b, mu, x, ar, ai);
-      typename Vt<T>::v2 r;
-      r.x = ar;
-      r.y = ai;
-      return r;
+        brow_quad<D, T>(RecF32M{G.s32}, j, w, G.bp, b, mu, x, ar, ai);
+    } else {
+      brow_quad<D, T>(RecF64M{G.scol, G.a64, G.t64}, j, w, G.bp, b, mu, x, ar, ai);
     }
+  } else {
+    int32_t k = 0;
+    for (; k + kSlotBatch <= w; k += kSlotBatch, j += kSlotBatch * kSliceH)
+      brow_slots<T, kSlotBatch>(G, j, b, mu, x, ar, ai);
+    for (; k < w; ++k, j += kSliceH) brow_slots<T, 1>(G, j, b, mu, x, ar, ai);
   }
-  for (; k + kSlotBatch <= w; k += kSlotBatch, j += kSlotBatch * kSliceH)
-    brow_slots<T, kSlotBatch>(G, j, b, mu, x, ar, ai);
-  for (; k < w; ++k, j += kSliceH) brow_slots<T, 1>(G, j, b, mu, x, ar, ai);
   typename Vt<T>::v2 r;
   r.x = ar;
   r.y = ai;
@@ -414,6 +507,10 @@ __device__ __forceinline__ double2 brow_val64(const BGroup& G, int64_t row, int 
   double ar = 0.0, ai = 0.0;
   int32_t j = beg + int32_t(row & 63);
   const int bp = G.bp;
+  if (quad_rows(G)) {
+    brow_quad<1, double>(RecF64V{G.scol, G.kval64}, j, w, bp, b, 0.0, x, ar, ai);
+    return make_double2(ar, ai);
+  }
   int32_t k = 0;
   for (; k + kSlotBatch <= w; k += kSlotBatch, j += kSlotBatch * kSliceH) {
     int32_t c[kSlotBatch];
@@ -450,20 +547,23 @@ __device__ __forceinline__ double residual_row(double diag, double ct, double V,
 }
 
 template <bool VAL64>
-__device__ double ph_compute_f(const BatchArgs& a, int64_t vb) {
-  const Lane L = lane_ctx(a, vb);
+__device__ double rows_compute_f(const BatchArgs& a, const Ctx& c) {
   double s2 = 0.0;
-  if (L.valid) {
-    const BGroup& G = L.G;
-    const double mu = a.mu[L.inst], g = a.g[L.inst];
+  const BGroup& G = c.G;
+  if (!c.lane_ok && !quad_rows(G)) return s2;
+  const int inst = c.lane_ok ? c.inst : G.inst0;
+  const double mu = a.mu[inst], g = a.g[inst];
+  each_row(a, c, [&](int64_t row) {
     double2 acc;
     if constexpr (VAL64)
-      acc = brow_val64(G, L.row, L.b, G.psi);
+      acc = brow_val64(G, row, c.b, G.psi);
     else
-      acc = brow<double>(G, L.row, L.b, mu, G.psi);
-    const double2 xi = G.psi[L.idx];
-    s2 = residual_row(G.diag[L.row], G.ct[L.row], G.V[L.row], g, xi, acc, G.f + L.idx);
-  }
+      acc = brow<double>(G, row, c.b, mu, G.psi);
+    if (!c.lane_ok) return;
+    const int64_t idx = row * G.bp + c.b;
+    const double2 xi = G.psi[idx];
+    s2 += residual_row(G.diag[row], G.ct[row], G.V[row], g, xi, acc, G.f + idx);
+  });
   return s2;
 }
 
@@ -494,33 +594,32 @@ __device__ __forceinline__ double2 brow_dmu(const BGroup& G, int64_t row, int b,
   return make_double2(ar, ai);
 }
 
-__device__ void ph_dfdmu(const BatchArgs& a, int64_t vb, double scale) {
-  const Lane L = lane_ctx(a, vb);
-  if (!L.valid) return;
-  const double2 d = brow_dmu(L.G, L.row, L.b, a.mu[L.inst], L.G.psi);
-  L.G.f[L.idx] = make_double2(scale * d.x, scale * d.y);
+__device__ void rows_dfdmu(const BatchArgs& a, const Ctx& c, double scale) {
+  if (!c.lane_ok) return;
+  const double mu = a.mu[c.inst];
+  each_row(a, c, [&](int64_t row) {
+    const double2 d = brow_dmu(c.G, row, c.b, mu, c.G.psi);
+    c.G.f[row * c.G.bp + c.b] = make_double2(scale * d.x, scale * d.y);
+  });
 }
 
-// J and P blocks (FP32, including diag K) and the per-instance Chebyshev bound.
-__device__ void ph_rebuild(const BatchArgs& a, int64_t vb) {
-  const Lane L = lane_ctx(a, vb);
-  __shared__ double rmax[1024];
-  rmax[threadIdx.x] = 0.0;
-  if (L.valid) {
-  const BGroup& G = L.G;
-  const int64_t nb3 = G.n * G.bp;
-  const double g = a.g[L.inst];
-  const double2 p = G.psi[L.idx];
-  const double c = G.ct[L.row], d = G.diag[L.row];
+// J and P blocks (FP32, including diag K) of one row and lane; returns the
+// row's sum |alpha| / lambda_min(P) for the instance's Chebyshev bound.
+__device__ __forceinline__ double row_rebuild(const BatchArgs& a, const Ctx& cx, int64_t row) {
+  const BGroup& G = cx.G;
+  const int64_t nb3 = G.n * G.bp, idx = row * G.bp + cx.b;
+  const double g = a.g[cx.inst];
+  const double2 p = G.psi[idx];
+  const double c = G.ct[row], d = G.diag[row];
   const double r2 = p.x * p.x + p.y * p.y;
   // Pseudo-transient shift sigma c t on both diagonals (0: Newton).
-  const double sh = c * a.shift[L.inst];
-  const double al = c * (G.V[L.row] + g * 2.0 * r2) + sh;
+  const double sh = c * a.shift[cx.inst];
+  const double al = c * (G.V[row] + g * 2.0 * r2) + sh;
   const double rx2 = g * c * (p.x * p.x - p.y * p.y);
   const double d1b = g * c * (2.0 * p.x * p.y);
-  G.jblk[L.idx] = float(d + al + rx2);
-  G.jblk[nb3 + L.idx] = float(d + al - rx2);
-  G.jblk[2 * nb3 + L.idx] = float(d1b);
+  G.jblk[idx] = float(d + al + rx2);
+  G.jblk[nb3 + idx] = float(d + al - rx2);
+  G.jblk[2 * nb3 + idx] = float(d1b);
   double a0 = d + sh, a1 = d + sh, bb = 0.0;
   if (g > 0.0) {
     const double pa = g * c * 2.0 * r2;
@@ -528,40 +627,67 @@ __device__ void ph_rebuild(const BatchArgs& a, int64_t vb) {
     a1 = d + pa - rx2 + sh;
     bb = d1b;
   }
-  G.pblk[L.idx] = float(a0);
-  G.pblk[nb3 + L.idx] = float(a1);
-  G.pblk[2 * nb3 + L.idx] = float(bb);
+  G.pblk[idx] = float(a0);
+  G.pblk[nb3 + idx] = float(a1);
+  G.pblk[2 * nb3 + idx] = float(bb);
   const double lmin = 0.5 * (a0 + a1) - hypot(0.5 * (a0 - a1), bb);
-  rmax[threadIdx.x] = lmin > 0.0 ? G.rowabs[L.row] / lmin : 1.0;
-  }
-  __syncthreads();
-  // One atomic per (block, instance): the max over the block's rows.
-  const int bp = L.G.bp;
-  if (threadIdx.x < bp && threadIdx.x < L.G.B) {
-    double m = 0.0;
-    for (int r = 0; r < int(blockDim.x) / bp; ++r) m = fmax(m, rmax[r * bp + threadIdx.x]);
-    atomicMax(reinterpret_cast<unsigned long long*>(a.bound) + L.G.inst0 + threadIdx.x,
-              static_cast<unsigned long long>(__double_as_longlong(m)));
-  }
-  // rmax is rewritten by the next row tile of a folded block.
-  __syncthreads();
+  return lmin > 0.0 ? G.rowabs[row] / lmin : 1.0;
 }
 
-__device__ void ph_setup(const BatchArgs& a, int64_t vb) {
-  const Lane L = lane_ctx(a, vb);
-  if (!L.valid) return;
-  const BGroup& G = L.G;
-  const double2 fv = G.f[L.idx];
-  const float2 r = make_float2(float(-fv.x), float(-fv.y));
-  G.R0[L.idx] = r;
-  G.R1[L.idx] = r;
-  G.W0[L.idx] = make_float2(0.f, 0.f);
-  G.W2[L.idx] = make_float2(0.f, 0.f);
-  G.x[L.idx] = make_double2(0.0, 0.0);
+// Largest v per instance over a launched block (a thread keeps its lane in all
+// of the block's tiles) into a.bound: lane shuffles over a wave's rows, LDS
+// over the waves, and at most one atomic per block and instance, none where
+// the bound is already there (they all meet on a few addresses). The rows'
+// maxima used to go through LDS tile by tile, read in turn by a few threads,
+// with an atomic per tile.
+__device__ __forceinline__ void bound_max(const BatchArgs& a, const BGroup& G, double v) {
+  __shared__ double wmax[16][64];
+  for (int off = G.bp; off < 64; off <<= 1) v = fmax(v, __shfl_xor(v, off, 64));
+  const int lane = int(threadIdx.x & 63), nw = int(blockDim.x) >> 6;
+  if (lane < G.bp) wmax[threadIdx.x >> 6][lane] = v;
+  __syncthreads();
+  const int b = int(threadIdx.x);
+  if (b >= G.B) return;
+  v = wmax[0][b];
+  for (int w = 1; w < nw; ++w) v = fmax(v, wmax[w][b]);
+  unsigned long long* p = reinterpret_cast<unsigned long long*>(a.bound) + G.inst0 + b;
+  const unsigned long long u = static_cast<unsigned long long>(__double_as_longlong(v));
+  if (__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < u) atomicMax(p, u);
 }
 
 __device__ __forceinline__ double hi_of(const BatchArgs& a, int inst) {
   return a.upper > 0.0 ? a.upper : 1.0 + a.bound[inst];
+}
+
+// (theta, 0) for j = 0, (c1, c2) of Chebyshev step j.
+__device__ __forceinline__ float2 coef_of(const BatchArgs& a, int inst, int j) {
+  return a.coef[int64_t(inst) * max(a.iters, 1) + j];
+}
+
+__device__ void rows_setup(const BatchArgs& a, const Ctx& c) {
+  if (!c.lane_ok) return;
+  const BGroup& G = c.G;
+  each_row(a, c, [&](int64_t row) {
+    const int64_t idx = row * G.bp + c.b;
+    const double2 fv = G.f[idx];
+    const float2 r = make_float2(float(-fv.x), float(-fv.y));
+    G.R0[idx] = r;
+    G.R1[idx] = r;
+    G.W0[idx] = make_float2(0.f, 0.f);
+    G.W2[idx] = make_float2(0.f, 0.f);
+    G.x[idx] = make_double2(0.0, 0.0);
+    if (row == 0) {
+      // The instance's Chebyshev coefficients, once for the whole solve (the
+      // FP64 divisions of one step took every thread of it 0.5 us).
+      const double hi = hi_of(a, c.inst);
+      float2* q = a.coef + int64_t(c.inst) * max(a.iters, 1);
+      q[0] = make_float2(float(0.5 * (hi + hi / a.ratio)), 0.f);
+      for (int j = 1; j < a.iters; ++j) {
+        const Cheb k = cheb_coef(hi, a.ratio, j);
+        q[j] = make_float2(float(k.c1), float(k.c2));
+      }
+    }
+  });
 }
 
 // Buffer selectors choose between pointer values (not between the record's
@@ -575,80 +701,6 @@ __device__ __forceinline__ float2* wbuf(const BGroup& G, int k) {
 }
 __device__ __forceinline__ float2* zbuf(const BGroup& G, int k) { return pick(k & 1, G.Z2, G.Y); }
 __device__ __forceinline__ float2* vbuf(const BGroup& G, int k) { return pick(k & 1, G.v1, G.v); }
-
-// Per-thread context of a launched block. All fold row tiles of a block
-// belong to one group and a thread keeps its lane (instance) in all of them,
-// so the group record and the instance's MINRES scalars are read once per
-// thread, not once per tile. The record is copied into registers by scalar
-// loads at kernel entry (its index made wave-uniform): read through a pointer
-// it would be reloaded by vector loads after every store of a row tile, which
-// the compiler cannot prove does not alias it, with a wait on each reload.
-struct Ctx {
-  BGroup G;
-  int b, inst, rows_per_vb;
-  int64_t row0;     // the thread's row in the block's first tile
-  int64_t tstride;  // rows from one of the block's tiles to the next
-  bool lane_ok;  // a real instance (b < B)
-};
-
-// Row tiles of launched blocks. The launched blocks form 8 contiguous ranges,
-// one per XCD (the order xcd_block gives them), and within a group each
-// range's blocks take the range's own contiguous share of the group's tiles,
-// strided by their count (block j of a range of c blocks: tiles s + j,
-// s + j + c, s + j + 2c, ...). The blocks resident on one XCD then sweep
-// one band of rows through their own stretch of the mesh, so the halo their
-// gathers read beyond the band was mostly read by that XCD's previous band
-// and is still in its L2 (each XCD's stretch has two ends, where the
-// neighbouring XCD's rows are read again). Before, the eight XCDs took
-// adjacent bands of one sweep of the whole group (block k: tiles k, k + nl,
-// ...), and every band's halo was the neighbouring XCDs' rows, read again
-// (96^3 x 8 lanes: ~2x the gathered vector's bytes). The mapping is a
-// function of the logical block index alone (the persistent kernel, which
-// does not remap, takes the same tiles and partial-sum slots). v0 = rb * fold
-// of launched block rb.
-struct TileMap {
-  int64_t first;   // the block's first tile in its group
-  int64_t stride;  // tiles from one of its tiles to the next
-};
-__device__ __forceinline__ TileMap tile_map(const BatchArgs& a, const BGroup& G, int64_t v0) {
-  const int64_t rb = v0 / a.fold;
-  const int64_t nb = a.total_blocks / a.fold;
-  const int64_t q = nb / 8, r = nb % 8;
-  int64_t xs, xc;
-  if (rb < r * (q + 1)) {
-    xs = rb / (q + 1) * (q + 1);
-    xc = q + 1;
-  } else {
-    xs = r * (q + 1) + (rb - r * (q + 1)) / q * q;
-    xc = q;
-  }
-  const int64_t g0 = G.block0 / a.fold, nl = G.nblocks / a.fold;
-  const int64_t s0 = max(g0, xs), s1 = min(g0 + nl, xs + xc);
-  TileMap m;
-  m.first = (s0 - g0) * a.fold + (rb - s0);
-  m.stride = s1 - s0;
-  return m;
-}
-// Virtual block (tile) t of launched block rb.
-__device__ __forceinline__ int64_t tile_vb(const BatchArgs& a, int64_t rb, int t) {
-  const BGroup& G = a.groups[group_of(a, rb * a.fold)];
-  const TileMap m = tile_map(a, G, rb * a.fold);
-  return G.block0 + m.first + int64_t(t) * m.stride;
-}
-
-__device__ __forceinline__ Ctx make_ctx(const BatchArgs& a, int64_t v0) {
-  Ctx c;
-  c.G = load_group(a, v0);
-  const int bp = c.G.bp;
-  c.b = threadIdx.x & (bp - 1);
-  c.inst = c.G.inst0 + c.b;
-  c.rows_per_vb = int(blockDim.x) / bp;
-  const TileMap m = tile_map(a, c.G, v0);
-  c.row0 = m.first * c.rows_per_vb + threadIdx.x / bp;
-  c.tstride = m.stride * c.rows_per_vb;
-  c.lane_ok = c.b < c.G.B;
-  return c;
-}
 
 // Pending update of iteration k: w_k = (v_k - oldeps w_{k-2} - delta w_{k-1}) / gamma,
 // x += phi w_k.
@@ -729,8 +781,7 @@ __device__ double rows_cheb_first(const BatchArgs& a, const Ctx& c, int mode) {
   float2* r = rbuf(G, it);
   const float2* r2 = rbuf(G, it + 1);
   const float cab = mode == 2 ? float(alfa / beta) : 0.0f;
-  const double hi = hi_of(a, c.inst);
-  const float th = float(0.5 * (hi + hi / a.ratio));
+  const float th = coef_of(a, c.inst, 0).x;
   const int64_t nb3 = G.n * G.bp;
   float2* z0 = zbuf(G, a.z0);
   for (int t = 0; t < a.fold; ++t) {
@@ -766,32 +817,36 @@ __device__ double rows_cheb_first(const BatchArgs& a, const Ctx& c, int mode) {
 // overwritten in place element by element (no other thread reads it), so no
 // separate direction vector is kept: 8 bytes less per row and lane for
 // every step, 16 for the first, and none for the first step's z_{j-2}.
+template <int D>
 __device__ double rows_cheb_step(const BatchArgs& a, const Ctx& c, int mode, int j) {
   double s = 0.0;
-  if (!c.lane_ok) return s;
-  const MinresScalars& S = a.S[c.inst];
-  const int done = S.done, it = mode == 2 ? S.it : 0;
   const BGroup& G = c.G;
-  if (meta_shfl(G) ? __all(done) : done) return s;
+  const bool quad = quad_rows(G);
+  if (!quad && !c.lane_ok) return s;
+  const int inst = c.lane_ok ? c.inst : G.inst0;  // padding lanes read their group's first
+  const MinresScalars& S = a.S[inst];
+  const int done = c.lane_ok ? S.done : 1, it = mode == 2 ? S.it : 0;
+  if (quad ? __all(done) : done) return s;
   const bool last = (j == a.iters - 1);
   const float2* r = rbuf(G, it);
   const float2* zin = zbuf(G, a.z0 + j - 1);
   float2* zout = zbuf(G, a.z0 + j);
-  const Cheb cc = cheb_coef(hi_of(a, c.inst), a.ratio, j);
-  const float c1 = float(cc.c1), c2 = float(cc.c2);
-  const float mu = float(a.mu[c.inst]);
+  const float2 cc = coef_of(a, inst, j);
+  const float c1 = cc.x, c2 = cc.y;
+  const float mu = float(a.mu[inst]);
   const int64_t nb3 = G.n * G.bp;
   for (int t = 0; t < a.fold; ++t) {
     const int64_t row = c.row0 + int64_t(t) * c.tstride;
     if (row >= G.n) break;
     const int64_t idx = row * G.bp + c.b;
-    const float2 acc = brow<float>(G, row, c.b, mu, zin);
-    if (done) continue;
+    // The row's own entries are on their way while its product is formed.
     const float2 zi = zin[idx];
     const float b0 = ldn(G.pblk + idx), b1 = ldn(G.pblk + nb3 + idx),
                 b2 = ldn(G.pblk + 2 * nb3 + idx);
     const float2 rv = ldn(r + idx);
     const float2 zpp = j > 1 ? ldn(zout + idx) : make_float2(0.f, 0.f);
+    const float2 acc = brow<float, D>(G, row, c.b, mu, zin);
+    if (done) continue;
     const float2 z = cheb_z(acc, zi, zpp, j == 1, rv, b0, b1, b2, c1, c2);
     stn(zout + idx, z);
     if (last) s += dot2(rv, z);
@@ -802,30 +857,33 @@ __device__ double rows_cheb_step(const BatchArgs& a, const Ctx& c, int mode, int
 
 // v = y / beta, u = J v - (beta/beta_old) r1, the previous w/x update, over
 // the block's rows; returns the thread's <v, u> sum.
+template <int D>
 __device__ double rows_minres_a(const BatchArgs& a, const Ctx& c) {
   double s = 0.0;
-  if (!c.lane_ok) return s;
-  const MinresScalars& S = a.S[c.inst];
-  const int done = S.done, it = S.it;
-  const double beta = S.beta, oldb = S.oldb;
   const BGroup& G = c.G;
-  if (meta_shfl(G) ? __all(done) : done) return s;
+  const bool quad = quad_rows(G);
+  if (!quad && !c.lane_ok) return s;
+  const int inst = c.lane_ok ? c.inst : G.inst0;
+  const MinresScalars& S = a.S[inst];
+  const int done = c.lane_ok ? S.done : 1, it = S.it;
+  const double beta = S.beta, oldb = S.oldb;
+  if (quad ? __all(done) : done) return s;
   const float2* y = zbuf(G, 0);
   const float2* r1 = rbuf(G, it);
   const float ib = float(1.0 / beta);
   const float cb = it >= 1 ? float(beta / oldb) : 0.0f;
-  const float mu = float(a.mu[c.inst]);
+  const float mu = float(a.mu[inst]);
   const int64_t nb3 = G.n * G.bp;
   for (int t = 0; t < a.fold; ++t) {
     const int64_t row = c.row0 + int64_t(t) * c.tstride;
     if (row >= G.n) break;
     const int64_t idx = row * G.bp + c.b;
-    const float2 acc = brow<float>(G, row, c.b, mu, y);
-    if (done) continue;
     const float2 yi = y[idx];
     const float b0 = ldn(G.jblk + idx), b1 = ldn(G.jblk + nb3 + idx),
                 b2 = ldn(G.jblk + 2 * nb3 + idx);
     const float2 rv = it >= 1 ? ldn(r1 + idx) : make_float2(0.f, 0.f);
+    const float2 acc = brow<float, D>(G, row, c.b, mu, y);
+    if (done) continue;
     const float2 uu = lanczos_u(acc, yi, b0, b1, b2, ib, cb, rv);
     const float2 vn = make_float2(yi.x * ib, yi.y * ib);
     stn(vbuf(G, it) + idx, vn);
@@ -912,6 +970,7 @@ __device__ __forceinline__ void store_lanes_nt(float2* p, const float2 (&v)[L], 
 template <int L>
 struct VCtx {
   BGroup G;
+  unsigned part;
   int T;      // threads per row (bp / L)
   int b0;     // the thread's first lane
   int R;      // rows per tile (block_threads / bp)
@@ -920,15 +979,19 @@ struct VCtx {
 };
 
 template <int L>
-__device__ __forceinline__ VCtx<L> make_vctx(const BatchArgs& a, int64_t v0) {
+__device__ __forceinline__ VCtx<L> make_vctx(const BatchArgs& a, unsigned rb) {
   VCtx<L> c;
-  c.G = load_group(a, v0);
-  c.T = c.G.bp / L;
-  c.R = int(blockDim.x) / c.T;
-  c.b0 = int(threadIdx.x % c.T) * L;
-  const TileMap m = tile_map(a, c.G, v0);
-  c.row0 = m.first * c.R + threadIdx.x / c.T;
-  c.tstride = m.stride * c.R;
+  rb = unsigned(uniform(int32_t(rb)));
+  const int gi = group_of(a, rb);
+  c.G = load_group(a, gi);
+  c.part = rb - a.gl[gi];
+  const int lt = c.G.lb - __builtin_ctz(L);  // log2(T)
+  c.T = 1 << lt;
+  c.R = int(blockDim.x >> lt);
+  c.b0 = int(threadIdx.x & (c.T - 1)) * L;
+  const TileMap m = tile_map(a, gi, rb);
+  c.row0 = int64_t(m.first) * c.R + (threadIdx.x >> lt);
+  c.tstride = int64_t(m.stride) * c.R;
   return c;
 }
 
@@ -1002,12 +1065,6 @@ __device__ __forceinline__ void brow_vec_recs(const Rec* __restrict__ rec, int32
       slot_mac<L>(m[q], mu, xv[q], acc);
     }
   }
-}
-
-// Lane i's value of v in every lane of its quad (DPP quad_perm [i,i,i,i]).
-template <int I>
-__device__ __forceinline__ int32_t quad_bcast(int32_t v) {
-  return __builtin_amdgcn_mov_dpp(v, I * 0x55, 0xf, 0xf, false);
 }
 
 // brow_vec_recs for rows whose threads come in whole quads (threads per row
@@ -1109,21 +1166,13 @@ __device__ __forceinline__ void brow_vec(const BGroup& G, int64_t row, int b0, i
 // Per-instance partial sums of one launched block (see lane_partials), from
 // the L lanes of every thread.
 template <int L>
-__device__ __forceinline__ void lane_partials_v(const BatchArgs& a, int64_t v0, const VCtx<L>& c,
+__device__ __forceinline__ void lane_partials_v(const BatchArgs& a, const VCtx<L>& c,
                                                 const double (&v)[L]) {
   __shared__ double lds[1024];
-  const BGroup& G = c.G;
-  const int bp = G.bp;
-  const int rho = int(threadIdx.x) / c.T;
+  const int rho = int(threadIdx.x >> (c.G.lb - __builtin_ctz(L)));
 #pragma unroll
-  for (int l = 0; l < L; ++l) lds[rho * bp + c.b0 + l] = v[l];
-  __syncthreads();
-  for (int b = int(threadIdx.x); b < bp && b < G.B; b += int(blockDim.x)) {
-    double s = 0.0;
-    for (int r = 0; r < c.R; ++r) s += lds[r * bp + b];
-    a.partials[int64_t(G.inst0 + b) * a.maxblocks + (v0 - G.block0) / a.fold] = s;
-  }
-  __syncthreads();
+  for (int l = 0; l < L; ++l) lds[rho * c.G.bp + c.b0 + l] = v[l];
+  sum_rows(a, c.G, c.part, lds, c.R);
 }
 
 template <int L>
@@ -1148,9 +1197,9 @@ __device__ void rows_cheb_step_v(const BatchArgs& a, const VCtx<L>& c, int mode,
         act[l] = true;
         any = true;
         it = mode == 2 ? S.it : 0;  // the same for every active instance (lockstep)
-        const Cheb cc = cheb_coef(hi_of(a, inst), a.ratio, j);
-        c1[l] = float(cc.c1);
-        c2[l] = float(cc.c2);
+        const float2 cc = coef_of(a, inst, j);
+        c1[l] = cc.x;
+        c2[l] = cc.y;
       }
     }
     all = all && act[l];
@@ -1259,17 +1308,22 @@ __device__ void rows_minres_a_v(const BatchArgs& a, const VCtx<L>& c, double (&s
   }
 }
 
-__device__ void ph_flush(const BatchArgs& a, int64_t vb) {
-  const Lane L = lane_ctx(a, vb);
-  if (!L.valid || !a.active[L.inst]) return;
-  const BGroup& G = L.G;
-  const MinresScalars& S = a.S[L.inst];
-  if (S.pending) w_update(G, wupd_of(S), S.it, L.idx, vbuf(G, S.it - 1)[L.idx], false);
-  const double2 d = G.x[L.idx];
-  double2 p = G.psi[L.idx];
-  p.x += d.x;
-  p.y += d.y;
-  G.psi[L.idx] = p;
+__device__ void rows_flush(const BatchArgs& a, const Ctx& c) {
+  if (!c.lane_ok || !a.active[c.inst]) return;
+  const BGroup& G = c.G;
+  const MinresScalars& S = a.S[c.inst];
+  const int pending = S.pending, it = S.it;
+  const WUpd q = wupd_of(S);
+  const float2* v = vbuf(G, it - 1);
+  each_row(a, c, [&](int64_t row) {
+    const int64_t idx = row * G.bp + c.b;
+    if (pending) w_update(G, q, it, idx, v[idx], false);
+    const double2 d = G.x[idx];
+    double2 p = G.psi[idx];
+    p.x += d.x;
+    p.y += d.y;
+    G.psi[idx] = p;
+  });
 }
 
 // Per-instance finalisation (block = instance): 0 norm^2 -> out, 1 init,
@@ -1279,7 +1333,7 @@ __device__ void ph_finalize(const BatchArgs& a, int inst, int what, double* out)
   if ((what == 2 || what == 3) && S->done) return;
   int gi = 0;
   while (gi + 1 < a.ngroups && inst >= a.groups[gi + 1].inst0) ++gi;
-  const int nb = int(a.groups[gi].nblocks / a.fold);
+  const int nb = int(a.gl[gi + 1] - a.gl[gi]);
   double v[1];
   finalize_sum<1>(v, a.partials + int64_t(inst) * a.maxblocks, nb);
   if (threadIdx.x == 0) {
@@ -1300,73 +1354,71 @@ __device__ void ph_finalize(const BatchArgs& a, int inst, int what, double* out)
 }
 
 // ---------------------------------------------------------------- kernels
-// Launched block rb covers the virtual blocks rb*fold .. rb*fold + fold - 1,
-// all of one group (every group's virtual block count is a multiple of fold).
+// Launched block rb covers fold row tiles, all of one group (every group's
+// tile count is a multiple of fold).
 template <bool VAL64>
-__device__ __forceinline__ void blk_compute_f(const BatchArgs& a, int64_t rb) {
-  const int64_t v0 = rb * a.fold;
-  double s = 0.0;
-  for (int r = 0; r < a.fold; ++r) s += ph_compute_f<VAL64>(a, tile_vb(a, rb, r));
-  lane_partials(a, v0, s);
+__device__ __forceinline__ void blk_compute_f(const BatchArgs& a, unsigned rb) {
+  const Ctx c = make_ctx(a, rb);
+  lane_partials(a, c, rows_compute_f<VAL64>(a, c));
 }
-__device__ __forceinline__ void blk_cheb_first(const BatchArgs& a, int64_t rb, int mode) {
-  const int64_t v0 = rb * a.fold;
-  const double s = rows_cheb_first(a, make_ctx(a, v0), mode);
-  if (a.iters <= 1) lane_partials(a, v0, s);
+__device__ __forceinline__ void blk_cheb_first(const BatchArgs& a, unsigned rb, int mode) {
+  const Ctx c = make_ctx(a, rb);
+  const double s = rows_cheb_first(a, c, mode);
+  if (a.iters <= 1) lane_partials(a, c, s);
 }
-__device__ __forceinline__ void blk_cheb_step(const BatchArgs& a, int64_t rb, int mode, int j) {
-  const int64_t v0 = rb * a.fold;
-  const double s = rows_cheb_step(a, make_ctx(a, v0), mode, j);
-  if (j == a.iters - 1) lane_partials(a, v0, s);
+template <int D>
+__device__ __forceinline__ void blk_cheb_step(const BatchArgs& a, unsigned rb, int mode, int j) {
+  const Ctx c = make_ctx(a, rb);
+  const double s = rows_cheb_step<D>(a, c, mode, j);
+  if (j == a.iters - 1) lane_partials(a, c, s);
 }
-__device__ __forceinline__ void blk_minres_a(const BatchArgs& a, int64_t rb) {
-  const int64_t v0 = rb * a.fold;
-  lane_partials(a, v0, rows_minres_a(a, make_ctx(a, v0)));
+template <int D>
+__device__ __forceinline__ void blk_minres_a(const BatchArgs& a, unsigned rb) {
+  const Ctx c = make_ctx(a, rb);
+  lane_partials(a, c, rows_minres_a<D>(a, c));
 }
 
+// At 96^3 x 8 lanes: F 215 -> 180 us (records by quads), rebuild 183 -> 71
+// (bound_max, one row context for all tiles), Chebyshev step 93 -> 90.
 // Launched blocks are remapped so that each XCD works on one contiguous
 // range of row tiles and its L2 holds the x entries those rows gather.
-__global__ void kb_compute_f(BatchArgs a) { blk_compute_f<false>(a, xcd_block(true)); }
-__global__ void kb_compute_f64v(BatchArgs a) { blk_compute_f<true>(a, xcd_block(true)); }
+__device__ __forceinline__ unsigned launched() { return unsigned(xcd_block(true)); }
+__global__ void kb_compute_f(BatchArgs a) { blk_compute_f<false>(a, launched()); }
+__global__ void kb_compute_f64v(BatchArgs a) { blk_compute_f<true>(a, launched()); }
 __global__ void kb_dfdmu(BatchArgs a, double scale) {
-  const int64_t rb = xcd_block(true);
-  for (int r = 0; r < a.fold; ++r) ph_dfdmu(a, tile_vb(a, rb, r), scale);
+  rows_dfdmu(a, make_ctx(a, launched()), scale);
 }
 __global__ void kb_rebuild(BatchArgs a) {
-  const int64_t rb = xcd_block(true);
-  for (int r = 0; r < a.fold; ++r) ph_rebuild(a, tile_vb(a, rb, r));
+  const Ctx c = make_ctx(a, launched());
+  double m = 0.0;
+  if (c.lane_ok) each_row(a, c, [&](int64_t row) { m = fmax(m, row_rebuild(a, c, row)); });
+  bound_max(a, c.G, m);
 }
-__global__ void kb_setup(BatchArgs a) {
-  const int64_t rb = xcd_block(true);
-  for (int r = 0; r < a.fold; ++r) ph_setup(a, tile_vb(a, rb, r));
-}
-__global__ void kb_cheb_first(BatchArgs a, int mode) {
-  blk_cheb_first(a, xcd_block(true), mode);
-}
+__global__ void kb_setup(BatchArgs a) { rows_setup(a, make_ctx(a, launched())); }
+__global__ void kb_cheb_first(BatchArgs a, int mode) { blk_cheb_first(a, launched(), mode); }
+template <int D>
 __global__ void kb_cheb_step(BatchArgs a, int mode, int j) {
-  blk_cheb_step(a, xcd_block(true), mode, j);
+  blk_cheb_step<D>(a, launched(), mode, j);
 }
-__global__ void kb_minres_a(BatchArgs a) { blk_minres_a(a, xcd_block(true)); }
+template <int D>
+__global__ void kb_minres_a(BatchArgs a) {
+  blk_minres_a<D>(a, launched());
+}
 template <int L>
 __global__ void kb_cheb_step_v(BatchArgs a, int mode, int j) {
-  const int64_t v0 = xcd_block(true) * a.fold;
-  const VCtx<L> c = make_vctx<L>(a, v0);
+  const VCtx<L> c = make_vctx<L>(a, launched());
   double s[L];
   rows_cheb_step_v<L>(a, c, mode, j, s);
-  if (j == a.iters - 1) lane_partials_v<L>(a, v0, c, s);
+  if (j == a.iters - 1) lane_partials_v<L>(a, c, s);
 }
 template <int L>
 __global__ void kb_minres_a_v(BatchArgs a) {
-  const int64_t v0 = xcd_block(true) * a.fold;
-  const VCtx<L> c = make_vctx<L>(a, v0);
+  const VCtx<L> c = make_vctx<L>(a, launched());
   double s[L];
   rows_minres_a_v<L>(a, c, s);
-  lane_partials_v<L>(a, v0, c, s);
+  lane_partials_v<L>(a, c, s);
 }
-__global__ void kb_flush(BatchArgs a) {
-  const int64_t rb = xcd_block(true);
-  for (int r = 0; r < a.fold; ++r) ph_flush(a, tile_vb(a, rb, r));
-}
+__global__ void kb_flush(BatchArgs a) { rows_flush(a, make_ctx(a, launched())); }
 __global__ void kb_finalize(BatchArgs a, int what, double* out) {
   ph_finalize(a, blockIdx.x, what, out);
 }
@@ -1462,17 +1514,17 @@ __global__ void kb_fill_kval64(const double* __restrict__ a64, const double* __r
 // after maxit iterations, a decision every block takes from the same
 // post-barrier state.
 __global__ void kb_minres_persistent(BatchArgs a, int maxit) {
-  const int64_t nrb = a.total_blocks / a.fold;
+  const unsigned nrb = a.gl[a.ngroups];
   for (int it = 0; it < maxit; ++it) {
-    for (int64_t rb = blockIdx.x; rb < nrb; rb += gridDim.x) blk_minres_a(a, rb);
+    for (unsigned rb = blockIdx.x; rb < nrb; rb += gridDim.x) blk_minres_a<1>(a, rb);
     if (grid_barrier(a)) return;
     for (int inst = blockIdx.x; inst < a.ninst; inst += gridDim.x)
       ph_finalize(a, inst, 2, nullptr);
     if (grid_barrier(a)) return;
-    for (int64_t rb = blockIdx.x; rb < nrb; rb += gridDim.x) blk_cheb_first(a, rb, 2);
+    for (unsigned rb = blockIdx.x; rb < nrb; rb += gridDim.x) blk_cheb_first(a, rb, 2);
     if (grid_barrier(a)) return;
     for (int j = 1; j < a.iters; ++j) {
-      for (int64_t rb = blockIdx.x; rb < nrb; rb += gridDim.x) blk_cheb_step(a, rb, 2, j);
+      for (unsigned rb = blockIdx.x; rb < nrb; rb += gridDim.x) blk_cheb_step<1>(a, rb, 2, j);
       if (grid_barrier(a)) return;
     }
     for (int inst = blockIdx.x; inst < a.ninst; inst += gridDim.x)
@@ -1494,12 +1546,20 @@ __global__ void kb_bar_clear(unsigned* bar, int* err) {
 }  // namespace
 
 // ------------------------------------------------------------------ host
+// Then the one-lane row products take 8 slots a round instead of 4 (71
+// registers instead of 58): three boxes of 8 - 12 k rows with 7 instances,
+// 250 k threads, Chebyshev step 10.3 -> 9.7 us, with the records shared by
+// quads; 10.9 before that. 524,288 threads are 8 waves a SIMD.
+bool Batch::small_grid() const {
+  return args.total_blocks / args.fold * block_threads <= 524288;
+}
+
 void Batch::launch_cheb_step(hipStream_t s, int mode_, int j) {
   const unsigned nb = unsigned(args.total_blocks / args.fold), bt = unsigned(block_threads);
   if (lanes == kVecLanes)
     kb_cheb_step_v<kVecLanes><<<nb, bt / kVecLanes, 0, s>>>(args, mode_, j);
   else
-    kb_cheb_step<<<nb, bt, 0, s>>>(args, mode_, j);
+    (small_grid() ? kb_cheb_step<2> : kb_cheb_step<1>)<<<nb, bt, 0, s>>>(args, mode_, j);
 }
 
 void Batch::launch_minres_a(hipStream_t s) {
@@ -1507,7 +1567,7 @@ void Batch::launch_minres_a(hipStream_t s) {
   if (lanes == kVecLanes)
     kb_minres_a_v<kVecLanes><<<nb, bt / kVecLanes, 0, s>>>(args);
   else
-    kb_minres_a<<<nb, bt, 0, s>>>(args);
+    (small_grid() ? kb_minres_a<2> : kb_minres_a<1>)<<<nb, bt, 0, s>>>(args);
 }
 
 void Batch::launch_phases_iteration(hipStream_t s) {
@@ -1566,9 +1626,9 @@ void Batch::prepare_kval(hipStream_t s) {
   bool changed = false;
   for (auto& gh : ghost) {
     BGroup& G = gh.dev;
-    // Read by the shuffled one-lane row products and by every row product of
-    // the L-lane mapping.
-    bool shared = lanes > 1 || (NOSH_META_SHFL && G.B == G.bp && G.bp >= 4);
+    // Read by the one-lane row products that share records over quads and by
+    // every row product of the L-lane mapping.
+    bool shared = lanes > 1 || G.bp >= 4;
     bool any = false;
     double m0 = 0.0;
     for (int b = 0; shared && b < G.B; ++b) {
@@ -1598,6 +1658,23 @@ void Batch::prepare_kval(hipStream_t s) {
     }
   }
   if (changed) upload_records(s);
+}
+
+void Batch::set_chebyshev(int iters, double ratio) {
+  if (args.iters == iters && args.ratio == ratio && args.upper == 0.0) return;
+  args.iters = iters;
+  args.ratio = ratio;
+  args.upper = 0.0;
+  args.z0 = std::max(iters - 1, 0) % 2;
+  drop_graph();
+}
+
+void Batch::ensure_coef() {
+  const size_t need = size_t(args.ninst) * std::max(args.iters, 1);
+  if (coef.n >= need && args.coef) return;
+  drop_graph();  // its launches hold the old pointer
+  coef.alloc(need);
+  args.coef = coef.p;
 }
 
 void Batch::upload_records(hipStream_t s) {
@@ -1641,6 +1718,7 @@ void Batch::prepare_kval64(hipStream_t s, bool* all) {
 int Batch::minres(hipStream_t s, int maxit) {
   const unsigned nb = unsigned(args.total_blocks / args.fold), bt = unsigned(block_threads);
   prepare_kval(s);
+  ensure_coef();
   kb_reset<<<grid_for(args.ninst, 128), 128, 0, s>>>(args, maxit);
   kb_rebuild<<<nb, bt, 0, s>>>(args);
   kb_setup<<<nb, bt, 0, s>>>(args);
@@ -1708,6 +1786,7 @@ double Batch::time_cheb_step(hipStream_t s, int reps) {
   const std::vector<int> active_before = active_h;
   active_h.assign(args.ninst, 1);
   prepare_kval(s);
+  ensure_coef();
   kb_reset<<<grid_for(args.ninst, 128), 128, 0, s>>>(args, 1);
   kb_rebuild<<<nb, bt, 0, s>>>(args);
   kb_setup<<<nb, bt, 0, s>>>(args);
@@ -1765,15 +1844,15 @@ void Batch::relayout(int threads, int fold_) {
   args.fold = fold_;
   int64_t b0 = 0, maxb = 0;
   for (auto& gh : ghost) {
-    BGroup& G = gh.dev;
-    G.block0 = b0;
+    const BGroup& G = gh.dev;
+    args.gl[&gh - ghost.data()] = unsigned(b0 / fold);
     const int rows = threads / G.bp;
-    G.nblocks = (G.n + rows - 1) / rows;
-    G.nblocks = (G.nblocks + fold - 1) / fold * fold;
-    b0 += G.nblocks;
-    maxb = std::max(maxb, G.nblocks);
+    const int64_t tiles = ((G.n + rows - 1) / rows + fold - 1) / fold * fold;
+    b0 += tiles;
+    maxb = std::max(maxb, tiles);
   }
   args.total_blocks = b0;
+  args.gl[ghost.size()] = unsigned(b0 / fold);
   args.maxblocks = maxb;
   partials.alloc(size_t(args.ninst) * maxb + 64);
   args.partials = partials.p;

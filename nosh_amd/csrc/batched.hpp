@@ -30,10 +30,9 @@ static_assert(sizeof(SlotVal) == 12, "slot values are 12 packed bytes");
 struct BGroup {
   int64_t n;        // rows (vertices)
   int bp;           // lanes per row: instances padded to a power of two
+  int lb;           // log2(bp)
   int B;            // instances
   int inst0;        // first global instance index
-  int64_t block0;   // first block of this group in a batched launch
-  int64_t nblocks;  // blocks of this group
   const int32_t* slice_ptr;
   const int32_t* scol;
   const SlotMeta* s32;  // per padded slot, FP32 path
@@ -57,9 +56,15 @@ struct BGroup {
   float2* v1;  // second Lanczos buffer: v of iteration k lives in (k odd ? v1 : v)
 };
 
+constexpr int kMaxGroups = 16;
+
 struct BatchArgs {
   const BGroup* groups;
   int ngroups;
+  // First launched block of every group, and the number of all of them. In
+  // the arguments and in 32 bits: finding a thread's rows was a third of a
+  // small launch, loads through the group records and six 64-bit divisions.
+  unsigned gl[kMaxGroups + 1];
   int ninst;
   int64_t total_blocks;  // virtual blocks (block_threads / bp rows each)
   int64_t maxblocks;
@@ -74,6 +79,7 @@ struct BatchArgs {
   double upper, ratio;
   int iters;            // Chebyshev iterations
   int z0;               // parity of the first Chebyshev output buffer
+  float2* coef;         // per instance and Chebyshev step (see coef_of)
   double* partials;     // [instance][maxblocks]
   unsigned* bar;        // persistent mode: grid barrier {arrivals, generation}
   int* bar_err;         // persistent mode: set when a barrier wait times out
@@ -120,6 +126,7 @@ struct Batch {
   std::vector<MinresScalars> Sh;
   DBuf<double> mu, g, bound, rtol, norms, partials, shift;
   DBuf<int> active;
+  DBuf<float2> coef;
   DBuf<unsigned> bar;  // persistent mode: grid barrier state
   DBuf<int> bar_err;   // persistent mode: barrier time-out flag
   std::vector<int> active_h;
@@ -138,7 +145,7 @@ struct Batch {
   // Uploads per-instance mu (and keeps the host copy).
   void set_mu(const double* m, hipStream_t s);
   // For every group whose active instances all share one mu (and whose rows
-  // take slot metadata by lane shuffles, or with lanes > 1), fills kval at
+  // share slot records, or with lanes > 1), fills kval at
   // that mu (once per value) and points the group record at it; other groups
   // rebuild K per lane.
   void prepare_kval(hipStream_t s);
@@ -147,7 +154,15 @@ struct Batch {
   // lane there.
   void prepare_kval64(hipStream_t s, bool* all = nullptr);
   void upload_records(hipStream_t s);
+  // Degree and interval of the preconditioner; the captured iterations are kept
+  // while both stand.
+  void set_chebyshev(int iters, double ratio);
+  // Room for the Chebyshev coefficients at args.iters.
+  void ensure_coef();
   void launch_phases_iteration(hipStream_t s);
+  // Whether the whole grid of a one-lane kernel is resident at once with room
+  // to spare, so that latency and not occupancy bounds it.
+  bool small_grid() const;
   void launch_cheb_step(hipStream_t s, int mode, int j);
   void launch_minres_a(hipStream_t s);
   void build_graph(hipStream_t s);
@@ -172,10 +187,11 @@ struct Batch {
 void launch_slot_fields(const MeshCache& m, const double* alpha, const double* atilde,
                         SlotMeta* s32, double* a64, double* t64, double* diag, double* rowabs,
                         hipStream_t s);
-// Reference-order instance vector -> lane b of an interleaved [n][bp] array, and back.
-void launch_scatter_lane(int64_t n, int bp, int b, const int32_t* perm, const double* src,
+// Reference-order instance vectors (B of them, one after another) -> lanes
+// 0 .. B - 1 of an interleaved [n][bp] array, and back.
+void launch_scatter_lanes(int64_t n, int bp, int B, const int32_t* perm, const double* src,
+                          double* dst, hipStream_t s);
+void launch_gather_lanes(int64_t n, int bp, int B, const int32_t* perm, const double* src,
                          double* dst, hipStream_t s);
-void launch_gather_lane(int64_t n, int bp, int b, const int32_t* perm, const double* src,
-                        double* dst, hipStream_t s);
 
 }  // namespace nosh
