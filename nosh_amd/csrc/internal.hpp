@@ -23,6 +23,7 @@ constexpr int kSliceH = 64;
 // reference edge id e coded as 2e (row = lower endpoint) or 2e+1 (row =
 // higher endpoint), -1 for padding (col = own row, value 0).
 struct MeshCache {
+  std::vector<Slab> slabs;  // hold the arrays below
   int nv = 3, ne = 3;
   int64_t n = 0, E = 0, T = 0;
   DBuf<double> coords;      // 3n

@@ -544,32 +544,45 @@ __global__ void k_invert_perm(const int32_t* __restrict__ perm, int64_t n,
   if (i < n) iperm[perm[i]] = int32_t(i);
 }
 
+// hipCUB passes with their scratch in a slab, which the next pass on the
+// stream reuses.
 template <class K, class V>
-void sort_pairs(const K* kin, K* kout, const V* vin, V* vout, int64_t N, int end_bit,
+void sort_pairs(const K* kin, K* kout, const V* vin, V* vout, int64_t N, int end_bit, Slab& tmp,
                 hipStream_t s) {
-  size_t tmp = 0;
-  NOSH_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp, kin, kout, vin, vout, int(N), 0,
+  size_t bytes = 0;
+  NOSH_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, bytes, kin, kout, vin, vout, int(N), 0,
                                               end_bit, s));
-  DBuf<char> t(tmp + 16);
-  NOSH_HIP(hipcub::DeviceRadixSort::SortPairs(t.p, tmp, kin, kout, vin, vout, int(N), 0,
-                                              end_bit, s));
-  NOSH_HIP(hipStreamSynchronize(s));
+  const size_t m = tmp.mark();
+  NOSH_HIP(hipcub::DeviceRadixSort::SortPairs(tmp.take<char>(bytes + 16), bytes, kin, kout, vin,
+                                              vout, int(N), 0, end_bit, s));
+  tmp.reset(m);
 }
 
-void inclusive_sum(const int32_t* in, int32_t* out, int64_t N, hipStream_t s) {
-  size_t tmp = 0;
-  NOSH_HIP(hipcub::DeviceScan::InclusiveSum(nullptr, tmp, in, out, int(N), s));
-  DBuf<char> t(tmp + 16);
-  NOSH_HIP(hipcub::DeviceScan::InclusiveSum(t.p, tmp, in, out, int(N), s));
-  NOSH_HIP(hipStreamSynchronize(s));
+void inclusive_sum(const int32_t* in, int32_t* out, int64_t N, Slab& tmp, hipStream_t s) {
+  size_t bytes = 0;
+  NOSH_HIP(hipcub::DeviceScan::InclusiveSum(nullptr, bytes, in, out, int(N), s));
+  const size_t m = tmp.mark();
+  NOSH_HIP(hipcub::DeviceScan::InclusiveSum(tmp.take<char>(bytes + 16), bytes, in, out, int(N), s));
+  tmp.reset(m);
 }
 
-void exclusive_sum(const int32_t* in, int32_t* out, int64_t N, hipStream_t s) {
-  size_t tmp = 0;
-  NOSH_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, in, out, int(N), s));
-  DBuf<char> t(tmp + 16);
-  NOSH_HIP(hipcub::DeviceScan::ExclusiveSum(t.p, tmp, in, out, int(N), s));
+void exclusive_sum(const int32_t* in, int32_t* out, int64_t N, Slab& tmp, hipStream_t s) {
+  size_t bytes = 0;
+  NOSH_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, in, out, int(N), s));
+  const size_t m = tmp.mark();
+  NOSH_HIP(hipcub::DeviceScan::ExclusiveSum(tmp.take<char>(bytes + 16), bytes, in, out, int(N), s));
+  tmp.reset(m);
+}
+
+int32_t read_i32(const int32_t* p, hipStream_t s) {
+  int32_t v = 0;
+  NOSH_HIP(hipMemcpyAsync(&v, p, 4, hipMemcpyDeviceToHost, s));
   NOSH_HIP(hipStreamSynchronize(s));
+  return v;
+}
+
+void zero_i32(int32_t* p, int64_t n, hipStream_t s) {
+  k_fill_i32<<<grid_for(n, kBlock), kBlock, 0, s>>>(p, n, 0);
 }
 
 int bits_for(uint64_t maxval) {
@@ -581,47 +594,46 @@ int bits_for(uint64_t maxval) {
 // Reverse Cuthill-McKee over a symmetric CSR graph (host). Start vertices
 // are pseudo-peripheral (George-Liu); neighbours are visited by ascending
 // degree, ties by ascending vertex id; components in order of their
-// lowest-numbered vertex.
-std::vector<int32_t> rcm_order(int64_t n, const std::vector<int32_t>& ptr,
-                               const std::vector<int32_t>& adj) {
-  std::vector<int32_t> deg(n);
-  for (int64_t v = 0; v < n; ++v) deg[v] = ptr[v + 1] - ptr[v];
-  std::vector<char> done(n, 0);
-  std::vector<int32_t> order;
-  order.reserve(n);
-  std::vector<int32_t> level(n, -1), touched;
+// lowest-numbered vertex. The searches run in one queue whose levels are
+// ranges of it, visits marked by the search's number. (With a vector per
+// level the 6.6 ms of RCM were a third of building a 117 k vertex mesh.)
+std::vector<int32_t> rcm_order(int64_t n, const int32_t* ptr, const int32_t* adj) {
+  std::vector<int32_t> seen(n, 0), queue(n);
+  int32_t search = 0;
+  auto deg = [&](int32_t v) { return ptr[v + 1] - ptr[v]; };
+  // The min-degree vertex (lowest id) of the last level from root, and the depth.
   auto bfs_last_level = [&](int32_t root, int* ecc) {
-    // Returns the min-degree vertex of the last BFS level from root.
-    touched.clear();
-    std::vector<int32_t> frontier{root}, next;
-    level[root] = 0;
-    touched.push_back(root);
+    ++search;
+    int32_t* const q = queue.data();
+    int64_t lo = 0, hi = 1;
+    q[0] = root;
+    seen[root] = search;
     int depth = 0;
-    std::vector<int32_t> last = frontier;
-    while (!frontier.empty()) {
-      next.clear();
-      for (int32_t v : frontier)
-        for (int32_t q = ptr[v]; q < ptr[v + 1]; ++q) {
-          const int32_t w = adj[q];
-          if (level[w] < 0) {
-            level[w] = depth + 1;
-            touched.push_back(w);
-            next.push_back(w);
+    for (;;) {
+      int64_t tail = hi;
+      for (int64_t i = lo; i < hi; ++i)
+        for (int32_t e = ptr[q[i]]; e < ptr[q[i] + 1]; ++e) {
+          const int32_t w = adj[e];
+          if (seen[w] != search) {
+            seen[w] = search;
+            q[tail++] = w;
           }
         }
-      if (next.empty()) break;
+      if (tail == hi) break;
       ++depth;
-      last = next;
-      frontier.swap(next);
+      lo = hi;
+      hi = tail;
     }
-    for (int32_t v : touched) level[v] = -1;
     *ecc = depth;
-    int32_t best = last[0];
-    for (int32_t v : last)
-      if (deg[v] < deg[best] || (deg[v] == deg[best] && v < best)) best = v;
+    int32_t best = q[lo];
+    for (int64_t i = lo; i < hi; ++i)
+      if (deg(q[i]) < deg(best) || (deg(q[i]) == deg(best) && q[i] < best)) best = q[i];
     return best;
   };
-  std::vector<int32_t> nb;
+  std::vector<char> done(n, 0);
+  std::vector<int32_t> order(n);
+  int64_t tail = 0;
+  std::vector<uint64_t> nb;
   for (int64_t seed = 0; seed < n; ++seed) {
     if (done[seed]) continue;
     int32_t root = int32_t(seed);
@@ -630,29 +642,25 @@ std::vector<int32_t> rcm_order(int64_t n, const std::vector<int32_t>& ptr,
     for (int iter = 0; iter < 8; ++iter) {
       int ecc2 = 0;
       const int32_t cand2 = bfs_last_level(cand, &ecc2);
-      if (ecc2 <= ecc) {
-        root = cand;
-        break;
-      }
       root = cand;
+      if (ecc2 <= ecc) break;
       ecc = ecc2;
       cand = cand2;
     }
-    size_t head = order.size();
-    order.push_back(root);
+    int64_t head = tail;
+    order[tail++] = root;
     done[root] = 1;
-    while (head < order.size()) {
+    while (head < tail) {
       const int32_t v = order[head++];
       nb.clear();
-      for (int32_t q = ptr[v]; q < ptr[v + 1]; ++q)
-        if (!done[adj[q]]) nb.push_back(adj[q]);
-      std::sort(nb.begin(), nb.end(), [&](int32_t a, int32_t b) {
-        return deg[a] != deg[b] ? deg[a] < deg[b] : a < b;
-      });
-      for (int32_t w : nb) {
+      for (int32_t e = ptr[v]; e < ptr[v + 1]; ++e) {
+        const int32_t w = adj[e];
+        if (done[w]) continue;
         done[w] = 1;
-        order.push_back(w);
+        nb.push_back(uint64_t(uint32_t(deg(w))) << 32 | uint32_t(w));
       }
+      if (nb.size() > 1) std::sort(nb.begin(), nb.end());
+      for (uint64_t w : nb) order[tail++] = int32_t(uint32_t(w));
     }
   }
   std::reverse(order.begin(), order.end());
@@ -668,189 +676,221 @@ std::unique_ptr<MeshCache> build_mesh_cache(const double* coords, int64_t n, con
   const int ne = nv == 3 ? 3 : 6;
   NOSH_CHECK(T * ne < (int64_t(1) << 31) && n < (int64_t(1) << 31), kInvalid,
              "mesh too large for 32-bit slot indices");
-  for (int64_t i = 0; i < T * nv; ++i)
-    NOSH_CHECK(cells[i] >= 0 && cells[i] < n, kInvalid, "cell vertex index out of range");
+  int32_t cmin = 0, cmax = 0;
+  for (int64_t i = 0; i < T * nv; ++i) {
+    cmin = std::min(cmin, cells[i]);
+    cmax = std::max(cmax, cells[i]);
+  }
+  NOSH_CHECK(cmin >= 0 && cmax < n, kInvalid, "cell vertex index out of range");
   auto m = std::make_unique<MeshCache>();
   m->nv = nv;
   m->ne = ne;
   m->n = n;
   m->T = T;
-  m->coords.alloc(3 * n);
+  const int64_t N = T * ne, Nv = T * nv;
+  const int64_t ns = (n + kSliceH - 1) / kSliceH;
+  m->nslices = ns;
+  m->slabs.reserve(3);
+  {
+    Slab& k = m->slabs.emplace_back(slab_bytes<double>(3 * n) + 2 * slab_bytes<double>(n) +
+                                    slab_bytes<int32_t>(Nv) + slab_bytes<int32_t>(N) +
+                                    2 * slab_bytes<int32_t>(n) + 3 * slab_bytes<int32_t>(ns + 1));
+    k.take(m->coords, 3 * n);
+    k.take(m->cells, Nv);
+    k.take(m->cell_edges, N);
+    k.take(m->cv, n);
+    k.take(m->cv_int, n);
+    k.take(m->perm, n);
+    k.take(m->iperm, n);
+    k.take(m->slice_ptr, ns + 1);
+    k.take(m->uptr, ns + 1);
+    k.take(m->lptr, ns + 1);
+  }
   m->coords.upload(coords, 3 * n, s);
-  m->cells.alloc(T * nv);
-  m->cells.upload(cells, T * nv, s);
+  m->cells.upload(cells, Nv, s);
 
-  const int64_t N = T * ne;
+  // Scratch of the whole build in one allocation, the arrays that stay in three:
+  // some seventy of them, each with its release and the wait that brings,
+  // took 10 of the 19 ms of a mesh of 117 k vertices and 640 k tetrahedra
+  // (now 8), and destroying it 3.3 ms (0.4). The scratch's peak is the first sort (24 N bytes of keys
+  // and positions in and out, and as much again for hipCUB).
+  Slab tmp(size_t(48 * N + 64 * n) + (1 << 20));
   const unsigned gN = grid_for(N, kBlock);
-  // 1. Sort cell-edge slots by (lower, higher) key, stably.
-  DBuf<uint64_t> keys(N), skeys(N);
-  DBuf<uint32_t> pos(N), spos(N);
-  k_edge_keys<<<gN, kBlock, 0, s>>>(m->cells.p, T, nv, ne, uint64_t(n), keys.p, pos.p);
   const int kbits = bits_for(uint64_t(n) * uint64_t(n));
-  sort_pairs(keys.p, skeys.p, pos.p, spos.p, N, kbits, s);
-  keys.release();
-  pos.release();
-  // 2. Runs and first appearances.
-  DBuf<int32_t> head(N), runid(N), isfirst(N), eid(N);
-  k_heads<<<gN, kBlock, 0, s>>>(skeys.p, N, head.p);
-  // runid[i] = (number of run heads at or before i) - 1.
-  inclusive_sum(head.p, runid.p, N, s);
-  int32_t nruns = 0;
-  NOSH_HIP(hipMemcpy(&nruns, runid.p + N - 1, 4, hipMemcpyDeviceToHost));
-  k_add<<<gN, kBlock, 0, s>>>(runid.p, N, -1);
-  const int64_t E = nruns;
-  m->E = E;
-  isfirst.zero(s);
-  k_mark_first<<<gN, kBlock, 0, s>>>(head.p, spos.p, N, isfirst.p);
-  exclusive_sum(isfirst.p, eid.p, N, s);
-  isfirst.release();
-  DBuf<int32_t> run_edge(E), edge_start(E), run_start(E + 1);
-  m->edges.alloc(2 * E);
-  k_run_edges<<<gN, kBlock, 0, s>>>(head.p, runid.p, spos.p, skeys.p, eid.p, N, uint64_t(n),
-                                    run_edge.p, m->edges.p, edge_start.p);
-  k_run_start<<<gN, kBlock, 0, s>>>(head.p, runid.p, N, run_start.p);
-  const int32_t Ni = int32_t(N);
-  NOSH_HIP(hipMemcpyAsync(run_start.p + E, &Ni, 4, hipMemcpyHostToDevice, s));
-  eid.release();
-  skeys.release();
-  // 3. Cell -> edges, ascending.
-  m->cell_edges.alloc(N);
-  k_cell_edges_canon<<<gN, kBlock, 0, s>>>(runid.p, spos.p, run_edge.p, N, m->cell_edges.p);
-  k_sort_cell_edges<<<grid_for(T, kBlock), kBlock, 0, s>>>(m->cell_edges.p, T, ne);
-  head.release();
-  runid.release();
-  // 4. Edge lengths, coefficients, covolumes.
-  m->len.alloc(E);
-  m->covol.alloc(E);
-  k_edge_length<<<grid_for(E, kBlock), kBlock, 0, s>>>(m->coords.p, m->edges.p, E, m->len.p);
-  DBuf<double> coef(N);
-  if (ne == 3)
-    k_edge_coefficients<3><<<grid_for(T, 128), 128, 0, s>>>(m->coords.p, m->edges.p,
-                                                            m->cell_edges.p, T, coef.p);
-  else
-    k_edge_coefficients<6><<<grid_for(T, 128), 128, 0, s>>>(m->coords.p, m->edges.p,
-                                                            m->cell_edges.p, T, coef.p);
-  k_covolume_runs<<<grid_for(E, kBlock), kBlock, 0, s>>>(run_start.p, run_edge.p, spos.p,
-                                                         m->cell_edges.p, coef.p, m->len.p, E, ne,
-                                                         m->covol.p);
-  NOSH_HIP(hipStreamSynchronize(s));
-  coef.release();
-  spos.release();
-  run_edge.release();
-  run_start.release();
-  edge_start.release();
+  int64_t E = 0;
+  {
+    // 1. Sort cell-edge slots by (lower, higher) key, stably.
+    uint32_t* spos = tmp.take<uint32_t>(N);
+    uint64_t* skeys = tmp.take<uint64_t>(N);
+    const size_t m1 = tmp.mark();
+    uint64_t* keys = tmp.take<uint64_t>(N);
+    uint32_t* pos = tmp.take<uint32_t>(N);
+    k_edge_keys<<<gN, kBlock, 0, s>>>(m->cells.p, T, nv, ne, uint64_t(n), keys, pos);
+    sort_pairs(keys, skeys, pos, spos, N, kbits, tmp, s);
+    tmp.reset(m1);
+    // 2. Runs and first appearances.
+    int32_t* head = tmp.take<int32_t>(N);
+    int32_t* runid = tmp.take<int32_t>(N);
+    int32_t* isfirst = tmp.take<int32_t>(N);
+    int32_t* eid = tmp.take<int32_t>(N);
+    k_heads<<<gN, kBlock, 0, s>>>(skeys, N, head);
+    // runid[i] = (number of run heads at or before i) - 1.
+    inclusive_sum(head, runid, N, tmp, s);
+    E = read_i32(runid + N - 1, s);
+    m->E = E;
+    k_add<<<gN, kBlock, 0, s>>>(runid, N, -1);
+    zero_i32(isfirst, N, s);
+    k_mark_first<<<gN, kBlock, 0, s>>>(head, spos, N, isfirst);
+    exclusive_sum(isfirst, eid, N, tmp, s);
+    {
+      Slab& k = m->slabs.emplace_back(slab_bytes<int32_t>(2 * E) + 2 * slab_bytes<double>(E));
+      k.take(m->edges, 2 * E);
+      k.take(m->len, E);
+      k.take(m->covol, E);
+    }
+    int32_t* run_edge = tmp.take<int32_t>(E);
+    int32_t* edge_start = tmp.take<int32_t>(E);
+    int32_t* run_start = tmp.take<int32_t>(E + 1);
+    k_run_edges<<<gN, kBlock, 0, s>>>(head, runid, spos, skeys, eid, N, uint64_t(n), run_edge,
+                                      m->edges.p, edge_start);
+    k_run_start<<<gN, kBlock, 0, s>>>(head, runid, N, run_start);
+    k_fill_i32<<<1, 1, 0, s>>>(run_start + E, 1, int32_t(N));
+    // 3. Cell -> edges, ascending.
+    k_cell_edges_canon<<<gN, kBlock, 0, s>>>(runid, spos, run_edge, N, m->cell_edges.p);
+    k_sort_cell_edges<<<grid_for(T, kBlock), kBlock, 0, s>>>(m->cell_edges.p, T, ne);
+    // 4. Edge lengths, coefficients, covolumes.
+    k_edge_length<<<grid_for(E, kBlock), kBlock, 0, s>>>(m->coords.p, m->edges.p, E, m->len.p);
+    double* coef = tmp.take<double>(N);
+    if (ne == 3)
+      k_edge_coefficients<3><<<grid_for(T, 128), 128, 0, s>>>(m->coords.p, m->edges.p,
+                                                              m->cell_edges.p, T, coef);
+    else
+      k_edge_coefficients<6><<<grid_for(T, 128), 128, 0, s>>>(m->coords.p, m->edges.p,
+                                                              m->cell_edges.p, T, coef);
+    k_covolume_runs<<<grid_for(E, kBlock), kBlock, 0, s>>>(
+        run_start, run_edge, spos, m->cell_edges.p, coef, m->len.p, E, ne, m->covol.p);
+    tmp.reset(0);
+  }
   // 5. Control volumes: per-cell contributions summed per vertex in cell order.
   {
-    const int64_t Nv = T * nv;
-    DBuf<double> cvc(Nv);
-    k_cell_cv<<<grid_for(T, 128), 128, 0, s>>>(m->coords.p, m->cells.p, T, nv, cvc.p);
-    DBuf<uint32_t> vk(Nv), svk(Nv), vp(Nv), svp(Nv);
-    k_u32_from_i32<<<grid_for(Nv, kBlock), kBlock, 0, s>>>(m->cells.p, Nv, vk.p);
-    k_iota<<<grid_for(Nv, kBlock), kBlock, 0, s>>>(vp.p, Nv);
-    sort_pairs(vk.p, svk.p, vp.p, svp.p, Nv, bits_for(uint64_t(n)), s);
-    DBuf<int32_t> vstart(n + 1);
-    k_segment_starts<<<grid_for(Nv + 1, kBlock), kBlock, 0, s>>>(svk.p, Nv, n, vstart.p);
-    m->cv.alloc(n);
-    k_vertex_cv<<<grid_for(n, kBlock), kBlock, 0, s>>>(vstart.p, svp.p, cvc.p, n, m->cv.p);
-    NOSH_HIP(hipStreamSynchronize(s));
+    double* cvc = tmp.take<double>(Nv);
+    k_cell_cv<<<grid_for(T, 128), 128, 0, s>>>(m->coords.p, m->cells.p, T, nv, cvc);
+    uint32_t* vk = tmp.take<uint32_t>(Nv);
+    uint32_t* svk = tmp.take<uint32_t>(Nv);
+    uint32_t* vp = tmp.take<uint32_t>(Nv);
+    uint32_t* svp = tmp.take<uint32_t>(Nv);
+    k_u32_from_i32<<<grid_for(Nv, kBlock), kBlock, 0, s>>>(m->cells.p, Nv, vk);
+    k_iota<<<grid_for(Nv, kBlock), kBlock, 0, s>>>(vp, Nv);
+    sort_pairs(vk, svk, vp, svp, Nv, bits_for(uint64_t(n)), tmp, s);
+    int32_t* vstart = tmp.take<int32_t>(n + 1);
+    k_segment_starts<<<grid_for(Nv + 1, kBlock), kBlock, 0, s>>>(svk, Nv, n, vstart);
+    k_vertex_cv<<<grid_for(n, kBlock), kBlock, 0, s>>>(vstart, svp, cvc, n, m->cv.p);
+    tmp.reset(0);
   }
-  // 6. Vertex order: reverse Cuthill-McKee over the reference-order graph.
+  // The directed graph in the order iperm gives (null: the reference's), as
+  // sorted rows, columns, edge codes and row starts.
   const int64_t ND = 2 * E;
-  std::vector<int32_t> perm_h(n);
+  struct Csr {
+    uint32_t* rows;
+    int32_t *cols, *codes, *start;
+  };
+  auto directed = [&](const int32_t* iperm) {
+    Csr c;
+    c.rows = tmp.take<uint32_t>(ND);
+    c.cols = tmp.take<int32_t>(ND);
+    c.codes = tmp.take<int32_t>(ND);
+    c.start = tmp.take<int32_t>(n + 1);
+    const size_t m1 = tmp.mark();
+    uint64_t* dk = tmp.take<uint64_t>(ND);
+    uint64_t* sdk = tmp.take<uint64_t>(ND);
+    int32_t* dv = tmp.take<int32_t>(ND);
+    k_directed<<<grid_for(E, kBlock), kBlock, 0, s>>>(m->edges.p, E, iperm, uint64_t(n), dk, dv);
+    sort_pairs(dk, sdk, dv, c.codes, ND, kbits, tmp, s);
+    k_rows_of<<<grid_for(ND, kBlock), kBlock, 0, s>>>(sdk, ND, uint64_t(n), c.rows, c.cols);
+    k_segment_starts<<<grid_for(ND + 1, kBlock), kBlock, 0, s>>>(c.rows, ND, n, c.start);
+    tmp.reset(m1);
+    return c;
+  };
+  // 6. Vertex order: reverse Cuthill-McKee over the reference-order graph.
+  std::vector<int32_t> perm_h;
   if (reorder) {
-    DBuf<uint64_t> dk(ND), sdk(ND);
-    DBuf<int32_t> dv(ND), sdv(ND);
-    k_directed<<<grid_for(E, kBlock), kBlock, 0, s>>>(m->edges.p, E, nullptr, uint64_t(n), dk.p,
-                                                      dv.p);
-    sort_pairs(dk.p, sdk.p, dv.p, sdv.p, ND, kbits, s);
-    DBuf<uint32_t> rows(ND);
-    DBuf<int32_t> cols(ND), rstart(n + 1);
-    k_rows_of<<<grid_for(ND, kBlock), kBlock, 0, s>>>(sdk.p, ND, uint64_t(n), rows.p, cols.p);
-    k_segment_starts<<<grid_for(ND + 1, kBlock), kBlock, 0, s>>>(rows.p, ND, n, rstart.p);
-    std::vector<int32_t> ptr_h(n + 1), adj_h(ND);
-    NOSH_HIP(hipMemcpyAsync(ptr_h.data(), rstart.p, 4 * (n + 1), hipMemcpyDeviceToHost, s));
-    NOSH_HIP(hipMemcpyAsync(adj_h.data(), cols.p, 4 * ND, hipMemcpyDeviceToHost, s));
+    const Csr c = directed(nullptr);
+    const std::unique_ptr<int32_t[]> ptr_h(new int32_t[n + 1]), adj_h(new int32_t[ND]);
+    NOSH_HIP(hipMemcpyAsync(ptr_h.get(), c.start, 4 * (n + 1), hipMemcpyDeviceToHost, s));
+    NOSH_HIP(hipMemcpyAsync(adj_h.get(), c.cols, 4 * ND, hipMemcpyDeviceToHost, s));
     NOSH_HIP(hipStreamSynchronize(s));
-    perm_h = rcm_order(n, ptr_h, adj_h);
+    perm_h = rcm_order(n, ptr_h.get(), adj_h.get());
+    tmp.reset(0);
   } else {
+    perm_h.resize(n);
     std::iota(perm_h.begin(), perm_h.end(), 0);
   }
-  m->perm.alloc(n);
   m->perm.upload(perm_h.data(), n, s);
-  m->iperm.alloc(n);
   k_invert_perm<<<grid_for(n, kBlock), kBlock, 0, s>>>(m->perm.p, n, m->iperm.p);
-  m->cv_int.alloc(n);
   k_gather_f64<<<grid_for(n, kBlock), kBlock, 0, s>>>(m->perm.p, m->cv.p, n, m->cv_int.p);
-  // 7. Internal sliced ELLPACK of the off-diagonal graph.
+  // 7. Internal sliced ELLPACK of the off-diagonal graph, and
+  // 8. the split layout of the same graph for the operator kernels.
   {
-    DBuf<uint64_t> dk(ND), sdk(ND);
-    DBuf<int32_t> dv(ND), sdv(ND);
-    k_directed<<<grid_for(E, kBlock), kBlock, 0, s>>>(m->edges.p, E, m->iperm.p, uint64_t(n),
-                                                      dk.p, dv.p);
-    sort_pairs(dk.p, sdk.p, dv.p, sdv.p, ND, kbits, s);
-    DBuf<uint32_t> rows(ND);
-    DBuf<int32_t> cols(ND), rstart(n + 1);
-    k_rows_of<<<grid_for(ND, kBlock), kBlock, 0, s>>>(sdk.p, ND, uint64_t(n), rows.p, cols.p);
-    k_segment_starts<<<grid_for(ND + 1, kBlock), kBlock, 0, s>>>(rows.p, ND, n, rstart.p);
-    const int64_t ns = (n + kSliceH - 1) / kSliceH;
-    m->nslices = ns;
-    DBuf<int32_t> w64(ns + 1);
-    w64.zero(s);
-    k_slice_width<<<grid_for(ns, kBlock), kBlock, 0, s>>>(rstart.p, n, ns, w64.p);
-    m->slice_ptr.alloc(ns + 1);
-    exclusive_sum(w64.p, m->slice_ptr.p, ns + 1, s);
-    int32_t total = 0;
-    NOSH_HIP(hipMemcpy(&total, m->slice_ptr.p + ns, 4, hipMemcpyDeviceToHost));
-    m->nnz_pad = total;
+    const Csr c = directed(m->iperm.p);
+    int32_t* w64 = tmp.take<int32_t>(ns + 1);
+    int32_t* wl64 = tmp.take<int32_t>(ns + 1);
+    int32_t* wu64 = tmp.take<int32_t>(ns + 1);
+    int32_t* nlow = tmp.take<int32_t>(n);
+    int32_t* nup = tmp.take<int32_t>(n);
+    for (int32_t* w : {w64, wl64, wu64}) zero_i32(w + ns, 1, s);
+    k_slice_width<<<grid_for(ns, kBlock), kBlock, 0, s>>>(c.start, n, ns, w64);
+    k_count_split<<<grid_for(n, kBlock), kBlock, 0, s>>>(c.start, c.cols, n, nlow, nup);
+    k_split_width<<<grid_for(ns, kBlock), kBlock, 0, s>>>(nlow, nup, n, ns, wl64, wu64);
+    exclusive_sum(w64, m->slice_ptr.p, ns + 1, tmp, s);
+    exclusive_sum(wu64, m->uptr.p, ns + 1, tmp, s);
+    exclusive_sum(wl64, m->lptr.p, ns + 1, tmp, s);
     std::vector<int32_t> wh(ns);
-    NOSH_HIP(hipMemcpy(wh.data(), w64.p, 4 * ns, hipMemcpyDeviceToHost));
-    m->max_width = 0;
-    for (int32_t w : wh) m->max_width = std::max(m->max_width, w / kSliceH);
-    m->scol.alloc(std::max<int64_t>(total, 1));
-    m->sedge.alloc(std::max<int64_t>(total, 1));
-    k_sell_pad<<<unsigned(ns), kBlock, 0, s>>>(m->slice_ptr.p, ns, n, m->scol.p, m->sedge.p);
-    k_sell_fill<<<grid_for(ND, kBlock), kBlock, 0, s>>>(rows.p, cols.p, sdv.p, rstart.p,
-                                                        m->slice_ptr.p, ND, m->scol.p,
-                                                        m->sedge.p);
-    // 8. The split layout of the same graph for the operator kernels.
-    DBuf<int32_t> nlow(n), nup(n), wl64(ns + 1), wu64(ns + 1);
-    wl64.zero(s);
-    wu64.zero(s);
-    k_count_split<<<grid_for(n, kBlock), kBlock, 0, s>>>(rstart.p, cols.p, n, nlow.p, nup.p);
-    k_split_width<<<grid_for(ns, kBlock), kBlock, 0, s>>>(nlow.p, nup.p, n, ns, wl64.p, wu64.p);
-    m->uptr.alloc(ns + 1);
-    m->lptr.alloc(ns + 1);
-    exclusive_sum(wu64.p, m->uptr.p, ns + 1, s);
-    exclusive_sum(wl64.p, m->lptr.p, ns + 1, s);
-    int32_t tu = 0, tl = 0;
-    NOSH_HIP(hipMemcpy(&tu, m->uptr.p + ns, 4, hipMemcpyDeviceToHost));
-    NOSH_HIP(hipMemcpy(&tl, m->lptr.p + ns, 4, hipMemcpyDeviceToHost));
+    int32_t total = 0, tu = 0, tl = 0;
+    NOSH_HIP(hipMemcpyAsync(wh.data(), w64, 4 * ns, hipMemcpyDeviceToHost, s));
+    NOSH_HIP(hipMemcpyAsync(&total, m->slice_ptr.p + ns, 4, hipMemcpyDeviceToHost, s));
+    NOSH_HIP(hipMemcpyAsync(&tu, m->uptr.p + ns, 4, hipMemcpyDeviceToHost, s));
+    NOSH_HIP(hipMemcpyAsync(&tl, m->lptr.p + ns, 4, hipMemcpyDeviceToHost, s));
+    NOSH_HIP(hipStreamSynchronize(s));
+    m->nnz_pad = total;
     m->nnz_u = tu;
     m->nnz_l = tl;
-    m->ucol.alloc(std::max<int64_t>(tu, 1));
-    m->uedge.alloc(std::max<int64_t>(tu, 1));
-    m->lcol.alloc(std::max<int64_t>(tl, 1));
-    m->lpos.alloc(std::max<int64_t>(tl, 1));
-    DBuf<int32_t> lcode(std::max<int64_t>(tl, 1)), upos(std::max<int64_t>(E, 1));
-    k_fill_i32<<<grid_for(tl, kBlock), kBlock, 0, s>>>(lcode.p, tl, -1);
+    m->max_width = 0;
+    for (int32_t w : wh) m->max_width = std::max(m->max_width, w / kSliceH);
+    const int64_t np = std::max<int64_t>(total, 1), nu = std::max<int64_t>(tu, 1),
+                  nl = std::max<int64_t>(tl, 1);
+    {
+      Slab& k = m->slabs.emplace_back(2 * slab_bytes<int32_t>(np) + 2 * slab_bytes<int32_t>(nu) +
+                                      2 * slab_bytes<int32_t>(nl) + slab_bytes<int16_t>(nu) +
+                                      slab_bytes<int16_t>(nl));
+      k.take(m->scol, np);
+      k.take(m->sedge, np);
+      k.take(m->ucol, nu);
+      k.take(m->uedge, nu);
+      k.take(m->lcol, nl);
+      k.take(m->lpos, nl);
+      k.take(m->uoff, nu);
+      k.take(m->loff, nl);
+    }
+    k_sell_pad<<<unsigned(ns), kBlock, 0, s>>>(m->slice_ptr.p, ns, n, m->scol.p, m->sedge.p);
+    k_sell_fill<<<grid_for(ND, kBlock), kBlock, 0, s>>>(c.rows, c.cols, c.codes, c.start,
+                                                        m->slice_ptr.p, ND, m->scol.p,
+                                                        m->sedge.p);
+    int32_t* lcode = tmp.take<int32_t>(nl);
+    int32_t* upos = tmp.take<int32_t>(std::max<int64_t>(E, 1));
+    int32_t* wide = tmp.take<int32_t>(1);
+    k_fill_i32<<<grid_for(tl, kBlock), kBlock, 0, s>>>(lcode, tl, -1);
     k_split_pad<<<unsigned(ns), kBlock, 0, s>>>(m->uptr.p, m->lptr.p, ns, n, tu, m->ucol.p,
                                                 m->uedge.p, m->lcol.p, m->lpos.p);
     k_split_fill<<<grid_for(ND, kBlock), kBlock, 0, s>>>(
-        rows.p, cols.p, sdv.p, rstart.p, nlow.p, m->uptr.p, m->lptr.p, ND, m->ucol.p,
-        m->uedge.p, m->lcol.p, lcode.p, upos.p);
-    k_split_lpos<<<grid_for(tl, kBlock), kBlock, 0, s>>>(lcode.p, upos.p, tl, m->lpos.p);
+        c.rows, c.cols, c.codes, c.start, nlow, m->uptr.p, m->lptr.p, ND, m->ucol.p, m->uedge.p,
+        m->lcol.p, lcode, upos);
+    k_split_lpos<<<grid_for(tl, kBlock), kBlock, 0, s>>>(lcode, upos, tl, m->lpos.p);
     // 16-bit column offsets when the bandwidth allows (2 bytes less per slot
     // for every kernel that reads the split layout).
-    m->uoff.alloc(std::max<int64_t>(tu, 1));
-    m->loff.alloc(std::max<int64_t>(tl, 1));
-    DBuf<int32_t> wide(1);
-    k_fill_i32<<<1, 1, 0, s>>>(wide.p, 1, 0);
-    k_col_off16<<<unsigned(ns), kBlock, 0, s>>>(m->uptr.p, m->ucol.p, ns, n, m->uoff.p, wide.p);
-    k_col_off16<<<unsigned(ns), kBlock, 0, s>>>(m->lptr.p, m->lcol.p, ns, n, m->loff.p, wide.p);
-    int32_t wide_h = 0;
-    NOSH_HIP(hipMemcpyAsync(&wide_h, wide.p, 4, hipMemcpyDeviceToHost, s));
-    NOSH_HIP(hipStreamSynchronize(s));
-    if (wide_h) {
+    k_fill_i32<<<1, 1, 0, s>>>(wide, 1, 0);
+    k_col_off16<<<unsigned(ns), kBlock, 0, s>>>(m->uptr.p, m->ucol.p, ns, n, m->uoff.p, wide);
+    k_col_off16<<<unsigned(ns), kBlock, 0, s>>>(m->lptr.p, m->lcol.p, ns, n, m->loff.p, wide);
+    if (read_i32(wide, s)) {
       m->uoff.release();
       m->loff.release();
     }
