@@ -269,3 +269,40 @@ def test_newton_matches_oracle(name):
     assert st_r["converged"] and st_r["final_norm_f"] <= 1e-10
     d = phase_align(psi_r, psi_o) - psi_o
     assert np.linalg.norm(d) / np.linalg.norm(psi_o) < 1e-9
+
+
+@pytest.mark.parametrize("ncell", [1, 7, 8, 299, 300])
+def test_row_products_at_the_split_sizes(ncell):
+    """Four and two waves a slice: a mesh of 4 rows, slices exactly full and one
+    row over (64, 81), the last mesh of the four-wave form and the first of the
+    two-wave form (90,000 and 90,601 rows; an odd number of slices leaves the
+    last workgroup half empty). F, K, J and P against the oracle, and a linear
+    solve of 20 iterations, whose reductions go through both ways of adding
+    the partial sums, against the same solve's residual from J."""
+    import nosh_amd as nosh
+    from oracle import oracle as O
+    coords, cells = mg.square_tri(ncell)
+    n = coords.shape[0]
+    case = dict(om=O.Mesh(coords, cells), gm=nosh.Mesh(coords, cells),
+                A=mg.magnetic_potential(coords))
+    g, mu = 1.3, 0.2
+    mvp = nosh.VectorFieldExplicitValues(case["gm"], case["A"], mu)
+    t = nosh.ScalarFieldConstant(case["gm"], 1.0)
+    model = nosh.Nls(case["gm"], mvp, nosh.ScalarFieldConstant(case["gm"], -1.0), g, t)
+    om = O.Model(case["om"], case["A"])
+    om.set_params(g, mu)
+    p = {"g": g, "mu": mu}
+    psi, phi = mg.random_state(n, 5), mg.random_state(n, 6)
+    assert rel_err(model.eval_f(psi, p), om.f(psi)) < TOL
+    J, P = model.create_W_op(), model.create_W_prec()
+    J.rebuild(p, psi)
+    P.rebuild(p, psi)
+    om.jac_rebuild(psi)
+    assert rel_err(J.apply(phi), om.jac(phi)) < TOL
+    b = om.f(psi)
+    x, it, rr = nosh.minres_solve(J, P, b, rtol=1e-14, max_iters=20)
+    assert it <= 20 and np.all(np.isfinite(x))
+    # MINRES never lets the residual grow from x = 0, in the M^{-1} norm.
+    r = b - om.jac(x)
+    assert r @ P.apply(r) <= (1 + 1e-10) * (b @ P.apply(b))
+    assert abs(np.sqrt(r @ P.apply(r) / (b @ P.apply(b))) - rr) <= 1e-8
