@@ -40,15 +40,37 @@ struct ColsW {
 constexpr int kDotThreads = 256;
 constexpr int kCombThreads = 256;
 
+// Sums of 16 values over the wave, each lane giving half of what it holds to
+// its partner and keeping the other half (17 exchanges; value by value, 96):
+// every lane ends with the value lane_value16(lane).
+__device__ __forceinline__ double wave_sum16(double (&v)[16], int lane) {
+#pragma unroll
+  for (int h = 8, off = 32; h >= 1; h >>= 1, off >>= 1) {
+    const bool hi = lane & off;
+#pragma unroll
+    for (int i = 0; i < h; ++i) {
+      const double keep = hi ? v[i + h] : v[i], give = hi ? v[i] : v[i + h];
+      v[i] = keep + __shfl_xor(give, off, 64);
+    }
+  }
+  v[0] += __shfl_xor(v[0], 2, 64);
+  return v[0] + __shfl_xor(v[0], 1, 64);
+}
+__device__ __forceinline__ int lane_value16(int lane) {
+  return (lane >> 5 & 1) * 8 + (lane >> 4 & 1) * 4 + (lane >> 3 & 1) * 2 + (lane >> 2 & 1);
+}
+
 // Partial sums of A_i . B_j over one row range for one 4 x 4 tile of (i, j).
 // One 1-D grid of nblk * ntiles workgroups; the logical index (XCD-remapped,
 // so that consecutive logical indices run on one XCD) is rb * ntiles + tile:
 // the tiles of one row range run side by side and re-read its columns from
 // that XCD's L2 rather than from HBM.
+// With one row range (nblk = 1) the sums go straight to out.
 __global__ __launch_bounds__(kDotThreads) void k_block_dots(ColsC A, int ma, ColsC B, int mb,
                                                             int64_t L2, int64_t per_block,
                                                             int nblk,
-                                                            double* __restrict__ partials) {
+                                                            double* __restrict__ partials,
+                                                            double* __restrict__ out) {
   const int ntj = (mb + 3) >> 2;
   const int ntiles = ((ma + 3) >> 2) * ntj;
   const int64_t logical = xcd_block(true);
@@ -80,12 +102,21 @@ __global__ __launch_bounds__(kDotThreads) void k_block_dots(ColsC A, int ma, Col
 #pragma unroll
       for (int j = 0; j < 4; ++j) acc[4 * i + j] += av[i].x * bv[j].x + av[i].y * bv[j].y;
   }
-  __shared__ double lds[16 * 16];
-  block_sum<16>(acc, lds);
-  if (threadIdx.x == 0) {
+  __shared__ double lds[kDotThreads / 64][16];
+  const int lane = int(threadIdx.x & 63);
+  const double v = wave_sum16(acc, lane);
+  if ((lane & 3) == 0) lds[threadIdx.x >> 6][lane_value16(lane)] = v;
+  __syncthreads();
+  if (threadIdx.x >= 16) return;
+  const int q = int(threadIdx.x);
+  double sum = lds[0][q];
 #pragma unroll
-    for (int q = 0; q < 16; ++q) partials[(int64_t(tile) * 16 + q) * nblk + rb] = acc[q];
-  }
+  for (int w = 1; w < kDotThreads / 64; ++w) sum += lds[w][q];
+  const int i = 4 * ti + (q >> 2), j = 4 * tj + (q & 3);
+  if (nblk > 1)
+    partials[(int64_t(tile) * 16 + q) * nblk + rb] = sum;
+  else if (i < ma && j < mb)
+    out[i * mb + j] = sum;
 }
 
 // out[i mb + j] = sum of the partials of (i, j) in block order; one block
@@ -106,32 +137,46 @@ struct CoefArg {
   double c[kArgCoefs];
 };
 
-// Y_j = beta Y_j + sum_c C[c k + j] S_c, two rows (one double2) per thread.
-// C is the by-value CA.c when BYVAL, else the device array Cd.
-template <bool BYVAL>
+// Y_j = beta Y_j + sum_c C[c k + j] S_c, two rows (one double2) per thread, for
+// k <= K outputs. C is cscale Cd (device) when Cd is given, else CA. The
+// coefficients go through LDS, padded to K columns, and four columns of S are
+// read ahead: read one at a time with a scalar load and a branch per
+// coefficient, 18 columns of 1089 rows took 8.4 us, all of it latency; now 5.3.
+template <int K>
 __global__ __launch_bounds__(kCombThreads) void k_block_combine(ColsC S, int m, CoefArg CA,
                                                                 const double* __restrict__ Cd,
-                                                                ColsW Y, int k, double beta,
-                                                                int64_t L2) {
-  const double* C = BYVAL ? CA.c : Cd;
+                                                                double cscale, ColsW Y, int k,
+                                                                double beta, int64_t L2) {
+  __shared__ double C[kMaxCols * K];
+  for (int i = threadIdx.x; i < m * K; i += kCombThreads) {
+    const int c = i / K, j = i - c * K;
+    C[i] = j < k ? (Cd ? cscale * Cd[c * k + j] : CA.c[c * k + j]) : 0.0;
+  }
+  __syncthreads();
   const int64_t r = int64_t(blockIdx.x) * kCombThreads + threadIdx.x;
   if (r >= L2) return;
-  double2 acc[16];
+  double2 acc[K];
 #pragma unroll
-  for (int j = 0; j < 16; ++j) acc[j] = make_double2(0.0, 0.0);
-  for (int c = 0; c < m; ++c) {
-    const double2 v = reinterpret_cast<const double2*>(S.p[c])[r];
+  for (int j = 0; j < K; ++j) acc[j] = make_double2(0.0, 0.0);
+  constexpr int U = 4;
+  for (int c0 = 0; c0 < m; c0 += U) {
+    double2 v[U];
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      if (j < k) {
-        const double w = C[c * k + j];
-        acc[j].x += w * v.x;
-        acc[j].y += w * v.y;
+    for (int u = 0; u < U; ++u)
+      if (c0 + u < m) v[u] = reinterpret_cast<const double2*>(S.p[c0 + u])[r];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (c0 + u >= m) break;
+#pragma unroll
+      for (int j = 0; j < K; ++j) {
+        const double w = C[(c0 + u) * K + j];
+        acc[j].x += w * v[u].x;
+        acc[j].y += w * v[u].y;
       }
     }
   }
 #pragma unroll
-  for (int j = 0; j < 16; ++j) {
+  for (int j = 0; j < K; ++j) {
     if (j < k) {
       double2* y = reinterpret_cast<double2*>(Y.p[j]) + r;
       double2 o = acc[j];
@@ -158,11 +203,43 @@ struct BlkOp {
   const double* bound;  // Chebyshev bound from the rebuild
   double upper, ratio;
   int iters;
+  double* coef;         // theta, then (c1, c2) of every Chebyshev step (k_blk_coef)
 };
 
+// Columns per thread and threads per workgroup: 8 and 256, so that a slot is
+// read once for all columns, or up to kBlkSmall rows 2 and 64: as many
+// workgroups along the columns as there are pairs, and four times as many along
+// the rows (the 1089 rows of a 32^2 square were 5 workgroups on 256 CUs). Whole
+// solves, 8 | 2 columns: 32^2 square 14.2 | 13.0 ms, 199^2 113.2 | 107.0, 320^2
+// (103041 rows) 197.9 | 192.2, 56^3 cube (185193 rows) 49.0 | 47.6, 72^3 (389017
+// rows) 97.6 | 102.8: the line lies where the second read of the slots no
+// longer comes out of the caches.
+constexpr int64_t kBlkSmall = 200000;
+
+__global__ void k_blk_coef(BlkOp o) {
+  const double hi = cheb_hi(o.bound, o.upper);
+  o.coef[0] = 0.5 * (hi + hi / o.ratio);
+  for (int j = 1; j < o.iters; ++j) {
+    const Cheb c = cheb_coef(hi, o.ratio, j);
+    o.coef[2 * j - 1] = c.c1;
+    o.coef[2 * j] = c.c2;
+  }
+}
+
+// Columns q0 .. q0 + NV - 1 of a list.
+template <int NV, class C>
+__device__ __forceinline__ auto cols_at(const C& X, int q0, int nv) {
+  struct {
+    decltype(X.p[0] + 0) p[NV];
+  } r;
+#pragma unroll
+  for (int q = 0; q < NV; ++q) r.p[q] = X.p[q < nv ? q0 + q : q0];
+  return r;
+}
+
 // Off-diagonal products of one row for nv <= NV columns.
-template <int NV>
-__device__ __forceinline__ void blk_row(const BlkOp& o, int64_t row, int nv, const ColsC& X,
+template <int NV, class Cols>
+__device__ __forceinline__ void blk_row(const BlkOp& o, int64_t row, int nv, const Cols& X,
                                         double2 (&acc)[NV]) {
   const int32_t sl = uniform(int32_t(row >> 6));
   const int lane = int(row & 63);
@@ -171,7 +248,7 @@ __device__ __forceinline__ void blk_row(const BlkOp& o, int64_t row, int nv, con
   // Upper part: values in place.
   for (int32_t j = uniform(o.sv.uptr[sl]) + lane, e = uniform(o.sv.uptr[sl + 1]); j < e;
        j += kSliceH) {
-    const int32_t c = __builtin_nontemporal_load(o.sv.ucol + j);
+    const int32_t c = o.sv.uoff ? int32_t(row) + o.sv.uoff[j] : o.sv.ucol[j];
     const double2 v = o.val[j];
 #pragma unroll
     for (int q = 0; q < NV; ++q) {
@@ -185,8 +262,8 @@ __device__ __forceinline__ void blk_row(const BlkOp& o, int64_t row, int nv, con
   // Lower part: the conjugate of the mirrored slot's value.
   for (int32_t j = uniform(o.sv.lptr[sl]) + lane, e = uniform(o.sv.lptr[sl + 1]); j < e;
        j += kSliceH) {
-    const int32_t c = __builtin_nontemporal_load(o.sv.lcol + j);
-    const double2 v = o.val[__builtin_nontemporal_load(o.sv.lpos + j)];
+    const int32_t c = o.sv.loff ? int32_t(row) + o.sv.loff[j] : o.sv.lcol[j];
+    const double2 v = o.val[o.sv.lpos[j]];
 #pragma unroll
     for (int q = 0; q < NV; ++q) {
       if (q < nv) {
@@ -200,9 +277,12 @@ __device__ __forceinline__ void blk_row(const BlkOp& o, int64_t row, int nv, con
 
 // Y_q = Koff X_q + B X_q.
 template <int NV>
-__global__ __launch_bounds__(kSB) void k_blk_apply(BlkOp o, int nv, ColsC X, ColsW Y) {
-  const int64_t row = xcd_block(true) * kSB + threadIdx.x;
+__global__ __launch_bounds__(kSB) void k_blk_apply(BlkOp o, int nvall, ColsC Xs, ColsW Ys) {
+  const int64_t row = xcd_block(true) * blockDim.x + threadIdx.x;
   if (row >= o.n) return;
+  const int q0 = int(blockIdx.y) * NV, nv = min(NV, nvall - q0);
+  const auto X = cols_at<NV>(Xs, q0, nv);
+  const auto Y = cols_at<NV>(Ys, q0, nv);
   double2 acc[NV];
   blk_row<NV>(o, row, nv, X, acc);
   const double b0 = o.blk[row], b1 = o.blk[o.n + row], b2 = o.blk[2 * o.n + row];
@@ -218,12 +298,15 @@ __global__ __launch_bounds__(kSB) void k_blk_apply(BlkOp o, int nv, ColsC X, Col
 
 // Chebyshev step 0 on P: Z_q = D^{-1} R_q / theta (and the direction D_q).
 template <int NV>
-__global__ __launch_bounds__(kSB) void k_blk_cheb_first(BlkOp o, int nv, ColsC R, ColsW Z,
-                                                        ColsW Dd) {
-  const int64_t row = int64_t(blockIdx.x) * kSB + threadIdx.x;
+__global__ __launch_bounds__(kSB) void k_blk_cheb_first(BlkOp o, int nvall, ColsC Rs, ColsW Zs,
+                                                        ColsW Ds) {
+  const int64_t row = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (row >= o.n) return;
-  const double hi = cheb_hi(o.bound, o.upper);
-  const double th = 0.5 * (hi + hi / o.ratio);
+  const int q0 = int(blockIdx.y) * NV, nv = min(NV, nvall - q0);
+  const auto R = cols_at<NV>(Rs, q0, nv);
+  const auto Z = cols_at<NV>(Zs, q0, nv);
+  const auto Dd = cols_at<NV>(Ds, q0, nv);
+  const double th = o.coef[0];
   const double b0 = o.blk[row], b1 = o.blk[o.n + row], b2 = o.blk[2 * o.n + row];
 #pragma unroll
   for (int q = 0; q < NV; ++q) {
@@ -240,11 +323,16 @@ __global__ __launch_bounds__(kSB) void k_blk_cheb_first(BlkOp o, int nv, ColsC R
 
 // Chebyshev step j >= 1: Zout = Zin + d, d = c1 d + c2 D^{-1}(R - P Zin).
 template <int NV>
-__global__ __launch_bounds__(kSB) void k_blk_cheb_step(BlkOp o, int nv, int j, ColsC R, ColsC Zin,
-                                                       ColsW Zout, ColsW Dd) {
-  const int64_t row = xcd_block(true) * kSB + threadIdx.x;
+__global__ __launch_bounds__(kSB) void k_blk_cheb_step(BlkOp o, int nvall, int j, ColsC Rs,
+                                                       ColsC Zis, ColsW Zos, ColsW Ds) {
+  const int64_t row = xcd_block(true) * blockDim.x + threadIdx.x;
   if (row >= o.n) return;
-  const Cheb c = cheb_coef(cheb_hi(o.bound, o.upper), o.ratio, j);
+  const int q0 = int(blockIdx.y) * NV, nv = min(NV, nvall - q0);
+  const auto R = cols_at<NV>(Rs, q0, nv);
+  const auto Zin = cols_at<NV>(Zis, q0, nv);
+  const auto Zout = cols_at<NV>(Zos, q0, nv);
+  const auto Dd = cols_at<NV>(Ds, q0, nv);
+  const double c1 = o.coef[2 * j - 1], c2 = o.coef[2 * j];
   const bool last = j == o.iters - 1;
   double2 acc[NV];
   blk_row<NV>(o, row, nv, Zin, acc);
@@ -260,8 +348,8 @@ __global__ __launch_bounds__(kSB) void k_blk_cheb_step(BlkOp o, int nv, int j, C
       dinv<double>(b0, b1, b2, res0, res1, &u0, &u1);
       double2* dp = reinterpret_cast<double2*>(Dd.p[q]) + row;
       double2 d = *dp;
-      d.x = c.c1 * d.x + c.c2 * u0;
-      d.y = c.c1 * d.y + c.c2 * u1;
+      d.x = c1 * d.x + c2 * u0;
+      d.y = c1 * d.y + c2 * u1;
       if (!last) *dp = d;
       reinterpret_cast<double2*>(Zout.p[q])[row] = make_double2(zi.x + d.x, zi.y + d.y);
     }
@@ -275,20 +363,28 @@ C cols_of(const V& v, size_t from, int cnt) {
   return c;
 }
 
+dim3 blk_grid(int64_t n, int nv) {
+  return n <= kBlkSmall ? dim3(grid_for(n, 64), unsigned(nv + 1) / 2) : dim3(grid_for(n, kSB), 1);
+}
+
 // Y = J X (or P X) for any number of columns, kBV at a time.
 void blk_apply(const BlkOp& o, const std::vector<double*>& X, const std::vector<double*>& Y,
                hipStream_t s) {
   for (size_t f = 0; f < X.size(); f += kBV) {
     const int nv = int(std::min<size_t>(kBV, X.size() - f));
-    k_blk_apply<kBV><<<grid_for(o.n, kSB), kSB, 0, s>>>(o, nv, cols_of<ColsC>(X, f, nv),
-                                                        cols_of<ColsW>(Y, f, nv));
+    const bool small = o.n <= kBlkSmall;
+    (small ? k_blk_apply<2> : k_blk_apply<kBV>)<<<blk_grid(o.n, nv), small ? 64 : kSB, 0, s>>>(
+        o, nv, cols_of<ColsC>(X, f, nv), cols_of<ColsW>(Y, f, nv));
   }
 }
 
 // Z = Chebyshev(P) R for every column; T and Dd are scratch columns.
 void blk_cheb(const BlkOp& o, const std::vector<double*>& R, const std::vector<double*>& Z,
               const std::vector<double*>& T, const std::vector<double*>& Dd, hipStream_t s) {
-  const unsigned nb = grid_for(o.n, kSB);
+  const bool small = o.n <= kBlkSmall;
+  const int threads = small ? 64 : kSB;
+  const auto first = small ? k_blk_cheb_first<2> : k_blk_cheb_first<kBV>;
+  const auto step = small ? k_blk_cheb_step<2> : k_blk_cheb_step<kBV>;
   const int steps = o.iters < 1 ? 1 : o.iters;
   for (size_t f = 0; f < R.size(); f += kBV) {
     const int nv = int(std::min<size_t>(kBV, R.size() - f));
@@ -296,11 +392,12 @@ void blk_cheb(const BlkOp& o, const std::vector<double*>& R, const std::vector<d
     const ColsW d = cols_of<ColsW>(Dd, f, nv);
     const ColsW zb[2] = {cols_of<ColsW>(Z, f, nv), cols_of<ColsW>(T, f, nv)};
     int cur = (steps - 1) % 2;
-    k_blk_cheb_first<kBV><<<nb, kSB, 0, s>>>(o, nv, r, zb[cur], d);
+    const dim3 nb = blk_grid(o.n, nv);
+    first<<<nb, threads, 0, s>>>(o, nv, r, zb[cur], d);
     for (int j = 1; j < steps; ++j) {
       ColsC zin{};
       for (int q = 0; q < nv; ++q) zin.p[q] = zb[cur].p[q];
-      k_blk_cheb_step<kBV><<<nb, kSB, 0, s>>>(o, nv, j, r, zin, zb[1 - cur], d);
+      step<<<nb, threads, 0, s>>>(o, nv, j, r, zin, zb[1 - cur], d);
       cur = 1 - cur;
     }
   }
@@ -359,59 +456,94 @@ std::vector<const double*> cat(std::initializer_list<const std::vector<double*>*
 
 }  // namespace
 
-void block_dots(const double* const* A, int ma, const double* const* B, int mb, int64_t L,
-                BlockWork& w, double* out, hipStream_t s) {
+namespace {
+void launch_dots(const double* const* A, int ma, const double* const* B, int mb, int64_t L,
+                 BlockWork& w, double* out, hipStream_t s) {
   NOSH_CHECK(ma >= 1 && mb >= 1 && ma <= kMaxCols && mb <= kMaxCols && L % 2 == 0, kInvalid,
              "block_dots: bad block shape");
   const int64_t L2 = L / 2;
-  const int64_t nblk = std::max<int64_t>(1, std::min<int64_t>(1024, L2 / (kDotThreads * 8)));
+  const int64_t nblk = std::max<int64_t>(1, std::min<int64_t>(1024, L2 / (kDotThreads * 4)));
   const int64_t per = (L2 + nblk - 1) / nblk;
   const int ntiles = ((ma + 3) / 4) * ((mb + 3) / 4);
   const size_t need = size_t(ntiles) * 16 * nblk;
   if (w.partials.n < need) w.partials.alloc(need);
-  if (w.out.n < size_t(ma * mb)) w.out.alloc(kMaxCols * kMaxCols);
   ColsC a{}, b{};
   for (int i = 0; i < ma; ++i) a.p[i] = A[i];
   for (int j = 0; j < mb; ++j) b.p[j] = B[j];
   k_block_dots<<<unsigned(nblk * ntiles), kDotThreads, 0, s>>>(a, ma, b, mb, L2, per, int(nblk),
-                                                               w.partials.p);
-  k_block_dots_final<<<unsigned(ntiles * 16), kFinalizeThreads, 0, s>>>(w.partials.p, int(nblk),
-                                                                       ma, mb, w.out.p);
-  NOSH_HIP(hipMemcpyAsync(out, w.out.p, sizeof(double) * ma * mb, hipMemcpyDeviceToHost, s));
-  NOSH_HIP(hipStreamSynchronize(s));
+                                                               w.partials.p, out);
+  if (nblk > 1)
+    k_block_dots_final<<<unsigned(ntiles * 16), kFinalizeThreads, 0, s>>>(w.partials.p, int(nblk),
+                                                                         ma, mb, out);
 }
 
-void block_combine(const double* const* S, int m, const double* C, double* const* Y, int k,
-                   double beta, int64_t L, BlockWork& w, hipStream_t s) {
+void launch_combine(const double* const* S, int m, const double* C, const double* Cd,
+                    double cscale, double* const* Y, int k, double beta, int64_t L,
+                    hipStream_t s) {
+  ColsC sc{};
+  ColsW yc{};
+  CoefArg ca{};
+  for (int i = 0; i < m; ++i) sc.p[i] = S[i];
+  for (int j = 0; j < k; ++j) yc.p[j] = Y[j];
+  if (C) std::memcpy(ca.c, C, sizeof(double) * m * k);
+  const int64_t L2 = L / 2;
+  const auto f = k <= 4 ? k_block_combine<4> : k <= 8 ? k_block_combine<8> : k_block_combine<16>;
+  f<<<grid_for(L2, kCombThreads), kCombThreads, 0, s>>>(sc, m, ca, Cd, cscale, yc, k, beta, L2);
+}
+
+void check_combine(const double* const* S, int m, double* const* Y, int k, int64_t L) {
   NOSH_CHECK(m >= 1 && m <= kMaxCols && k >= 1 && k <= 16 && L % 2 == 0, kInvalid,
              "block_combine: bad block shape");
   for (int j = 0; j < k; ++j)
     for (int i = 0; i < m; ++i)
       NOSH_CHECK(Y[j] != S[i], kInvalid, "block_combine: output aliases an input");
-  ColsC sc{};
-  ColsW yc{};
-  for (int i = 0; i < m; ++i) sc.p[i] = S[i];
-  for (int j = 0; j < k; ++j) yc.p[j] = Y[j];
-  const int64_t L2 = L / 2;
-  const unsigned grid = grid_for(L2, kCombThreads);
+}
+}  // namespace
+
+void block_dots(const double* const* A, int ma, const double* const* B, int mb, int64_t L,
+                BlockWork& w, double* out, hipStream_t s) {
+  if (!w.host)
+    NOSH_HIP(hipHostMalloc(reinterpret_cast<void**>(&w.host),
+                           sizeof(double) * kMaxCols * kMaxCols));
+  launch_dots(A, ma, B, mb, L, w, w.host, s);
+  NOSH_HIP(hipStreamSynchronize(s));
+  std::memcpy(out, w.host, sizeof(double) * ma * mb);
+}
+
+void block_dots_device(const double* const* A, int ma, const double* const* B, int mb, int64_t L,
+                       BlockWork& w, hipStream_t s) {
+  if (!w.out.p) w.out.alloc(kMaxCols * kMaxCols);
+  launch_dots(A, ma, B, mb, L, w, w.out.p, s);
+}
+
+void block_combine(const double* const* S, int m, const double* C, double* const* Y, int k,
+                   double beta, int64_t L, BlockWork& w, hipStream_t s) {
+  check_combine(S, m, Y, k, L);
   if (m * k <= kArgCoefs) {
-    CoefArg ca;
-    std::memcpy(ca.c, C, sizeof(double) * m * k);
-    k_block_combine<true><<<grid, kCombThreads, 0, s>>>(sc, m, ca, nullptr, yc, k, beta, L2);
+    launch_combine(S, m, C, nullptr, 1.0, Y, k, beta, L, s);
     return;
   }
   if (w.coef.n < size_t(kMaxCols * 16)) w.coef.alloc(kMaxCols * 16);
   // Synchronous upload: the host array may change right after this call.
   NOSH_HIP(hipStreamSynchronize(s));
   NOSH_HIP(hipMemcpy(w.coef.p, C, sizeof(double) * m * k, hipMemcpyHostToDevice));
-  k_block_combine<false><<<grid, kCombThreads, 0, s>>>(sc, m, CoefArg{}, w.coef.p, yc, k, beta,
-                                                       L2);
+  launch_combine(S, m, nullptr, w.coef.p, 1.0, Y, k, beta, L, s);
+}
+
+void block_subtract(const double* const* S, int m, double* const* Y, int k, int64_t L,
+                    BlockWork& w, hipStream_t s) {
+  check_combine(S, m, Y, k, L);
+  launch_combine(S, m, nullptr, w.out.p, -1.0, Y, k, 1.0, L, s);
 }
 
 void sym_eig(int n, std::vector<double> A, std::vector<double>& w, std::vector<double>& V) {
   // Cyclic Jacobi rotations (Golub & Van Loan, Matrix Computations, 8.5):
   // each rotation zeroes A_pq with t = tan(phi) the smaller root of
-  // t^2 + 2 t zeta - 1 = 0, zeta = (A_qq - A_pp) / (2 A_pq).
+  // t^2 + 2 t zeta - 1 = 0, zeta = (A_qq - A_pp) / (2 A_pq). The entry is set
+  // to that zero: as the rounding of the two updates, eps of the diagonal, it
+  // kept the off-diagonal part from ever meeting the end test, and an 18 x 18
+  // problem went through all 100 sweeps where 7 or 8 meet it (the smallest six
+  // of the Jacobian on 1089 vertices: 40 ms -> 12 ms, with the test as it was).
   V.assign(size_t(n) * n, 0.0);
   for (int i = 0; i < n; ++i) V[size_t(i) * n + i] = 1.0;
   for (int sweep = 0; sweep < 100; ++sweep) {
@@ -440,6 +572,7 @@ void sym_eig(int n, std::vector<double> A, std::vector<double>& w, std::vector<d
           A[size_t(p) * n + k] = c * apk - sn * aqk;
           A[size_t(q) * n + k] = sn * apk + c * aqk;
         }
+        A[size_t(p) * n + q] = A[size_t(q) * n + p] = 0.0;
         for (int k = 0; k < n; ++k) {
           const double vkp = V[size_t(k) * n + p], vkq = V[size_t(k) * n + q];
           V[size_t(k) * n + p] = c * vkp - sn * vkq;
@@ -478,16 +611,15 @@ struct Lobpcg {
     block_dots(A.data(), int(A.size()), B.data(), int(B.size()), L, bw, r.data(), s);
     return r;
   }
-  // Y -= Q (Q^T Y) for orthonormal Q; tracked: AY -= AQ (same coefficients).
+  // Y -= Q (Q^T Y) for orthonormal Q; tracked: AY -= AQ (same coefficients,
+  // which stay on the device).
   void project(const std::vector<const double*>& Q, std::vector<double*>& Y,
                const std::vector<const double*>* AQ = nullptr, std::vector<double*>* AY = nullptr) {
     if (Q.empty() || Y.empty()) return;
-    std::vector<double> c = dots(Q, cview(Y));
-    for (double& v : c) v = -v;
-    block_combine(Q.data(), int(Q.size()), c.data(), Y.data(), int(Y.size()), 1.0, L, bw, s);
-    if (AQ && AY)
-      block_combine(AQ->data(), int(AQ->size()), c.data(), AY->data(), int(AY->size()), 1.0, L,
-                    bw, s);
+    const std::vector<const double*> y = cview(Y);
+    block_dots_device(Q.data(), int(Q.size()), y.data(), int(y.size()), L, bw, s);
+    block_subtract(Q.data(), int(Q.size()), Y.data(), int(Y.size()), L, bw, s);
+    if (AQ && AY) block_subtract(AQ->data(), int(AQ->size()), AY->data(), int(AY->size()), L, bw, s);
   }
   // Replaces V (and AV) by an orthonormal basis of span(V) (SVQB); returns
   // the number of columns kept.
@@ -566,8 +698,10 @@ int lobpcg_jacobian(nosh_nls_s* nls, const double* psi_int, const std::map<std::
   launch_rebuild_blocks(m, nls->keo->kv, nls->ct.p, V, g, psi_int, nls->jblk.p, nls->pblk.p,
                         nls->bound.p, s);
   int applies = 0;
+  DBuf<double> coef(2 * size_t(std::max(o.cheb_iters, 1)));
   BlkOp jop{n, sell_view(m), nls->keo->kv.val.p, nls->jblk.p, nls->bound.p, 0.0,
-            o.cheb_ratio, o.cheb_iters};
+            o.cheb_ratio, o.cheb_iters, coef.p};
+  k_blk_coef<<<1, 1, 0, s>>>(jop);
   BlkOp pop = jop;
   pop.blk = nls->pblk.p;
   auto applyJ = [&](const std::vector<double*>& X, std::vector<double*>& Y) {
@@ -671,22 +805,17 @@ int lobpcg_jacobian(nosh_nls_s* nls, const double* psi_int, const std::map<std::
       lb.pool.give(W);
       W = Z;
     }
-    const auto cX = cview(X);
-    const auto cAX = cview(AX);
-    for (int rep = 0; rep < 2; ++rep) {
-      lb.project(Q, W);
-      lb.project(cX, W);
-    }
+    // Against the phase direction and X (orthonormal together), twice.
+    std::vector<const double*> QX(Q);
+    QX.insert(QX.end(), X.begin(), X.end());
+    for (int rep = 0; rep < 2; ++rep) lb.project(QX, W);
     lb.svqb(W);
     if (W.empty()) break;  // the residuals vanished to rounding
     AW = lb.pool.take(int(W.size()));
     applyJ(W, AW);
     if (!Pd.empty()) {
-      const auto cW = cview(W), cAW = cview(AW);
-      for (int rep = 0; rep < 2; ++rep) {
-        lb.project(cX, Pd, &cAX, &AP);
-        lb.project(cW, Pd, &cAW, &AP);
-      }
+      const std::vector<const double*> XW = cat({&X, &W}), AXW = cat({&AX, &AW});
+      for (int rep = 0; rep < 2; ++rep) lb.project(XW, Pd, &AXW, &AP);
       lb.svqb(Pd, &AP);
     }
     // Rayleigh-Ritz on S = [X, W, P].

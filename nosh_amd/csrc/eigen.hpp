@@ -17,7 +17,13 @@ constexpr int kMaxCols = 48;
 // Scratch of the block operations (grown on demand).
 struct BlockWork {
   DBuf<double> partials, out, coef;
-  std::vector<double> host;
+  double* host = nullptr;  // pinned, written by the kernels themselves
+  BlockWork() = default;
+  BlockWork(const BlockWork&) = delete;
+  BlockWork& operator=(const BlockWork&) = delete;
+  ~BlockWork() {
+    if (host) (void)hipHostFree(host);
+  }
 };
 
 // out (host, ma x mb, row-major) = A^T B over L rows; columns by pointer.
@@ -25,10 +31,18 @@ struct BlockWork {
 void block_dots(const double* const* A, int ma, const double* const* B, int mb, int64_t L,
                 BlockWork& w, double* out, hipStream_t s);
 
+// The same left in w.out on the device, without waiting.
+void block_dots_device(const double* const* A, int ma, const double* const* B, int mb, int64_t L,
+                       BlockWork& w, hipStream_t s);
+
 // Y_j = beta Y_j + sum_i C[i k + j] S_i for j < k (C host, m x k row-major).
 // No Y_j may alias an S_i.
 void block_combine(const double* const* S, int m, const double* C, double* const* Y, int k,
                    double beta, int64_t L, BlockWork& w, hipStream_t s);
+
+// Y_j -= sum_i w.out[i k + j] S_i (the coefficients block_dots_device left).
+void block_subtract(const double* const* S, int m, double* const* Y, int k, int64_t L,
+                    BlockWork& w, hipStream_t s);
 
 // Symmetric eigendecomposition of a small dense matrix (cyclic Jacobi):
 // A (n x n row-major, symmetric) -> w ascending, V[i n + j] = component i of

@@ -246,3 +246,40 @@ def test_invalid_options_are_errors_not_crashes():
     assert np.linalg.norm(om.f(psi)) <= 1e-9
     ev, _, st = nosh.jacobian_eigenpairs(model, psi, {"g": 1.0, "mu": 0.05}, nev=2, tol=1e-9)
     assert st["converged"] == 2 and ev[0] > 0
+
+
+@pytest.mark.parametrize("nev,block", [(1, 1), (2, 3), (5, 8), (16, 16)])
+def test_eigenvalues_at_other_block_sizes(nev, block):
+    """Block products of 1 to 48 columns (every width of the combination kernel,
+    the padded ones, and blocks above 8, whose X and P are combined apart):
+    the smallest eigenvalues of the 8x8 square's J, phase mode deflated, against
+    numpy's eigh of the oracle's dense J."""
+    import nosh_amd as nosh
+    c, t, model, om = _setup(8)
+    psi = _meissner(model, c.shape[0], 0.2)
+    w, wd, _ = _dense_spectrum(om, psi, 0.2)
+    ev, _, st = nosh.jacobian_eigenpairs(model, psi, {"g": 1.0, "mu": 0.2}, nev=nev,
+                                         block_size=block, tol=1e-10, max_iters=2000)
+    assert st["converged"] == nev
+    assert np.allclose(ev, wd[:nev], rtol=1e-8, atol=1e-11 * np.abs(w).max())
+
+
+@pytest.mark.parametrize("ncell", [446, 447])
+def test_eigenvectors_at_the_column_split(ncell):
+    """199809 and 200704 rows, the two sides of the line between two and eight
+    columns a thread: the pairs of J at psi = 1, mu = 0 are pairs of the
+    oracle's J. The solver ends at 1e-8 of the largest Rayleigh quotient of its
+    start, random vectors; |J x| / |x| of one such vector is no smaller."""
+    import nosh_amd as nosh
+    c, t, model, om = _setup(ncell)
+    psi = np.zeros(2 * c.shape[0])
+    psi[0::2] = 1.0
+    ev, vec, st = nosh.jacobian_eigenpairs(model, psi, {"g": 1.0, "mu": 0.0}, nev=2, vectors=True,
+                                           tol=1e-8, max_iters=1000)
+    assert st["converged"] == 2
+    om.set_params(1.0, 0.0)
+    om.jac_rebuild(psi)
+    x = np.random.default_rng(5).standard_normal(psi.size)
+    scale = np.linalg.norm(om.jac(x)) / np.linalg.norm(x)
+    for j in range(2):
+        assert np.linalg.norm(om.jac(vec[j]) - ev[j] * vec[j]) <= 2e-8 * scale
