@@ -76,6 +76,7 @@ struct ChebArgs {
   V2<T>* r;            // residual (written by mode 2's first step)
   const V2<T>* r2;     // mode 2: the previous residual
   const V2<T>* u;      // mode 2: J v - (beta/oldb) r1
+  V2<T>* D;            // the Chebyshev direction (FP32)
   MinresScalars* S;
   double* coef;
   const double* pa;    // partial sums of alfa, na of them (mode 2)
@@ -144,10 +145,11 @@ __global__ __launch_bounds__(kBlock) void k_cheb_first(ChebArgs<T> a, int mode, 
   block_partials<1>(s2, a.pb);
 }
 
-// Chebyshev step j >= 1 in three-term form,
-//   z_j = z_{j-1} + c1 (z_{j-1} - z_{j-2}) + c2 D^{-1} (r - P z_{j-1}),
-// z_{-1} = 0; z_{j-2} sits in z_j's buffer and is overwritten by its own
-// thread, so no direction vector is stored.
+// Chebyshev step j >= 1: z_j = z_{j-1} + d_j, d_0 = z_0,
+// d_j = c1 d_{j-1} + c2 D^{-1} (r - P z_{j-1}). In FP64 d_{j-1} is the
+// difference of the last two z (z_{j-2} sits in z_j's buffer and is overwritten
+// by its own thread), which saves a write (96^3: 3 % of a solve). In FP32 it is
+// stored by the steps that have a next one, not to carry the rounding of z.
 template <class T, int P>
 __global__ __launch_bounds__(kBlock) void k_cheb_step(ChebArgs<T> a, int mode, int j,
                                                      const V2<T>* __restrict__ zin,
@@ -158,12 +160,21 @@ __global__ __launch_bounds__(kBlock) void k_cheb_step(ChebArgs<T> a, int mode, i
   const int done = mode != 0 ? S->done : 0;
   const RowBlock<P> rb(a.n);
   const int64_t row = rb.row;
-  V2<T> zi{}, rv{}, zpp{};
+  V2<T> zi{}, rv{}, d{};
   T b0 = T(1), b1 = T(1), b2 = T(0);
   if (rb.owner) {
     zi = zin[row];
     rv = a.r[row];
-    if (j > 1) zpp = zout[row];
+    d = zi;
+    if (j > 1) {
+      if constexpr (sizeof(T) == 4) {
+        d = a.D[row];
+      } else {
+        const V2<T> zpp = zout[row];
+        d.x -= zpp.x;
+        d.y -= zpp.y;
+      }
+    }
     b0 = a.pblk[row], b1 = a.pblk[a.n + row], b2 = a.pblk[2 * a.n + row];
   }
   const T c1 = T(a.coef[2 * j - 1]), c2 = T(a.coef[2 * j]);
@@ -175,9 +186,12 @@ __global__ __launch_bounds__(kBlock) void k_cheb_step(ChebArgs<T> a, int mode, i
     const T res1 = rv.y - (acc.y + b2 * zi.x + b1 * zi.y);
     T u0, u1;
     dinv<T>(b0, b1, b2, res0, res1, &u0, &u1);
+    d.x = c1 * d.x + c2 * u0;
+    d.y = c1 * d.y + c2 * u1;
     V2<T> z;
-    z.x = zi.x + (c1 * (zi.x - zpp.x) + c2 * u0);
-    z.y = zi.y + (c1 * (zi.y - zpp.y) + c2 * u1);
+    z.x = zi.x + d.x;
+    z.y = zi.y + d.y;
+    if (sizeof(T) == 4 && j != a.iters - 1) a.D[row] = d;
     zout[row] = z;
     s2 = double(rv.x) * double(z.x) + double(rv.y) * double(z.y);
   }
@@ -351,6 +365,7 @@ void MinresWork<T>::ensure(int64_t n_) {
   if (n == n_) return;
   n = n_;
   for (auto* b : {&Y, &Z2, &v, &u, &R0, &R1, &W0, &W1, &W2}) b->alloc(n);
+  if (sizeof(T) == 4) D.alloc(n);
   x.alloc(n);
   partials.alloc(2 * size_t(grid_for(n, kSliceH) + 4));  // one per slice, whatever its waves
   if (!S.p) S.alloc(2);
@@ -377,6 +392,7 @@ static ChebArgs<T> cheb_args(const MeshCache& m, const PrecView<T>& P, MinresWor
   a.ratio = P.ratio;
   a.iters = P.iters;
   a.u = w.u.p;
+  a.D = w.D.p;
   a.S = w.S.p;
   a.coef = w.coef.p;
   a.pa = w.partials.p;

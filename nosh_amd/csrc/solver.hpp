@@ -20,7 +20,7 @@ struct MinresScalars {
 template <class T>
 struct MinresWork {
   int64_t n = -1;
-  DBuf<V2<T>> Y, Z2, v, u, R0, R1, W0, W1, W2;
+  DBuf<V2<T>> Y, Z2, v, u, R0, R1, D, W0, W1, W2;
   DBuf<double2> x;
   DBuf<double> partials;  // of alfa, then of beta^2
   DBuf<double> coef;      // Chebyshev coefficients of the current chain
