@@ -736,7 +736,7 @@ def surrogate_mfma(rows, stream, dev, nin=9, width=256, depth=4, reps=5):
     flop_all = 2.0 * rows * (nin * width + (depth - 1) * width * width + width * 2)
     ach = flop_mfma / t / 1e12
     say(f"surrogate inference: {rows} rows in {t*1e3:.2f} ms -> {ach:.1f} TFLOP/s on MFMA")
-    return {"bound": "mfma", "kernel": "k_mlp_infer<8> (fused BF16 MLP inference)",
+    return {"bound": "mfma", "kernel": "k_mlp_fused (fused BF16 MLP inference)",
             "rows": rows, "ms_per_launch": round(t * 1e3, 3), "achieved": round(ach, 1),
             "peak": 2500.0, "unit": "TFLOP/s", "frac": round(ach / 2500.0, 4),
             "all_layers_TFLOPs": round(flop_all / t / 1e12, 1)}
