@@ -306,3 +306,34 @@ def test_row_products_at_the_split_sizes(ncell):
     r = b - om.jac(x)
     assert r @ P.apply(r) <= (1 + 1e-10) * (b @ P.apply(b))
     assert abs(np.sqrt(r @ P.apply(r) / (b @ P.apply(b))) - rr) <= 1e-8
+
+
+@pytest.mark.parametrize("ring", [16, 33, 100])
+@pytest.mark.parametrize("reorder", [True, False])
+def test_fp32_products_of_long_rows(ring, reorder):
+    """A fan's centre has a row of `ring` slots, more than a wave may leave in
+    LDS (the owner adds the rest), in the upper half as vertex 0 and in the
+    lower one as the last vertex. One Newton step of 8 MINRES iterations with
+    FP32 inner solves against the FP64 one: the update within 1e-4 of its norm
+    (100 terms of a row x 8 iterations x 5 products x the FP32 unit roundoff
+    6e-8 is 2.4e-4 at the very worst, and roundings do not all add up)."""
+    import nosh_amd as nosh
+    a = 2 * np.pi * np.arange(ring) / ring
+    rim = np.stack([np.cos(a), np.sin(a), 0 * a], axis=1)
+    for centre in (0, ring):
+        coords = np.insert(rim, centre, 0.0, axis=0)
+        k = np.arange(ring) + (centre == 0)
+        cells = np.stack([np.full(ring, centre), k, np.roll(k, -1)], axis=1).astype(np.int32)
+        gm = nosh.Mesh(coords, cells, reorder=reorder)
+        mvp = nosh.VectorFieldExplicitValues(gm, mg.magnetic_potential(coords), 0.2)
+        model = nosh.Nls(gm, mvp, nosh.ScalarFieldConstant(gm, -1.0), 1.3,
+                         nosh.ScalarFieldConstant(gm, 1.0))
+        psi0 = mg.random_state(ring + 1, 5)
+        step = []
+        for precision in (0, 1):
+            psi, _ = nosh.newton_solve(model, psi0, {"g": 1.3, "mu": 0.2}, tol=0.0, max_iters=1,
+                                       minres_rtol=0.0, minres_max_iters=8, cheb_iters=5,
+                                       cheb_ratio=30.0, precision=precision)
+            step.append(psi - psi0)
+        assert np.linalg.norm(step[0]) > 1e-3
+        assert np.linalg.norm(step[1] - step[0]) <= 1e-4 * np.linalg.norm(step[0])
