@@ -360,8 +360,8 @@ int nosh_mlp_set_params(nosh_mlp_t mlp, const float* params);
 int nosh_mlp_forward(nosh_mlp_t mlp, const float* X, int64_t M, float* Y);
 int nosh_mlp_forward_device(nosh_mlp_t mlp, const float* X, int64_t M, float* Y, void* stream);
 /* Inference only: the same outputs as nosh_mlp_forward from one fused kernel
- * (activations in LDS between the layers, all of them on MFMA) when width is
- * 64, 128 or 256 and n_in <= 32, as the forward does too; otherwise the
+ * (activations in LDS between the layers) when width is 64, 128 or 256 and
+ * n_in <= 32, as the forward does too; otherwise, to the same bits, the
  * layer-by-layer path. */
 int nosh_mlp_infer(nosh_mlp_t mlp, const float* X, int64_t M, float* Y);
 int nosh_mlp_infer_device(nosh_mlp_t mlp, const float* X, int64_t M, float* Y, void* stream);

@@ -35,24 +35,26 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int kBM = 64, kBN = 128, kBK = 32, kPad = 8;
 constexpr int kLds = kBK + kPad;  // bf16 per LDS row
 
-// With u = sqrt(2/pi) (z + 0.044715 z^3) the tanh form is z sigma(2u):
-// (1 + tanh u) / 2 = 1 / (1 + exp(-2u)), one hardware exponential and one
-// reciprocal (relative error ~1e-6, far below the BF16 rounding the
-// activations take next), and no cancellation for negative z. exp(-2u) = inf
-// gives 0, 0 gives 1. Five ordinary and two quarter-rate instructions; they,
-// not the matrix cores, set the pace of the fused network.
-__device__ __forceinline__ float gelu_sigma(float z) {
-  const float k = -2.0f * 0.7978845608028654f * 1.4426950408889634f;  // -2 sqrt(2/pi) log2(e)
-  const float e = __builtin_amdgcn_exp2f(z * (k + k * 0.044715f * z * z));
-  return __builtin_amdgcn_rcpf(1.0f + e);
+// r = 1 / (exp(2u) + 1), u = sqrt(2/pi) (z + 0.044715 z^3), with the hardware
+// exponential and reciprocal (relative error ~1e-6, far below the BF16 rounding
+// the activations take next; exp(2u) = inf gives 0, 0 gives 1): tanh u = 1 - 2 r.
+__device__ __forceinline__ float gelu_r(float z) {
+  const float c = 0.7978845608028654f;  // sqrt(2/pi)
+  return __builtin_amdgcn_rcpf(__expf(2.0f * c * (z + 0.044715f * z * z * z)) + 1.0f);
 }
 
-__device__ __forceinline__ float gelu(float z) { return z * gelu_sigma(z); }
+// z/2 (1 + tanh u), the halvings exact: the bits are those of
+// 0.5f * z * (1.0f + (1.0f - 2.0f * r)) at one instruction less. Its nine
+// ordinary and two quarter-rate instructions, not the matrix cores, set the
+// pace of the fused network. (z (1 - r) would be one less yet, but does not
+// round tanh u as the derivative does; those last bits flip BF16 roundings of
+// the activations, 1e-4 of the outputs at depth 4.)
+__device__ __forceinline__ float gelu(float z) { return z * (0.5f + (0.5f - gelu_r(z))); }
 
 __device__ __forceinline__ float dgelu(float z) {
   const float c = 0.7978845608028654f;
-  const float t = gelu_sigma(z);
-  return t + z * t * (1.0f - t) * (2.0f * c + 6.0f * c * 0.044715f * z * z);
+  const float t = 1.0f - 2.0f * gelu_r(z);
+  return 0.5f * (1.0f + t) + 0.5f * z * (1.0f - t * t) * c * (1.0f + 3.0f * 0.044715f * z * z);
 }
 
 struct GemmArgs {
@@ -303,8 +305,8 @@ __global__ void k_f32_to_bf16(const float* __restrict__ a, int64_t n, __bf16* __
 // ------------------------------------------------------- fused network
 // Widths 64, 128 and 256 with n_in <= 32: the whole network for R = 128, 64 or
 // 32 rows in one workgroup of 4 waves, the activations (BF16) in LDS between layers,
-// every layer on MFMA with FP32 accumulation; in training the same kernel
-// goes on to the loss and back through the layers.
+// all layers but the last on MFMA with FP32 accumulation; in training the same
+// kernel goes on to the loss and back through the layers.
 //
 // Weights come as operand fragments: the 64 lanes' 8-element operands of one
 // MFMA in lane order, 1 KB contiguous (make_fragments lays them out once
@@ -319,13 +321,17 @@ __global__ void k_f32_to_bf16(const float* __restrict__ a, int64_t n, __bf16* __
 // staged through LDS (135 KB, one workgroup a CU): 1.5 LDS reads an MFMA
 // where 1 read of 8 cycles in 32 is the limit of four waves.
 // Measured (width 256, depth 4, n_in 7): inference of 912,673 rows 2310 ->
-// 542 us (670 TFLOP/s; the GELUs alone are ~0.35 ms of vector issue), four
-// Adam steps on 16,384 rows 5.95 -> 0.67 ms (1.06 with 128 rows a workgroup).
+// 568 us (640 TFLOP/s; the GELUs alone are ~0.46 ms of vector issue), four
+// Adam steps on 16,384 rows 5.95 -> 0.66 ms (1.06 with 128 rows a workgroup).
 //
-// Layer 0 takes its FP32 inputs as three BF16 parts of 8 bits each
-// (x = x1 + x2 + x3 exactly), times the same BF16 weight: exact products,
-// FP32 sums, as the scalar form. The same split serves dy and x in the
-// weight gradients.
+// Every value is, bit for bit, that of the layer-by-layer path: layer 0 runs on
+// the FP32 matrix instruction (32x32x2, whose sums round like the chain of
+// fmaf over the inputs, from the bias on), the hidden layers take the same
+// k-steps, and the last layer is the FP32 chain over k, a row and output per
+// lane with its weights in scalar registers (on the matrix cores 30 of 32
+// columns would be padding).
+// In the weight gradients x and dy are split into three BF16 parts of 8 bits
+// each (x = x1 + x2 + x3 exactly): exact products with the BF16 dz and h.
 constexpr int kFusedMaxIn = 32;
 constexpr int kMaxLayers = 18;
 constexpr int kFrag = 512;  // bf16 per operand fragment
@@ -333,10 +339,11 @@ constexpr int kFrag = 512;  // bf16 per operand fragment
 struct FusedArgs {
   const float* X;
   int64_t M;
-  int nin, kp, depth, nout;  // kp: 3 nin + 1 rounded up to 32
-  const bf16x8* wf;          // forward fragments: layer 0, hidden layers, last layer
-  const bf16x8* wb;          // transposed fragments of the hidden layers (training)
-  const __bf16* wlast;       // last layer, [nout][width]
+  int nin, kx, kp, depth, nout;  // kx: nin rounded up to 2; kp: 3 nin + 1 up to 32
+  const float* w0;           // layer 0's FP32 fragments
+  const bf16x8* wf;          // forward fragments of the hidden layers
+  const bf16x8* wb;          // transposed ones (training)
+  const float* wlast;        // last layer, [nout][width]
   const float* bias;
   int64_t boff[kMaxLayers];
   float* Y;  // inference
@@ -352,9 +359,9 @@ struct FusedArgs {
   int dy_lds;      // LDS offset of the rows' dy
 };
 
-// Fragments per layer.
-__host__ __device__ inline int64_t frags_first(int width, int kp) {
-  return int64_t(width / 32) * (kp / 16);
+// Fragments per layer (layer 0: 64 floats each, 32 outputs of 2 inputs).
+__host__ __device__ inline int64_t frags_first(int width, int kx) {
+  return int64_t(width / 32) * (kx / 2);
 }
 __host__ __device__ inline int64_t frags_hidden(int width) {
   return int64_t(width / 32) * (width / 16);
@@ -477,88 +484,110 @@ k_mlp_fused(FusedArgs g) {
     *reinterpret_cast<uint2*>(act + r * LD + n) = make_uint2(pack2(a, b), pack2(c, d));
   };
   auto zslot = [&](int l, int i) { return ((blk * g.depth + l) * C::Q + i) * 256 + tid; };
-  // z = acc + bias, h = gelu(z) of layer l into the activations.
+  // z = acc + bias (layer 0 starts from it), h = gelu(z) into the activations.
   auto activate = [&](int l) {
     const float* bl = g.bias + g.boff[l];
     __syncthreads();  // every wave has read the previous activations
     each([&](int i, int r, int n, float4 v) {
-      const float4 b = *reinterpret_cast<const float4*>(bl + n);
-      v = make_float4(v.x + b.x, v.y + b.y, v.z + b.z, v.w + b.w);
+      if (l > 0) {
+        const float4 b = *reinterpret_cast<const float4*>(bl + n);
+        v = make_float4(v.x + b.x, v.y + b.y, v.z + b.z, v.w + b.w);
+      }
       if constexpr (TRAIN) g.z[zslot(l, i)] = v;
       put(r, n, gelu(v.x), gelu(v.y), gelu(v.z), gelu(v.w));
     });
     __syncthreads();
   };
 
-  // Layer 0 from the split inputs (stored over the activations).
-  const int lx = g.kp + 8;
-  for (int i = tid; i < kRows * g.kp; i += 256) {
-    const int r = i / g.kp, k = i - r * g.kp;
-    const int part = k / g.nin, c = k - part * g.nin;
-    __bf16 v = __bf16(k == 3 * g.nin ? 1.0f : 0.0f);
-    if (part < 3) v = split_part(r < rows ? g.X[(r0 + r) * g.nin + c] : 0.0f, part);
-    act[r * lx + k] = v;
+  // Layer 0 (its inputs where the activations will be; an odd row pitch).
+  float* xs = reinterpret_cast<float*>(lds);
+  const int lx = g.kx + 1;
+  for (int i = tid; i < kRows * g.kx; i += 256) {
+    const int r = i / g.kx, c = i - r * g.kx;
+    xs[r * lx + c] = r < rows && c < g.nin ? g.X[(r0 + r) * g.nin + c] : 0.0f;
   }
-  const bf16x8* whid = g.wf + frags_first(W, g.kp) * 64;
-  if (g.depth > 1) prefetch(whid);
+  if (g.depth > 1) prefetch(g.wf);
   __syncthreads();
-  clear();
-  for (int kc = 0; kc < g.kp / 16; ++kc) {
-    bf16x8 a[NT];
 #pragma unroll
-    for (int t = 0; t < NT; ++t) a[t] = g.wf[((n0 / 32 + t) * (g.kp / 16) + kc) * 64 + lane];
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float4 b =
+          *reinterpret_cast<const float4*>(g.bias + g.boff[0] + n0 + t * 32 + 8 * q + 4 * half);
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        acc[m][t][4 * q] = b.x, acc[m][t][4 * q + 1] = b.y;
+        acc[m][t][4 * q + 2] = b.z, acc[m][t][4 * q + 3] = b.w;
+      }
+    }
+  for (int kc = 0; kc < g.kx / 2; ++kc) {
+    float a[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) a[t] = g.w0[((n0 / 32 + t) * (g.kx / 2) + kc) * 64 + lane];
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
-      const bf16x8 b = *reinterpret_cast<const bf16x8*>(act + (m0 + m * 32 + col) * lx + kc * 16 +
-                                                        8 * half);
+      const float b = xs[(m0 + m * 32 + col) * lx + 2 * kc + half];
 #pragma unroll
       for (int t = 0; t < NT; ++t)
-        acc[m][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[t], b, acc[m][t], 0, 0, 0);
+        acc[m][t] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[t], b, acc[m][t], 0, 0, 0);
     }
   }
-  if constexpr (TRAIN) transpose_out(act, lx, g.kp / 32, g.xT);
+  if constexpr (TRAIN) {
+    const int tiles = g.kp / 32;
+    for (int f = wave; f < tiles * (kRows / 16); f += 4) {
+      const int mc = f / tiles, k = (f - mc * tiles) * 32 + col;
+      const int part = k / g.nin, c = k - part * g.nin;
+      bf16x8 v;
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        v[j] = part < 3 ? split_part(xs[(mc * 16 + 8 * half + j) * lx + c], part)
+                        : __bf16(k == 3 * g.nin ? 1.0f : 0.0f);
+      g.xT[((blk * (kRows / 16) + mc) * tiles + (f - mc * tiles)) * 64 + lane] = v;
+    }
+  }
   activate(0);
   const int64_t lstride = nchunk * (W / 32) * 64;  // one layer of hT / dzT
   for (int l = 1; l < g.depth; ++l) {
     if constexpr (TRAIN) transpose_out(act, LD, W / 32, g.hT + (l - 1) * lstride);
-    product(whid + (l - 1) * frags_hidden(W) * 64);
-    if (l + 1 < g.depth) prefetch(whid + l * frags_hidden(W) * 64);
+    product(g.wf + (l - 1) * frags_hidden(W) * 64);
+    if (l + 1 < g.depth) prefetch(g.wf + l * frags_hidden(W) * 64);
     activate(l);
   }
-  // Last layer: wave w takes the rows 32 w .. 32 w + 31 while there are any.
-  const bool owave = wave < kRows / 32;
-  f32x16 out;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) out[r] = 0.0f;
-  const bf16x8* wo = whid + (g.depth - 1) * frags_hidden(W) * 64;
-  const int orow = wave * 32 + col;
-  if (owave) {
+  // Last layer: f(row, output, y) once for each.
+  constexpr int kGroups = (kRows + 63) / 64;  // of 64 rows
+  auto last_layer = [&](auto f) {
+    for (int u = wave; u < kGroups * g.nout; u += 4) {
+      const int o = uniform(u / kGroups), r = (u % kGroups) * 64 + lane;
+      if (r >= kRows) continue;
+#if __HIP_DEVICE_COMPILE__
+      // Never written by this kernel, and the same for the whole wave.
+      const auto w = (const __attribute__((address_space(4))) float*)(g.wlast + int64_t(o) * W);
+#else
+      const float* w = g.wlast + int64_t(o) * W;
+#endif
+      float s = g.bias[g.boff[g.depth] + o];
 #pragma unroll 4
-    for (int kc = 0; kc < KC; ++kc)
-      out = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-          wo[kc * 64 + lane],
-          *reinterpret_cast<const bf16x8*>(act + orow * LD + kc * 16 + 8 * half), out, 0, 0, 0);
-  }
-  const float* bo = g.bias + g.boff[g.depth];
-  if constexpr (!TRAIN) {
+      for (int k = 0; k < W; k += 8) {
+        const bf16x8 h = *reinterpret_cast<const bf16x8*>(act + r * LD + k);
 #pragma unroll
-    for (int r = 0; r < 8; ++r) {  // n_out <= 16
-      const int o = 8 * (r >> 2) + 4 * half + (r & 3);
-      if (o < g.nout && orow < rows && owave) g.Y[(r0 + orow) * g.nout + o] = out[r] + bo[o];
+        for (int e = 0; e < 8; ++e) s += float(h[e]) * w[k + e];
+      }
+      f(r, o, s);
     }
+  };
+  if constexpr (!TRAIN) {
+    last_layer([&](int r, int o, float y) {
+      if (r < rows) g.Y[(r0 + r) * g.nout + o] = y;
+    });
     return;
   } else {
     float* dys = reinterpret_cast<float*>(lds + g.dy_lds);
     double sq[1] = {0.0};
-#pragma unroll
-    for (int r = 0; r < 8; ++r) {
-      const int o = 8 * (r >> 2) + 4 * half + (r & 3);
-      if (o >= g.nout || !owave) continue;
-      float d = 0.0f;
-      if (orow < rows) d = out[r] + bo[o] - g.T[(r0 + orow) * g.nout + o];
-      dys[orow * g.nout + o] = 2.0f * d * g.scale;
+    last_layer([&](int r, int o, float y) {
+      const float d = r < rows ? y - g.T[(r0 + r) * g.nout + o] : 0.0f;
+      dys[r * g.nout + o] = 2.0f * d * g.scale;
       sq[0] += double(d) * double(d);
-    }
+    });
     transpose_out(act, LD, W / 32, g.hT + (g.depth - 1) * lstride);
     const bf16x8* wback = g.wb + (g.depth - 2) * frags_hidden(W) * 64;
     if (g.depth > 1) prefetch(wback);
@@ -583,11 +612,11 @@ k_mlp_fused(FusedArgs g) {
       float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
       for (int o = 0; o < g.nout; ++o) {
         const float d = dys[r * g.nout + o];
-        const __bf16* w = g.wlast + int64_t(o) * W + n;
-        s.x += d * float(w[0]);
-        s.y += d * float(w[1]);
-        s.z += d * float(w[2]);
-        s.w += d * float(w[3]);
+        const float4 w = *reinterpret_cast<const float4*>(g.wlast + int64_t(o) * W + n);
+        s.x += d * w.x;
+        s.y += d * w.y;
+        s.z += d * w.z;
+        s.w += d * w.w;
       }
       const float4 z = g.z[zslot(g.depth - 1, i)];
       put(r, n, s.x * dgelu(z.x), s.y * dgelu(z.y), s.z * dgelu(z.z), s.w * dgelu(z.w));
@@ -609,43 +638,35 @@ k_mlp_fused(FusedArgs g) {
 }
 
 // Operand fragments of the BF16 weights (see k_mlp_fused): element j of lane
-// l in fragment (t, c) of a matrix A is A[32 t + l % 32][16 c + 8 (l / 32) + j].
-// Layer 0 repeats its columns for the three input parts.
+// l in fragment (t, c) of a matrix A is A[32 t + l % 32][16 c + 8 (l / 32) + j];
+// layer 0's are FP32, A[32 t + l % 32][2 c + l / 32], zero past the last input.
+// The last layer is stored as FP32 rows.
 struct FragArgs {
   const __bf16* w;
-  int nin, kp, width, depth, nout;
+  int nin, kx, width, depth, nout;
   int64_t woff[kMaxLayers];
+  float *w0, *wlast;
   bf16x8 *wf, *wb;
 };
 __global__ void k_make_fragments(FragArgs g) {
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int64_t f = i >> 6;
   const int lane = int(i & 63), row = lane & 31, k8 = 8 * (lane >> 5);
   const int W = g.width;
-  const int64_t n0 = frags_first(W, g.kp), nh = frags_hidden(W);
-  const int64_t nf = n0 + (g.depth - 1) * nh + W / 16;
-  bf16x8 v;
+  const int64_t nh = frags_hidden(W), n0 = frags_first(W, g.kx), f = i >> 6;
   if (f < n0) {
-    const int t = int(f / (g.kp / 16)), c = int(f - int64_t(t) * (g.kp / 16));
-    const __bf16* w = g.w + g.woff[0] + int64_t(32 * t + row) * g.nin;
-    for (int j = 0; j < 8; ++j) {
-      const int k = 16 * c + k8 + j;
-      v[j] = k < 3 * g.nin ? w[k % g.nin] : __bf16(0.0f);
-    }
-    g.wf[i] = v;
-  } else if (f < nf - W / 16) {
-    const int l = int((f - n0) / nh) + 1;
-    const int q = int((f - n0) - (l - 1) * nh), t = q / (W / 16), c = q - t * (W / 16);
+    const int t = int(f / (g.kx / 2)), k = 2 * int(f % (g.kx / 2)) + (lane >> 5);
+    g.w0[i] = k < g.nin ? float(g.w[g.woff[0] + int64_t(32 * t + row) * g.nin + k]) : 0.0f;
+  }
+  if (f < (g.depth - 1) * nh) {
+    const int l = int(f / nh) + 1;
+    const int q = int(f - (l - 1) * nh), t = q / (W / 16), c = q - t * (W / 16);
     const __bf16* w = g.w + g.woff[l];
     g.wf[i] = *reinterpret_cast<const bf16x8*>(w + int64_t(32 * t + row) * W + 16 * c + k8);
+    bf16x8 v;
     for (int j = 0; j < 8; ++j) v[j] = w[int64_t(16 * c + k8 + j) * W + 32 * t + row];
-    g.wb[i - n0 * 64] = v;
-  } else if (f < nf) {
-    const int c = int(f - (nf - W / 16));
-    const __bf16* w = g.w + g.woff[g.depth] + int64_t(row) * W + 16 * c + k8;
-    for (int j = 0; j < 8; ++j) v[j] = row < g.nout ? w[j] : __bf16(0.0f);
-    g.wf[i] = v;
+    g.wb[i] = v;
   }
+  if (i < int64_t(g.nout) * W) g.wlast[i] = float(g.w[g.woff[g.depth] + i]);
 }
 
 // All weight and bias gradients of a minibatch: products over the rows of the
@@ -939,11 +960,13 @@ bool Mlp::fused() const {
 
 namespace {
 
+int even_cols(int nin) { return (nin + 1) / 2 * 2; }
 int split_cols(int nin) { return (3 * nin + 1 + 31) / 32 * 32; }
 
 template <int W, int R, bool TRAIN>
 void launch_fused(FusedArgs g, hipStream_t s) {
-  const size_t top = std::max(size_t(R) * Tiling<W, R>::LD * 2, size_t(R) * (g.kp + 8) * 2);
+  const size_t top = size_t(R) * Tiling<W, R>::LD * 2;  // the inputs need less
+  static_assert(Tiling<W, R>::LD * 2 >= (kFusedMaxIn + 1) * 4, "room for the inputs");
   const size_t lds = top + (TRAIN ? size_t(R) * g.nout * 4 : 0);
   g.dy_lds = int(top);
   // More than the 64 KB a kernel may use by default at 128 rows of width 256.
@@ -991,12 +1014,14 @@ FusedArgs fused_args(const Mlp& n, const float* X, int64_t M) {
   g.X = X;
   g.M = M;
   g.nin = n.nin;
+  g.kx = even_cols(n.nin);
   g.kp = split_cols(n.nin);
   g.depth = n.depth;
   g.nout = n.nout;
+  g.w0 = n.w32.p;
+  g.wlast = n.w32.p + frags_first(n.width, g.kx) * 64;
   g.wf = reinterpret_cast<const bf16x8*>(n.wfrag.p);
   g.wb = reinterpret_cast<const bf16x8*>(n.wfrag_t.p);
-  g.wlast = n.wbf.p + n.woff[n.depth];
   g.bias = n.master.p + n.nweights;
   for (int l = 0; l <= n.depth; ++l) g.boff[l] = n.boff[l];
   return g;
@@ -1006,23 +1031,27 @@ FusedArgs fused_args(const Mlp& n, const float* X, int64_t M) {
 
 void Mlp::make_fragments(hipStream_t s) {
   if (!fused()) return;
-  const int kp = split_cols(nin);
-  const int64_t nf = frags_first(width, kp) + (depth - 1) * frags_hidden(width) + width / 16;
+  const int kx = even_cols(nin);
+  const int64_t n0 = frags_first(width, kx), nh = (depth - 1) * frags_hidden(width);
   if (!wfrag.p) {
-    wfrag.alloc(nf * kFrag);
-    wfrag_t.alloc(std::max<int64_t>(1, (depth - 1) * frags_hidden(width)) * kFrag);
+    w32.alloc(n0 * 64 + int64_t(nout) * width);
+    wfrag.alloc(std::max<int64_t>(1, nh) * kFrag);
+    wfrag_t.alloc(std::max<int64_t>(1, nh) * kFrag);
   }
   FragArgs g{};
   g.w = wbf.p;
   g.nin = nin;
-  g.kp = kp;
+  g.kx = kx;
   g.width = width;
   g.depth = depth;
   g.nout = nout;
+  g.w0 = w32.p;
+  g.wlast = w32.p + n0 * 64;
   for (int l = 0; l <= depth; ++l) g.woff[l] = woff[l];
   g.wf = reinterpret_cast<bf16x8*>(wfrag.p);
   g.wb = reinterpret_cast<bf16x8*>(wfrag_t.p);
-  k_make_fragments<<<g1(nf * 64), 256, 0, s>>>(g);
+  const int64_t threads = std::max({n0 * 64, nh * 64, int64_t(nout) * width});
+  k_make_fragments<<<g1(threads), 256, 0, s>>>(g);
 }
 
 void Mlp::ensure_fused(int64_t M) {

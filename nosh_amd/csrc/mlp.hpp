@@ -24,10 +24,11 @@ struct Mlp {
   DBuf<__bf16> dzb, dza;
   DBuf<float> y, dy, red;
   DBuf<double> partials, loss;
-  // Fused path: operand fragments of the weights (and of the transposed
-  // hidden ones), and one minibatch's pre-activations and row fragments
-  // (capacity fcap rows).
+  // Fused path: operand fragments of the hidden layers' weights and of their
+  // transposes, layer 0's fragments and the last layer in FP32, and one
+  // minibatch's pre-activations and row fragments (capacity fcap rows).
   DBuf<__bf16> wfrag, wfrag_t;
+  DBuf<float> w32;
   int64_t fcap = 0;
   DBuf<float> zs;
   DBuf<__bf16> hT, dzT, xT, dyT;

@@ -72,23 +72,46 @@ def test_training_reduces_loss():
     assert losses[-1] < 0.1 * losses[0]
 
 
-@pytest.mark.parametrize("width,M", [(256, 1000), (256, 70000), (128, 300), (64, 129)])
-def test_fused_inference_matches_forward(width, M):
-    """The one-kernel inference (activations in LDS, MFMA hidden layers) gives
-    forward()'s outputs: same roundings and summation order, so equal up to
-    FMA contraction differences; and it agrees with the bf16-emulating
-    oracle."""
-    net = _net(nin=9, width=width, seed=5)
+@pytest.mark.parametrize("width,depth,nin,M", [
+    (256, 4, 9, 1000), (256, 2, 8, 16321), (256, 2, 9, 32641), (128, 3, 1, 300),
+    (128, 2, 32, 16384), (128, 2, 5, 32768), (64, 2, 9, 129), (64, 1, 31, 20000),
+    (64, 4, 7, 32641)])
+def test_fused_inference_matches_forward(width, depth, nin, M):
+    """The one-kernel network gives the layer-by-layer path's values bit for
+    bit (the same roundings in the same order of summation), at every number
+    of rows a workgroup takes. The layer-by-layer path is that of a network
+    with more than 32 inputs: here the same network with 64 inputs of which
+    those past the first n_in are zero, as are their weights, so that they add
+    nothing. The two sum the gradients in orders of their own: their FP32 sums
+    of some 500 rows at a time keep 1e-5 of sum |terms|, which is up to
+    sqrt(M) = 180 times the gradient for targets without structure."""
+    net = _net(nin=nin, width=width, depth=depth, seed=5)
+    wide = _net(nin=64, width=width, depth=depth, seed=6)
     rng = np.random.default_rng(7)
-    X = rng.normal(0, 1, (M, 9)).astype(np.float32)
-    y_f = net.forward(X)
-    y_i = net.infer(X)
-    d = np.abs(y_i - y_f).max() / max(np.abs(y_f).max(), 1e-30)
-    print("fused vs layered max rel diff", d)
-    assert d < 1e-5
+    p = net.get_params()
+    p[net.nweights:] = rng.uniform(-0.2, 0.2, net.nparams - net.nweights)
+    net.set_params(p)
+
+    def widen(v):
+        first = np.zeros((width, 64), np.float32)
+        first[:, :nin] = v[:width * nin].reshape(width, nin)
+        return np.concatenate([first.ravel(), v[width * nin:]])
+
+    wide.set_params(widen(p))
+    X = rng.normal(0, 1, (M, nin)).astype(np.float32)
+    Xw = np.concatenate([X, np.zeros((M, 64 - nin), np.float32)], axis=1)
+    T = rng.normal(0, 1, (M, 2)).astype(np.float32)
+    y = wide.forward(Xw)
+    np.testing.assert_array_equal(wide.infer(Xw), y)
+    np.testing.assert_array_equal(net.forward(X), y)
+    np.testing.assert_array_equal(net.infer(X), y)
+    loss, g = net.gradients(X, T)
+    loss_w, g_w = wide.gradients(Xw, T)
+    assert abs(loss - loss_w) <= 1e-12 * loss_w  # the same squares, summed in FP64
+    assert np.linalg.norm(widen(g) - g_w) <= 2e-3 * np.linalg.norm(g_w)
     if M <= 1000:
-        y_bf, _, _ = MO.forward(net.get_params(), X, net.dims, bf=True)
-        assert np.linalg.norm(y_i - y_bf) / np.linalg.norm(y_bf) < 5e-3
+        y_bf, _, _ = MO.forward(p, X, net.dims, bf=True)
+        assert np.linalg.norm(y - y_bf) / np.linalg.norm(y_bf) < 5e-3
 
 
 def test_first_adam_step_closed_form():
