@@ -52,30 +52,46 @@ __device__ __forceinline__ int32_t ld_uniform(const int32_t* p) {
 // 3321 / 3878 us in FP32). Columns and positions are ordinary loads: as
 // non-temporal ones they miss the Infinity Cache when the next product reads
 // them again (96^3: 5219 us). Eight slots at a time instead of four: 6126 us.
-template <int P>
+//
+// The slice's slot ranges come with the row, before anything that the kernel
+// decides by a load (a solver's `done` flag): both loads are then under way
+// together. FP64: the range of the wave's half; FP32: those of both halves
+// (see sell_ordered).
+template <class T, int P>
 struct RowBlock {
   static constexpr int kSlices = 4 / P;  // per workgroup
   int64_t row;
   int part;    // of the slice, wave-uniform
   bool owner;  // this thread owns `row`
-  __device__ __forceinline__ RowBlock(int64_t n) {
+  int32_t beg[sizeof(T) == 4 ? 2 : 1], end[sizeof(T) == 4 ? 2 : 1];
+  __device__ __forceinline__ RowBlock(int64_t n, const SellView& S) : beg{}, end{} {
     const int w = uniform(int(threadIdx.x >> 6));
+    const int64_t slice = xcd_block(true) * kSlices + w / P;
     part = w % P;
-    row = (xcd_block(true) * kSlices + w / P) * kSliceH + (threadIdx.x & 63);
+    row = slice * kSliceH + (threadIdx.x & 63);
     owner = row < n && part == 0;
+    if (slice * kSliceH < n) {
+      const int32_t s = uniform(int32_t(slice));
+      if constexpr (sizeof(T) == 4) {
+        beg[0] = ld_uniform(S.uptr + s), end[0] = ld_uniform(S.uptr + s + 1);
+        beg[1] = ld_uniform(S.lptr + s), end[1] = ld_uniform(S.lptr + s + 1);
+      } else {
+        const int32_t* p = part < P / 2 ? S.uptr : S.lptr;
+        beg[0] = ld_uniform(p + s), end[0] = ld_uniform(p + s + 1);
+      }
+    }
   }
 };
 
 template <class T, bool OFF16, int P>
-__device__ __forceinline__ V2<T> sell_part(int64_t row, int part, const SellView& S,
+__device__ __forceinline__ V2<T> sell_part(const RowBlock<T, P>& rb, const SellView& S,
                                            const V2<T>* __restrict__ val,
                                            const V2<T>* __restrict__ x) {
   constexpr int H = P / 2;  // waves per half
-  const int32_t s = uniform(int32_t(row >> 6));
-  const int32_t first = kSliceH * (part % H) + int32_t(row & 63), r32 = int32_t(row);
+  const int32_t r32 = int32_t(rb.row), b = rb.beg[0], e = rb.end[0];
+  const int32_t first = kSliceH * (rb.part % H) + (r32 & 63);
   T ar = T(0), ai = T(0);
-  if (part < H) {
-    const int32_t b = uniform(S.uptr[s]), e = uniform(S.uptr[s + 1]);
+  if (rb.part < H) {
 #pragma unroll 4
     for (int32_t j = b + first; j < e; j += H * kSliceH) {
       const int32_t c = OFF16 ? r32 + int32_t(S.uoff[j]) : S.ucol[j];
@@ -85,7 +101,6 @@ __device__ __forceinline__ V2<T> sell_part(int64_t row, int part, const SellView
       ai += v.x * xv.y + v.y * xv.x;
     }
   } else {
-    const int32_t b = uniform(S.lptr[s]), e = uniform(S.lptr[s + 1]);
 #pragma unroll 4
     for (int32_t j = b + first; j < e; j += H * kSliceH) {
       const int32_t c = OFF16 ? r32 + int32_t(S.loff[j]) : S.lcol[j];
@@ -133,19 +148,17 @@ template <int P>
 constexpr int kTerms = P == 4 ? 8 : 16;
 
 template <bool OFF16, int P>
-__device__ __forceinline__ float2 sell_ordered(const RowBlock<P>& rb, int64_t n, const SellView& S,
-                                               const float2* __restrict__ val,
+__device__ __forceinline__ float2 sell_ordered(const RowBlock<float, P>& rb, int64_t n,
+                                               const SellView& S, const float2* __restrict__ val,
                                                const float2* __restrict__ x,
                                                float2 (&mine)[P - 1][kTerms<P>][kSliceH]) {
   const int lane = int(threadIdx.x & 63);
-  const int32_t s = uniform(int32_t(rb.row >> 6)), r32 = int32_t(rb.row);
+  const int32_t r32 = int32_t(rb.row);
   float2 acc = make_float2(0.f, 0.f);
   // Slots of part q: [from[q], to[q]) of its half.
-  int32_t b[2] = {0, 0}, from[P] = {}, to[P] = {};
+  int32_t from[P] = {}, to[P] = {};
   if (rb.row < n) {
-    b[0] = uniform(S.uptr[s]), b[1] = uniform(S.lptr[s]);
-    const int32_t len[2] = {(uniform(S.uptr[s + 1]) - b[0]) / kSliceH,
-                            (uniform(S.lptr[s + 1]) - b[1]) / kSliceH};
+    const int32_t len[2] = {(rb.end[0] - rb.beg[0]) / kSliceH, (rb.end[1] - rb.beg[1]) / kSliceH};
 #pragma unroll
     for (int q = 0; q < P; ++q) {
       const int32_t l = len[q / (P / 2)], cut = P == 4 ? (l + 1) / 2 : l;
@@ -156,7 +169,7 @@ __device__ __forceinline__ float2 sell_ordered(const RowBlock<P>& rb, int64_t n,
     for (int q = 0; q < P; ++q) {
       if (rb.part != q) continue;
       const bool up = q < P / 2;
-      const int32_t at = b[up ? 0 : 1] + lane;
+      const int32_t at = rb.beg[up ? 0 : 1] + lane;
       if (q == 0) {
 #pragma unroll 4
         for (int32_t k = from[q]; k < to[q]; ++k) {
@@ -178,7 +191,7 @@ __device__ __forceinline__ float2 sell_ordered(const RowBlock<P>& rb, int64_t n,
 #pragma unroll
     for (int q = 1; q < P; ++q) {
       const bool up = q < P / 2;
-      const int32_t at = b[up ? 0 : 1] + lane, cnt = min(to[q] - from[q], kTerms<P>);
+      const int32_t at = rb.beg[up ? 0 : 1] + lane, cnt = min(to[q] - from[q], kTerms<P>);
 #pragma unroll 4
       for (int32_t k = 0; k < cnt; ++k) {
         const float2 t = mine[q - 1][k][lane];
@@ -202,11 +215,11 @@ __device__ __forceinline__ float2 sell_ordered(const RowBlock<P>& rb, int64_t n,
 // instead of 4), else as 32-bit indices. Every thread of the workgroup calls
 // it (there is a barrier).
 template <class T, int P>
-__device__ __forceinline__ V2<T> row_product(const RowBlock<P>& rb, int64_t n, const SellView& S,
-                                             const V2<T>* __restrict__ val,
+__device__ __forceinline__ V2<T> row_product(const RowBlock<T, P>& rb, int64_t n,
+                                             const SellView& S, const V2<T>* __restrict__ val,
                                              const V2<T>* __restrict__ x) {
   if constexpr (sizeof(T) == 4) {
-    __shared__ float2 terms[RowBlock<P>::kSlices][P - 1][kTerms<P>][kSliceH];
+    __shared__ float2 terms[RowBlock<T, P>::kSlices][P - 1][kTerms<P>][kSliceH];
     auto& mine = terms[uniform(int(threadIdx.x >> 6)) / P];
     return S.uoff ? sell_ordered<true, P>(rb, n, S, val, x, mine)
                   : sell_ordered<false, P>(rb, n, S, val, x, mine);
@@ -216,8 +229,7 @@ __device__ __forceinline__ V2<T> row_product(const RowBlock<P>& rb, int64_t n, c
     V2<T> acc;
     acc.x = acc.y = T(0);
     if (rb.row < n)
-      acc = S.uoff ? sell_part<T, true, P>(rb.row, rb.part, S, val, x)
-                   : sell_part<T, false, P>(rb.row, rb.part, S, val, x);
+      acc = S.uoff ? sell_part<T, true, P>(rb, S, val, x) : sell_part<T, false, P>(rb, S, val, x);
     if (rb.part > 0) sums[w][lane] = acc;
     __syncthreads();
     if (rb.part == 0) {
@@ -256,13 +268,13 @@ __device__ __forceinline__ double wave_max(double v) {
 
 // Sum of v over each slice's rows (lanes of its owning wave; v = 0 where no row
 // is owned) to partials[slice].
-template <int P>
-__device__ __forceinline__ void slice_partials(const RowBlock<P>& rb, double v,
+template <class T, int P>
+__device__ __forceinline__ void slice_partials(const RowBlock<T, P>& rb, double v,
                                                double* __restrict__ partials) {
   if (rb.part != 0) return;
   v = wave_sum(v);
   if ((threadIdx.x & 63) == 0)
-    partials[blockIdx.x * RowBlock<P>::kSlices + (threadIdx.x >> 6) / P] = v;
+    partials[blockIdx.x * RowBlock<T, P>::kSlices + (threadIdx.x >> 6) / P] = v;
 }
 
 // Block-wide sums of NV values; the totals end up in every lane of wave 0.

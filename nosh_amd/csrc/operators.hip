@@ -136,7 +136,7 @@ __global__ __launch_bounds__(kBlock) void k_keo_apply(
     int64_t n, SellView S,
     const double2* __restrict__ val, const double* __restrict__ diag,
     const double2* __restrict__ x, double2* __restrict__ y, const int32_t* __restrict__ perm) {
-  const RowBlock<P> rb(n);
+  const RowBlock<double, P> rb(n, S);
   const int64_t row = rb.row;
   const int64_t out = perm && rb.owner ? perm[row] : row;
   const double2 acc = row_product<double, P>(rb, n, S, val, x);
@@ -154,7 +154,7 @@ __global__ __launch_bounds__(kBlock) void k_compute_f(
     const double* __restrict__ ct, const double* __restrict__ V, double g,
     const double2* __restrict__ x, double2* __restrict__ f, double* __restrict__ partials,
     const int32_t* __restrict__ perm) {
-  const RowBlock<P> rb(n);
+  const RowBlock<double, P> rb(n, S);
   const int64_t row = rb.row;
   const int64_t out = perm && rb.owner ? perm[row] : row;
   double s2 = 0.0;
@@ -167,7 +167,7 @@ __global__ __launch_bounds__(kBlock) void k_compute_f(
     f[out] = r;
     s2 = r.x * r.x + r.y * r.y;
   }
-  if (partials) slice_partials<P>(rb, s2, partials);
+  if (partials) slice_partials(rb, s2, partials);
 }
 
 __global__ __launch_bounds__(kFinThreads) void k_finalize_store(
@@ -183,7 +183,7 @@ __global__ __launch_bounds__(kBlock) void k_dfdp(
     const double2* __restrict__ dval, const double* __restrict__ ct, int is_g, double dvdp,
     const double* __restrict__ dvdp_vec, const double2* __restrict__ x, double2* __restrict__ y,
     const int32_t* __restrict__ perm) {
-  const RowBlock<P> rb(n);
+  const RowBlock<double, P> rb(n, S);
   const int64_t row = rb.row;
   const int64_t out = perm && rb.owner ? perm[row] : row;
   const double2 acc = row_product<double, P>(rb, n, S, dval, x);
@@ -253,7 +253,7 @@ __global__ __launch_bounds__(kBlock) void k_block_apply(
     int64_t n, SellView S,
     const V2<T>* __restrict__ val, const T* __restrict__ blk, const V2<T>* __restrict__ x,
     V2<T>* __restrict__ y, const int32_t* __restrict__ perm) {
-  const RowBlock<P> rb(n);
+  const RowBlock<T, P> rb(n, S);
   const int64_t row = rb.row;
   const int64_t out = perm && rb.owner ? perm[row] : row;
   const V2<T> acc = row_product<T, P>(rb, n, S, val, x);

@@ -20,9 +20,10 @@
 // (kFoldMax), else by a one-block kernel in between. The Givens state is then
 // written by A's first block to the other of two records, since the other
 // blocks still read the old one. The host only polls the `done` flag every
-// few iterations, so iterations issued after convergence write nothing; it
-// counts the iterations it issues, which fixes every buffer rotation (r1/r2,
-// w) until then.
+// few iterations, so iterations issued after convergence leave before their
+// row products (seven of them at 96^3: 0.17 ms, where working through the
+// products without storing them took 1.1); it counts the iterations it issues,
+// which fixes every buffer rotation (r1/r2, w) until then.
 // Vectors are FP64 or FP32 (template T); inner products, norms, recurrence
 // scalars and the solution accumulator are always FP64.
 
@@ -92,8 +93,9 @@ __global__ __launch_bounds__(kBlock) void k_cheb_first(ChebArgs<T> a, int mode, 
   const int64_t row = int64_t(blockIdx.x) * kBlock + threadIdx.x;
   double alfa = 0.0;
   if (mode == 2) {
-    alfa = a.fold ? block_total(thread_sum(a.pa, a.na)) : S->alfa;
+    alfa = a.fold ? thread_sum(a.pa, a.na) : S->alfa;
     if (S->done) return;
+    if (a.fold) alfa = block_total(alfa);
     if (a.fold && blockIdx.x == 0 && threadIdx.x == 0) {
       S->alfa = alfa;
       S->pending = 0;
@@ -154,38 +156,32 @@ template <class T, int P>
 __global__ __launch_bounds__(kBlock) void k_cheb_step(ChebArgs<T> a, int mode, int j,
                                                      const V2<T>* __restrict__ zin,
                                                      V2<T>* __restrict__ zout) {
-  const MinresScalars* S = a.S;
-  // Read here, used after the row product: one load less in front of it (a
-  // no-op launch then costs as much as a real one; see minres_solve's poll).
-  const int done = mode != 0 ? S->done : 0;
-  const RowBlock<P> rb(a.n);
+  const MinresScalars* S = a.S;  // never null, if of no use in mode 0
+  const RowBlock<T, P> rb(a.n, a.sv);
+  if (S->done && mode != 0) return;
   const int64_t row = rb.row;
   V2<T> zi{}, rv{}, d{};
   T b0 = T(1), b1 = T(1), b2 = T(0);
   if (rb.owner) {
     zi = zin[row];
     rv = a.r[row];
-    d = zi;
-    if (j > 1) {
-      if constexpr (sizeof(T) == 4) {
-        d = a.D[row];
-      } else {
-        const V2<T> zpp = zout[row];
-        d.x -= zpp.x;
-        d.y -= zpp.y;
-      }
-    }
+    if (j > 1) d = sizeof(T) == 4 ? a.D[row] : zout[row];
     b0 = a.pblk[row], b1 = a.pblk[a.n + row], b2 = a.pblk[2 * a.n + row];
   }
   const T c1 = T(a.coef[2 * j - 1]), c2 = T(a.coef[2 * j]);
   const V2<T> acc = row_product<T, P>(rb, a.n, a.sv, a.pval, zin);
-  if (done) return;
   double s2 = 0.0;
   if (rb.owner) {
     const T res0 = rv.x - (acc.x + b0 * zi.x + b2 * zi.y);
     const T res1 = rv.y - (acc.y + b2 * zi.x + b1 * zi.y);
     T u0, u1;
     dinv<T>(b0, b1, b2, res0, res1, &u0, &u1);
+    if (j == 1) {
+      d = zi;
+    } else if (sizeof(T) == 8) {
+      d.x = zi.x - d.x;
+      d.y = zi.y - d.y;
+    }
     d.x = c1 * d.x + c2 * u0;
     d.y = c1 * d.y + c2 * u1;
     V2<T> z;
@@ -196,7 +192,7 @@ __global__ __launch_bounds__(kBlock) void k_cheb_step(ChebArgs<T> a, int mode, i
     s2 = double(rv.x) * double(z.x) + double(rv.y) * double(z.y);
   }
   if (mode == 0 || j != a.iters - 1) return;
-  slice_partials<P>(rb, s2, a.pb);
+  slice_partials(rb, s2, a.pb);
 }
 
 // beta^2 = sum of the partials of <r, z>: MINRES initialisation (mode 1) or
@@ -264,14 +260,18 @@ __global__ __launch_bounds__(kBlock) void k_minres_a(MinresArgs<T> a, int it, co
                                                      const double* pb, int nb, double* pa) {
   __shared__ MinresScalars S;
   double sum = nb > 0 ? thread_sum(pb, nb) : 0.0;
-  const RowBlock<P> rb(a.n);
+  const RowBlock<T, P> rb(a.n, a.sv);
+  if (Sin->done) {
+    if (nb > 0 && blockIdx.x == 0 && threadIdx.x == 0) *Sout = *Sin;
+    return;
+  }
   const int64_t row = rb.row;
   const V2<T> acc = row_product<T, P>(rb, a.n, a.sv, a.jval, a.y);
   if (nb > 0) sum = block_total(sum);
   if (threadIdx.x == 0) {
     S = *Sin;
     if (nb > 0) {
-      if (!S.done) givens_update(&S, sum);
+      givens_update(&S, sum);
       if (blockIdx.x == 0) *Sout = S;
     }
   }
@@ -300,7 +300,7 @@ __global__ __launch_bounds__(kBlock) void k_minres_a(MinresArgs<T> a, int it, co
     a.u[row] = uu;
     s = double(vn.x) * double(uu.x) + double(vn.y) * double(uu.y);
   }
-  slice_partials<P>(rb, s, pa);
+  slice_partials(rb, s, pa);
 }
 
 // Applies the last pending w/x update, then psi += x when psi != nullptr.

@@ -337,3 +337,41 @@ def test_fp32_products_of_long_rows(ring, reorder):
             step.append(psi - psi0)
         assert np.linalg.norm(step[0]) > 1e-3
         assert np.linalg.norm(step[1] - step[0]) <= 1e-4 * np.linalg.norm(step[0])
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_iterations_after_convergence_do_no_work(precision):
+    """MINRES is issued eight iterations at a time and stops inside them: the
+    rest must leave before their row products. A solve that stops in its first
+    iteration, with seven issued after it, against one of a single iteration
+    and one of eight: 7 x 9 empty launches of some 5 us beside seven iterations of
+    0.2 - 0.3 ms at 96^3 (they must cost less than half)."""
+    import time
+
+    import torch
+    import nosh_amd as nosh
+    coords, cells = mg.kuhn_cube(96)
+    gm = nosh.Mesh(coords, cells)
+    mvp = nosh.VectorFieldExplicitValues(gm, mg.magnetic_potential(coords), 0.05)
+    model = nosh.Nls(gm, mvp, nosh.ScalarFieldConstant(gm, -1.0), 1.0,
+                     nosh.ScalarFieldConstant(gm, 1.0))
+    start = torch.from_numpy(mg.random_state(coords.shape[0], 3)).cuda()
+    psi = torch.empty_like(start)
+
+    def solve(rtol, iters):
+        best = 1e9
+        for _ in range(6):
+            psi.copy_(start)
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            st = nosh.newton_solve_device(model, psi.data_ptr(), {"g": 1.0, "mu": 0.05}, tol=0.0,
+                                          max_iters=1, forcing=0, minres_rtol=rtol,
+                                          minres_max_iters=iters, cheb_iters=6, cheb_ratio=300.0,
+                                          precision=precision)
+            best = min(best, time.perf_counter() - t)
+        return best, st["minres_iters_total"]
+
+    (one, n1), (stopped, ns), (eight, n8) = solve(1e9, 1), solve(1e9, 8), solve(0.0, 8)
+    assert (n1, ns, n8) == (1, 1, 8)
+    print("one, stopped, eight iterations: %.3f %.3f %.3f ms" % (1e3 * one, 1e3 * stopped, 1e3 * eight))
+    assert stopped - one < 0.5 * (eight - one)
