@@ -66,15 +66,21 @@ double gibbs_dev(nosh_nls_s* nls, ContWork& w, const double* psi_int, hipStream_
 // (the field's gauge makes dK/dmu psi vanish at mu = 0) that rounding made the
 // singular system inconsistent: MINRES ran to its iteration limit and the
 // tangent grew along i psi by whatever its last bits were.
+//
+// Every workgroup of the projection adds the partial sums itself, which saves a
+// launch. At most kPhaseBlocks of them (four a CU, 2 loads a thread of each)
+// walk the rows in strides: with one per 256 rows those sums were read as many
+// times as there were of them, 24 GB at 10^7 rows beside 0.3 GB of vectors.
+constexpr unsigned kPhaseBlocks = 1024;
+
 __global__ __launch_bounds__(256) void k_phase_dots(int64_t n, const double2* __restrict__ psi,
                                                     const double2* __restrict__ r,
                                                     double* __restrict__ partials) {
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   double v[2] = {0.0, 0.0};
-  if (i < n) {
+  for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < n; i += int64_t(gridDim.x) * 256) {
     const double2 p = psi[i], q = r[i];
-    v[0] = p.x * q.y - p.y * q.x;
-    v[1] = p.x * p.x + p.y * p.y;
+    v[0] += p.x * q.y - p.y * q.x;
+    v[1] += p.x * p.x + p.y * p.y;
   }
   block_partials<2>(v, partials);
 }
@@ -87,13 +93,13 @@ __global__ __launch_bounds__(256) void k_phase_project(int64_t n, const double2*
   finalize_sum<2>(v, partials, int(gridDim.x));
   if (threadIdx.x == 0) c = v[1] > 0.0 ? v[0] / v[1] : 0.0;
   __syncthreads();
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double2 p = psi[i];
-  double2 q = r[i];
-  q.x += c * p.y;
-  q.y -= c * p.x;
-  r[i] = q;
+  for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < n; i += int64_t(gridDim.x) * 256) {
+    const double2 p = psi[i];
+    double2 q = r[i];
+    q.x += c * p.y;
+    q.y -= c * p.x;
+    r[i] = q;
+  }
 }
 
 // Tangent t with J(psi) t = -dF/dp(psi); returns MINRES iterations.
@@ -110,7 +116,7 @@ int tangent(nosh_nls_s* nls, ContWork& w, const std::string& param, double* psi_
   // dF/dp: dK/dp psi + (p == "g" ? ct |psi|^2 psi : ct dV/dp psi).
   launch_dfdp(m, w.dk->kv, nls->ct.p, psi_int, param == "g", nls->V->sf.dvdp_constant(param),
               nls->V->sf.dvdp_values(param, s), w.rhs.p, s);
-  const unsigned gn = grid_for(n, 256);
+  const unsigned gn = std::min(grid_for(n, 256), kPhaseBlocks);
   if (w.partials.n < 2 * size_t(gn)) w.partials.alloc(2 * size_t(gn));
   const auto psi2 = reinterpret_cast<const double2*>(psi_int);
   const auto rhs2 = reinterpret_cast<double2*>(w.rhs.p);

@@ -145,3 +145,25 @@ def test_surrogate_continuation_on_disk():
                                  **kw)
     assert sum(r["newton_iters"] for r in rec[P + 1:]) <= sum(r["newton_iters"]
                                                              for r in rec_t[P + 1:])
+
+
+def test_tangent_on_more_rows_than_the_projection_has_threads():
+    """At mu = 0 dF/dmu is rounding noise and J is singular along i psi: the
+    tangent's solve ends only because every row of its right-hand side is
+    projected. 521^2 = 271,441 rows, 9,297 more than the projection's 1024
+    workgroups of 256 threads hold one each."""
+    import nosh_amd as nosh
+    coords, cells = mg.square_tri(520)
+    mesh, model = _model(coords, cells)
+    psi0 = np.ones(coords.shape[0], dtype=np.complex128).view(np.float64)
+    used, last = [], []
+    for predictor in (0, 1):
+        psi, rec = nosh.continuation(model, psi0, {"g": 1.0, "mu": 0.0}, "mu", 0.0, 0.01, 1,
+                                     predictor=predictor, tol=1e-10, cheb_iters=6,
+                                     cheb_ratio=300.0, minres_max_iters=6000)
+        assert all(r["converged"] for r in rec)
+        used.append(rec[-1]["minres_iters"])
+        last.append(rec[-1])
+    print("MINRES iterations without and with the tangent", used)
+    assert used[1] < used[0] + 6000
+    assert last[1]["newton_iters"] <= last[0]["newton_iters"]
