@@ -26,7 +26,6 @@
 
 #include <algorithm>
 #include <numeric>
-#include <queue>
 
 #include "internal.hpp"
 
@@ -93,20 +92,17 @@ __global__ void k_mark_first(const int32_t* __restrict__ head, const uint32_t* _
   if (head[i]) isfirst[spos[i]] = 1;
 }
 
-// For every run head: the edge id of its first slot, the endpoints, the
-// start of the run in sorted order.
+// For every run head: the edge id of its first slot, and the endpoints.
 __global__ void k_run_edges(const int32_t* __restrict__ head, const int32_t* __restrict__ runid,
                             const uint32_t* __restrict__ spos, const uint64_t* __restrict__ skeys,
                             const int32_t* __restrict__ eid_at_pos, int64_t N, uint64_t n,
-                            int32_t* __restrict__ run_edge, int32_t* __restrict__ edges,
-                            int32_t* __restrict__ edge_start) {
+                            int32_t* __restrict__ run_edge, int32_t* __restrict__ edges) {
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= N || !head[i]) return;
   const int32_t e = eid_at_pos[spos[i]];
   run_edge[runid[i]] = e;
   edges[2 * e] = int32_t(skeys[i] / n);
   edges[2 * e + 1] = int32_t(skeys[i] % n);
-  edge_start[e] = int32_t(i);
 }
 
 __global__ void k_cell_edges_canon(const int32_t* __restrict__ runid,
@@ -690,7 +686,7 @@ std::unique_ptr<MeshCache> build_mesh_cache(const double* coords, int64_t n, con
   const int64_t N = T * ne, Nv = T * nv;
   const int64_t ns = (n + kSliceH - 1) / kSliceH;
   m->nslices = ns;
-  m->slabs.reserve(3);
+  m->slabs.reserve(4);
   {
     Slab& k = m->slabs.emplace_back(slab_bytes<double>(3 * n) + 2 * slab_bytes<double>(n) +
                                     slab_bytes<int32_t>(Nv) + slab_bytes<int32_t>(N) +
@@ -709,11 +705,11 @@ std::unique_ptr<MeshCache> build_mesh_cache(const double* coords, int64_t n, con
   m->coords.upload(coords, 3 * n, s);
   m->cells.upload(cells, Nv, s);
 
-  // Scratch of the whole build in one allocation, the arrays that stay in three:
+  // Scratch of the whole build in one allocation, the arrays that stay in four:
   // some seventy of them, each with its release and the wait that brings,
   // took 10 of the 19 ms of a mesh of 117 k vertices and 640 k tetrahedra
-  // (now 8), and destroying it 3.3 ms (0.4). The scratch's peak is the first sort (24 N bytes of keys
-  // and positions in and out, and as much again for hipCUB).
+  // (now 8), and destroying it 3.3 ms (0.4). The scratch's peak is the first sort
+  // (24 N bytes of keys and positions in and out, and as much again for hipCUB).
   Slab tmp(size_t(48 * N + 64 * n) + (1 << 20));
   const unsigned gN = grid_for(N, kBlock);
   const int kbits = bits_for(uint64_t(n) * uint64_t(n));
@@ -749,10 +745,9 @@ std::unique_ptr<MeshCache> build_mesh_cache(const double* coords, int64_t n, con
       k.take(m->covol, E);
     }
     int32_t* run_edge = tmp.take<int32_t>(E);
-    int32_t* edge_start = tmp.take<int32_t>(E);
     int32_t* run_start = tmp.take<int32_t>(E + 1);
     k_run_edges<<<gN, kBlock, 0, s>>>(head, runid, spos, skeys, eid, N, uint64_t(n), run_edge,
-                                      m->edges.p, edge_start);
+                                      m->edges.p);
     k_run_start<<<gN, kBlock, 0, s>>>(head, runid, N, run_start);
     k_fill_i32<<<1, 1, 0, s>>>(run_start + E, 1, int32_t(N));
     // 3. Cell -> edges, ascending.
@@ -860,16 +855,16 @@ std::unique_ptr<MeshCache> build_mesh_cache(const double* coords, int64_t n, con
                   nl = std::max<int64_t>(tl, 1);
     {
       Slab& k = m->slabs.emplace_back(2 * slab_bytes<int32_t>(np) + 2 * slab_bytes<int32_t>(nu) +
-                                      2 * slab_bytes<int32_t>(nl) + slab_bytes<int16_t>(nu) +
-                                      slab_bytes<int16_t>(nl));
+                                      2 * slab_bytes<int32_t>(nl));
       k.take(m->scol, np);
       k.take(m->sedge, np);
       k.take(m->ucol, nu);
       k.take(m->uedge, nu);
       k.take(m->lcol, nl);
       k.take(m->lpos, nl);
-      k.take(m->uoff, nu);
-      k.take(m->loff, nl);
+      Slab& o = m->slabs.emplace_back(slab_bytes<int16_t>(nu) + slab_bytes<int16_t>(nl));
+      o.take(m->uoff, nu);
+      o.take(m->loff, nl);
     }
     k_sell_pad<<<unsigned(ns), kBlock, 0, s>>>(m->slice_ptr.p, ns, n, m->scol.p, m->sedge.p);
     k_sell_fill<<<grid_for(ND, kBlock), kBlock, 0, s>>>(c.rows, c.cols, c.codes, c.start,
@@ -886,13 +881,14 @@ std::unique_ptr<MeshCache> build_mesh_cache(const double* coords, int64_t n, con
         m->lcol.p, lcode, upos);
     k_split_lpos<<<grid_for(tl, kBlock), kBlock, 0, s>>>(lcode, upos, tl, m->lpos.p);
     // 16-bit column offsets when the bandwidth allows (2 bytes less per slot
-    // for every kernel that reads the split layout).
+    // for every kernel that reads the split layout), else their memory is given back.
     k_fill_i32<<<1, 1, 0, s>>>(wide, 1, 0);
     k_col_off16<<<unsigned(ns), kBlock, 0, s>>>(m->uptr.p, m->ucol.p, ns, n, m->uoff.p, wide);
     k_col_off16<<<unsigned(ns), kBlock, 0, s>>>(m->lptr.p, m->lcol.p, ns, n, m->loff.p, wide);
     if (read_i32(wide, s)) {
       m->uoff.release();
       m->loff.release();
+      m->slabs.pop_back();
     }
   }
   return m;

@@ -339,6 +339,38 @@ def test_fp32_products_of_long_rows(ring, reorder):
         assert np.linalg.norm(step[1] - step[0]) <= 1e-4 * np.linalg.norm(step[0])
 
 
+def test_wide_mesh_does_not_hold_column_offsets():
+    """A mesh whose columns do not fit 16 bits gives the memory of their offsets
+    back: it holds its arrays (24 B a vertex of coordinates and 24 B of control
+    volumes and orders, vertices and edges of the cells, 24 B an edge, two
+    numbers a slot of the full structure and of each half of the split one) and
+    no more than the 2 MB pages of five allocations (less what the runtime still
+    had of earlier ones), where the offsets of an 80^3 cube without an order
+    would be another 20 MB."""
+    import torch
+    import nosh_amd as nosh
+    c0, t0 = mg.kuhn_cube(80)
+    n = c0.shape[0]
+    perm = np.random.default_rng(8).permutation(n)
+    inv = np.empty(n, dtype=np.int32)
+    inv[perm] = np.arange(n)
+    coords, cells = c0[perm], inv[t0]
+    small = nosh.Mesh(*mg.kuhn_cube(4))  # what the first mesh of a process allocates
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    gm = nosh.Mesh(coords, cells, reorder=False)
+    held = before - torch.cuda.mem_get_info()[0]
+    lay = gm.layout()
+    assert lay["column_bytes"] == 4
+    slots = lay["nnz_pad"] + lay["nnz_upper"] + lay["nnz_lower"]
+    arrays = 48 * n + 4 * 10 * len(cells) + 24 * gm.num_edges + 8 * slots
+    offsets = 2 * (lay["nnz_upper"] + lay["nnz_lower"])
+    print("held %.1f MB, arrays %.1f, offsets %.1f" % (held / 1e6, arrays / 1e6, offsets / 1e6))
+    assert offsets > 20e6
+    assert held <= arrays + 5 * 2 ** 21
+    del small
+
+
 @pytest.mark.parametrize("precision", [0, 1])
 def test_iterations_after_convergence_do_no_work(precision):
     """MINRES is issued eight iterations at a time and stops inside them: the
