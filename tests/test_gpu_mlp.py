@@ -146,12 +146,28 @@ def test_first_adam_step_closed_form():
 
 @pytest.mark.parametrize("nin,width,depth,nout,M", [
     (1, 64, 1, 1, 1), (7, 64, 2, 2, 127), (10, 128, 3, 2, 128), (11, 128, 2, 3, 129),
-    (21, 256, 2, 11, 257), (32, 256, 3, 16, 500), (9, 256, 4, 2, 40000)])
+    (21, 256, 2, 11, 257), (32, 256, 3, 16, 500), (9, 256, 4, 2, 40000), (5, 64, 2, 16, 63),
+    (6, 256, 1, 3, 33), (7, 256, 2, 2, 16321), (7, 128, 2, 2, 16385), (7, 128, 2, 2, 32641),
+    (7, 64, 2, 2, 32641)])
 def test_fused_network_shapes(nin, width, depth, nout, M):
-    """The fused kernels at the edges of their tiles: rows around the 128-row
-    workgroups and the 512-row gradient splits, inputs around the 32-column
-    tiles of their three-part split (3 n_in + 1 = 31, 34, 64, 97), one hidden
-    layer, and outputs on both sides of one 32-row tile of 3 n_out."""
+    """The fused kernels at the edges of their tiles: rows around the 32-, 64-
+    and 128-row workgroups and the 512-row gradient splits, inputs around the
+    32-column tiles of their three-part split (3 n_in + 1 = 31, 34, 64, 97), one
+    hidden layer, and outputs on both sides of one 32-row tile of 3 n_out."""
+    _check_against_oracle(nin, width, depth, nout, M)
+
+
+@pytest.mark.parametrize("nin,width,depth,nout,M", [
+    (7, 192, 3, 2, 1000), (40, 64, 2, 3, 500), (33, 128, 1, 1, 65), (64, 256, 2, 16, 127),
+    (1, 320, 2, 2, 1), (9, 512, 2, 2, 1025)])
+def test_layered_network_shapes(nin, width, depth, nout, M):
+    """The layer-by-layer path of every other shape: widths without a fused
+    kernel and more than 32 inputs, rows around its 64-row tiles, its 32-row
+    reduction chunks and its 1024-row gradient splits."""
+    _check_against_oracle(nin, width, depth, nout, M)
+
+
+def _check_against_oracle(nin, width, depth, nout, M):
     net = _net(nin=nin, width=width, depth=depth, nout=nout, seed=9)
     rng = np.random.default_rng(12)
     p = net.get_params()

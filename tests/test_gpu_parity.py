@@ -271,14 +271,15 @@ def test_newton_matches_oracle(name):
     assert np.linalg.norm(d) / np.linalg.norm(psi_o) < 1e-9
 
 
-@pytest.mark.parametrize("ncell", [1, 7, 8, 299, 300])
+@pytest.mark.parametrize("ncell", [1, 7, 8, 299, 300, 511, 512])
 def test_row_products_at_the_split_sizes(ncell):
     """Four and two waves a slice: a mesh of 4 rows, slices exactly full and one
     row over (64, 81), the last mesh of the four-wave form and the first of the
     two-wave form (90,000 and 90,601 rows; an odd number of slices leaves the
-    last workgroup half empty). F, K, J and P against the oracle, and a linear
-    solve of 20 iterations, whose reductions go through both ways of adding
-    the partial sums, against the same solve's residual from J."""
+    last workgroup half empty), the last one whose partial sums the next kernel
+    adds and the first with a kernel for them in between (4096 and 4113 slices).
+    F, K, J and P against the oracle, and a linear solve of 20 iterations
+    against the same solve's residual from J."""
     import nosh_amd as nosh
     from oracle import oracle as O
     coords, cells = mg.square_tri(ncell)
@@ -298,7 +299,12 @@ def test_row_products_at_the_split_sizes(ncell):
     J.rebuild(p, psi)
     P.rebuild(p, psi)
     om.jac_rebuild(psi)
+    om.prec_rebuild(psi)
+    keo = nosh.Keo(case["gm"], t, mvp)
+    keo.set_parameters(p)
+    assert rel_err(keo.apply(phi), om.keo(phi)) < TOL
     assert rel_err(J.apply(phi), om.jac(phi)) < TOL
+    assert rel_err(P.apply_operator(phi), om.prec_op(phi)) < TOL
     b = om.f(psi)
     x, it, rr = nosh.minres_solve(J, P, b, rtol=1e-14, max_iters=20)
     assert it <= 20 and np.all(np.isfinite(x))
@@ -337,6 +343,40 @@ def test_fp32_products_of_long_rows(ring, reorder):
             step.append(psi - psi0)
         assert np.linalg.norm(step[0]) > 1e-3
         assert np.linalg.norm(step[1] - step[0]) <= 1e-4 * np.linalg.norm(step[0])
+
+
+@pytest.mark.parametrize("ring", [33, 100])
+@pytest.mark.parametrize("reorder", [True, False])
+def test_fp32_products_of_long_rows_in_large_meshes(ring, reorder):
+    """The same with two waves a slice, each with a whole half of the row and
+    room for 16 terms in LDS: two fans, one centre the first of its vertices and
+    one the last, beside a square of more than 90,000 rows. The fans' own part
+    of the update within 1e-3 of its norm: a term left out is 1 in 100."""
+    import nosh_amd as nosh
+    coords, cells = mg.square_tri(300)
+    a = 2 * np.pi * np.arange(ring) / ring
+    rim = np.stack([np.cos(a), np.sin(a), 0 * a], axis=1)
+    square = len(coords)
+    for centre in (0, ring):
+        k = np.arange(ring) + (centre == 0)
+        fan = np.stack([np.full(ring, centre), k, np.roll(k, -1)], axis=1) + len(coords)
+        cells = np.concatenate([cells, fan]).astype(np.int32)
+        coords = np.concatenate([coords, np.insert(rim, centre, 0.0, axis=0)])
+    gm = nosh.Mesh(coords, cells, reorder=reorder)
+    mvp = nosh.VectorFieldExplicitValues(gm, mg.magnetic_potential(coords), 0.2)
+    model = nosh.Nls(gm, mvp, nosh.ScalarFieldConstant(gm, -1.0), 1.3,
+                     nosh.ScalarFieldConstant(gm, 1.0))
+    psi0 = mg.random_state(len(coords), 5)
+    step = []
+    for precision in (0, 1):
+        psi, _ = nosh.newton_solve(model, psi0, {"g": 1.3, "mu": 0.2}, tol=0.0, max_iters=1,
+                                   minres_rtol=0.0, minres_max_iters=8, cheb_iters=5,
+                                   cheb_ratio=30.0, precision=precision)
+        step.append(psi - psi0)
+    for part, bound in ((slice(None), 1e-4), (slice(2 * square, None), 1e-3)):
+        norm = np.linalg.norm(step[0][part])
+        assert norm > 1e-3
+        assert np.linalg.norm(step[1][part] - step[0][part]) <= bound * norm
 
 
 def test_wide_mesh_does_not_hold_column_offsets():
