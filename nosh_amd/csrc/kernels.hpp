@@ -10,9 +10,18 @@ namespace nosh {
 template <class T>
 using V2 = typename Vec2<T>::type;
 
-// Meshes up to this many rows use P = 4, larger ones P = 2 (see RowBlock): at
-// 69 k rows (40^3) P = 4 takes 787 us where P = 2 takes 866, at 118 k 1126
-// against 1010.
+// Meshes up to this many rows use P = 4, larger ones P = 2 (see RowBlock), in
+// 2D (3 + 3 slots a row) as in 3D (7 + 7) and in FP32 as in FP64. A Newton step
+// of 16 MINRES iterations, P = 4 | 2, in us:
+//   rows                 FP64          FP32
+//   10,201  (100^2)    595 |  636    615 |  668
+//   68,921  (40^3)     772 |  862    781 |  809
+//   90,601  (300^2)    753 |  746    762 |  747
+//   91,125  (44^3)     857 |  893    839 |  830
+//   117,649 (48^3)    1085 | 1031    921 |  908
+//   160,801 (400^2)    985 |  874    961 |  822
+//   491,401 (700^2)   2331 | 2218   1923 | 1646
+//   912,673 (96^3)    5554 | 4935   3887 | 3514
 constexpr int64_t kSplitRows = 90000;
 
 // MI355X dispatches consecutive workgroups round-robin over its 8 XCDs.
@@ -41,17 +50,18 @@ __device__ __forceinline__ int32_t ld_uniform(const int32_t* p) {
 }
 
 // Row products of one workgroup of 256 threads. P waves share a 64-row slice:
-// P = 4: two take its upper slots and two its lower ones (every other slot
-// each); P = 2: one takes the upper slots, one the lower ones. The first of
-// them adds the sums through LDS and owns the slice's rows. One wave a slice
+// P = 4: two take its upper slots and two its lower ones (FP64: every other slot
+// each; FP32: the first and the second half of them); P = 2: one takes the upper
+// slots, one the lower ones. The first of them adds the sums (FP32: the terms,
+// see sell_ordered) through LDS and owns the slice's rows. One wave a slice
 // walks a chain of some twelve dependent loads (slot pointer, columns,
 // gathers, first above then below the diagonal); P waves are P times as many,
 // with a part of the chain each. A Newton step of 16 MINRES iterations (112
 // products) with one, two and four waves a slice: 20^3 cube 878 / 746 / 664 us,
-// 48^3 1310 / 1010 / 1126 us, 96^3 5997 / 5025 / 5597 us in FP64 (3994 /
-// 3321 / 3878 us in FP32). Columns and positions are ordinary loads: as
-// non-temporal ones they miss the Infinity Cache when the next product reads
-// them again (96^3: 5219 us). Eight slots at a time instead of four: 6126 us.
+// 48^3 1310 / 1010 / 1126 us, 96^3 5997 / 5025 / 5597 us in FP64. Columns and
+// positions are ordinary loads: as non-temporal ones they miss the Infinity
+// Cache when the next product reads them again (96^3: 5219 us). Eight slots at
+// a time instead of four: 6126 us.
 //
 // The slice's slot ranges come with the row, before anything that the kernel
 // decides by a load (a solver's `done` flag): both loads are then under way
@@ -144,6 +154,11 @@ __device__ __forceinline__ float2 sell_term(bool up, int32_t j, int32_t r32, con
   return t;
 }
 
+// The rows of a Kuhn cube have 7 + 7 slots, more about jittered or irregular
+// vertices. Twice as many terms (24 KB of LDS with P = 4, 32 with P = 2) leave
+// too few workgroups a CU: 16 iterations at 96^3 take 4523 us against 3512, at
+// 700^2 2123 against 1645. Half as many: 3460 and 1626, but a half row of 9
+// slots with P = 2 is then partly one wave's.
 template <int P>
 constexpr int kTerms = P == 4 ? 8 : 16;
 

@@ -315,14 +315,15 @@ __global__ void k_f32_to_bf16(const float* __restrict__ a, int64_t n, __bf16* __
 // next four k-steps' fragments are loaded while the current four multiply,
 // and the next layer's first ones before the GELU epilogue. The weights
 // are the A operand: a lane then holds four consecutive outputs of one row
-// and stores them as 8 bytes. LDS (68 KB at width 256) and registers (256)
+// and stores them as 8 bytes. LDS (68 KB at width 256) and registers (196)
 // let two workgroups share a CU, so one's GELUs run beside the other's
 // MFMAs. Before, every wave computed 32 rows x all columns with the weights
 // staged through LDS (135 KB, one workgroup a CU): 1.5 LDS reads an MFMA
 // where 1 read of 8 cycles in 32 is the limit of four waves.
 // Measured (width 256, depth 4, n_in 7): inference of 912,673 rows 2310 ->
-// 568 us (640 TFLOP/s; the GELUs alone are ~0.46 ms of vector issue), four
-// Adam steps on 16,384 rows 5.95 -> 0.66 ms (1.06 with 128 rows a workgroup).
+// 568 us (640 TFLOP/s; its 2.4e8 vector instructions of a wave are 0.5 ms of
+// issue, the GELUs 0.4 of them), four Adam steps on 16,384 rows 5.95 -> 0.66 ms
+// (1.06 with 128 rows a workgroup).
 //
 // Every value is, bit for bit, that of the layer-by-layer path: layer 0 runs on
 // the FP32 matrix instruction (32x32x2, whose sums round like the chain of
