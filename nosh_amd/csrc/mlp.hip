@@ -31,6 +31,7 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kBM = 64, kBN = 128, kBK = 32, kPad = 8;
 constexpr int kLds = kBK + kPad;  // bf16 per LDS row
@@ -328,13 +329,18 @@ __global__ void k_f32_to_bf16(const float* __restrict__ a, int64_t n, __bf16* __
 // Every value is, bit for bit, that of the layer-by-layer path: layer 0 runs on
 // the FP32 matrix instruction (32x32x2, whose sums round like the chain of
 // fmaf over the inputs, from the bias on), the hidden layers take the same
-// k-steps, and the last layer is the FP32 chain over k, a row and output per
-// lane with its weights in scalar registers (on the matrix cores 30 of 32
-// columns would be padding).
+// k-steps, and the last layer is an FP32 chain over k again, as such or (beyond
+// kChainOut outputs) on the 16x16x4 matrix instruction.
 // In the weight gradients x and dy are split into three BF16 parts of 8 bits
 // each (x = x1 + x2 + x3 exactly): exact products with the BF16 dz and h.
 constexpr int kFusedMaxIn = 32;
 constexpr int kMaxLayers = 18;
+// Most outputs that the last layer takes as chains on the vector units: a wave
+// of them costs 512 instructions, a wave of matrix tiles 64 dependent ones of 32
+// cycles whatever the outputs. 300,000 rows of width 256 and depth 4, chains |
+// tiles: 4 outputs 221 | 224 us, 8 outputs 244 | 228, 16 outputs 294 | 239; 912,673
+// rows with 2 outputs 568 | 606.
+constexpr int kChainOut = 4;
 constexpr int kFrag = 512;  // bf16 per operand fragment
 
 struct FusedArgs {
@@ -345,6 +351,7 @@ struct FusedArgs {
   const bf16x8* wf;          // forward fragments of the hidden layers
   const bf16x8* wb;          // transposed ones (training)
   const float* wlast;        // last layer, [nout][width]
+  const float* wl;           // the same as FP32 fragments
   const float* bias;
   int64_t boff[kMaxLayers];
   float* Y;  // inference
@@ -554,27 +561,54 @@ k_mlp_fused(FusedArgs g) {
     if (l + 1 < g.depth) prefetch(g.wf + l * frags_hidden(W) * 64);
     activate(l);
   }
-  // Last layer: f(row, output, y) once for each.
-  constexpr int kGroups = (kRows + 63) / 64;  // of 64 rows
+  // Last layer: f(row, output, y) once for each. Up to kChainOut outputs go a
+  // row and output per lane, weights in scalar registers, more of them through
+  // the matrix cores, 16 rows a tile.
+  constexpr int kTiles = (kRows + 63) / 64;  // of a wave, or groups of 64 rows
   auto last_layer = [&](auto f) {
-    for (int u = wave; u < kGroups * g.nout; u += 4) {
-      const int o = uniform(u / kGroups), r = (u % kGroups) * 64 + lane;
-      if (r >= kRows) continue;
+    if (g.nout <= kChainOut) {
+      for (int u = wave; u < kTiles * g.nout; u += 4) {
+        const int o = uniform(u / kTiles), r = (u % kTiles) * 64 + lane;
+        if (r >= kRows) continue;
 #if __HIP_DEVICE_COMPILE__
-      // Never written by this kernel, and the same for the whole wave.
-      const auto w = (const __attribute__((address_space(4))) float*)(g.wlast + int64_t(o) * W);
+        // Never written by this kernel, and the same for the whole wave.
+        const auto w = (const __attribute__((address_space(4))) float*)(g.wlast + int64_t(o) * W);
 #else
-      const float* w = g.wlast + int64_t(o) * W;
+        const float* w = g.wlast + int64_t(o) * W;
 #endif
-      float s = g.bias[g.boff[g.depth] + o];
+        float s = g.bias[g.boff[g.depth] + o];
 #pragma unroll 4
-      for (int k = 0; k < W; k += 8) {
-        const bf16x8 h = *reinterpret_cast<const bf16x8*>(act + r * LD + k);
+        for (int k = 0; k < W; k += 8) {
+          const bf16x8 h = *reinterpret_cast<const bf16x8*>(act + r * LD + k);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) s += float(h[e]) * w[k + e];
+          for (int e = 0; e < 8; ++e) s += float(h[e]) * w[k + e];
+        }
+        f(r, o, s);
       }
-      f(r, o, s);
+      return;
     }
+    if (wave * 16 >= kRows) return;
+    const int q = lane >> 4, r = wave * 16 + (lane & 15);
+    f32x4 out[kTiles];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float b = 4 * q + e < g.nout ? g.bias[g.boff[g.depth] + 4 * q + e] : 0.0f;
+#pragma unroll
+      for (int t = 0; t < kTiles; ++t) out[t][e] = b;
+    }
+#pragma unroll 8
+    for (int k = 0; k < W; k += 4) {
+      const float a = g.wl[k * 16 + lane];
+#pragma unroll
+      for (int t = 0; t < kTiles; ++t)
+        out[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, float(act[(r + 64 * t) * LD + k + q]),
+                                                      out[t], 0, 0, 0);
+    }
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (4 * q + e < g.nout) f(r + 64 * t, 4 * q + e, out[t][e]);
   };
   if constexpr (!TRAIN) {
     last_layer([&](int r, int o, float y) {
@@ -641,12 +675,13 @@ k_mlp_fused(FusedArgs g) {
 // Operand fragments of the BF16 weights (see k_mlp_fused): element j of lane
 // l in fragment (t, c) of a matrix A is A[32 t + l % 32][16 c + 8 (l / 32) + j];
 // layer 0's are FP32, A[32 t + l % 32][2 c + l / 32], zero past the last input.
-// The last layer is stored as FP32 rows.
+// The last layer is stored as FP32 rows and as FP32 fragments of 16 outputs and
+// 4 inputs: A[l % 16][4 c + l / 16].
 struct FragArgs {
   const __bf16* w;
   int nin, kx, width, depth, nout;
   int64_t woff[kMaxLayers];
-  float *w0, *wlast;
+  float *w0, *wlast, *wl;
   bf16x8 *wf, *wb;
 };
 __global__ void k_make_fragments(FragArgs g) {
@@ -668,6 +703,10 @@ __global__ void k_make_fragments(FragArgs g) {
     g.wb[i] = v;
   }
   if (i < int64_t(g.nout) * W) g.wlast[i] = float(g.w[g.woff[g.depth] + i]);
+  if (i < 16 * int64_t(W)) {
+    const int o = lane & 15, k = int(f) * 4 + (lane >> 4);
+    g.wl[i] = o < g.nout ? float(g.w[g.woff[g.depth] + int64_t(o) * W + k]) : 0.0f;
+  }
 }
 
 // All weight and bias gradients of a minibatch: products over the rows of the
@@ -1021,6 +1060,7 @@ FusedArgs fused_args(const Mlp& n, const float* X, int64_t M) {
   g.nout = n.nout;
   g.w0 = n.w32.p;
   g.wlast = n.w32.p + frags_first(n.width, g.kx) * 64;
+  g.wl = g.wlast + int64_t(n.nout) * n.width;
   g.wf = reinterpret_cast<const bf16x8*>(n.wfrag.p);
   g.wb = reinterpret_cast<const bf16x8*>(n.wfrag_t.p);
   g.bias = n.master.p + n.nweights;
@@ -1035,7 +1075,7 @@ void Mlp::make_fragments(hipStream_t s) {
   const int kx = even_cols(nin);
   const int64_t n0 = frags_first(width, kx), nh = (depth - 1) * frags_hidden(width);
   if (!wfrag.p) {
-    w32.alloc(n0 * 64 + int64_t(nout) * width);
+    w32.alloc(n0 * 64 + int64_t(nout + 16) * width);
     wfrag.alloc(std::max<int64_t>(1, nh) * kFrag);
     wfrag_t.alloc(std::max<int64_t>(1, nh) * kFrag);
   }
@@ -1048,10 +1088,11 @@ void Mlp::make_fragments(hipStream_t s) {
   g.nout = nout;
   g.w0 = w32.p;
   g.wlast = w32.p + n0 * 64;
+  g.wl = g.wlast + int64_t(nout) * width;
   for (int l = 0; l <= depth; ++l) g.woff[l] = woff[l];
   g.wf = reinterpret_cast<bf16x8*>(wfrag.p);
   g.wb = reinterpret_cast<bf16x8*>(wfrag_t.p);
-  const int64_t threads = std::max({n0 * 64, nh * 64, int64_t(nout) * width});
+  const int64_t threads = std::max({n0 * 64, nh * 64, int64_t(16) * width});
   k_make_fragments<<<g1(threads), 256, 0, s>>>(g);
 }
 

@@ -72,21 +72,22 @@ def test_training_reduces_loss():
     assert losses[-1] < 0.1 * losses[0]
 
 
-@pytest.mark.parametrize("width,depth,nin,M", [
-    (256, 4, 9, 1000), (256, 2, 8, 16321), (256, 2, 9, 32641), (128, 3, 1, 300),
-    (128, 2, 32, 16384), (128, 2, 5, 32768), (64, 2, 9, 129), (64, 1, 31, 20000),
-    (64, 4, 7, 32641)])
-def test_fused_inference_matches_forward(width, depth, nin, M):
+@pytest.mark.parametrize("width,depth,nin,M,nout", [
+    (256, 4, 9, 1000, 2), (256, 2, 8, 16321, 16), (256, 2, 9, 32641, 5), (128, 3, 1, 300, 1),
+    (128, 2, 32, 16384, 4), (128, 2, 5, 32768, 16), (64, 2, 9, 129, 5), (64, 1, 31, 20000, 16),
+    (64, 4, 7, 32641, 3), (256, 1, 3, 33, 8), (128, 2, 7, 95, 13)])
+def test_fused_inference_matches_forward(width, depth, nin, M, nout):
     """The one-kernel network gives the layer-by-layer path's values bit for
     bit (the same roundings in the same order of summation), at every number
-    of rows a workgroup takes. The layer-by-layer path is that of a network
+    of rows a workgroup takes and in both forms of the last layer (up to four
+    outputs and more). The layer-by-layer path is that of a network
     with more than 32 inputs: here the same network with 64 inputs of which
     those past the first n_in are zero, as are their weights, so that they add
     nothing. The two sum the gradients in orders of their own: their FP32 sums
     of some 500 rows at a time keep 1e-5 of sum |terms|, which is up to
     sqrt(M) = 180 times the gradient for targets without structure."""
-    net = _net(nin=nin, width=width, depth=depth, seed=5)
-    wide = _net(nin=64, width=width, depth=depth, seed=6)
+    net = _net(nin=nin, width=width, depth=depth, nout=nout, seed=5)
+    wide = _net(nin=64, width=width, depth=depth, nout=nout, seed=6)
     rng = np.random.default_rng(7)
     p = net.get_params()
     p[net.nweights:] = rng.uniform(-0.2, 0.2, net.nparams - net.nweights)
@@ -100,7 +101,7 @@ def test_fused_inference_matches_forward(width, depth, nin, M):
     wide.set_params(widen(p))
     X = rng.normal(0, 1, (M, nin)).astype(np.float32)
     Xw = np.concatenate([X, np.zeros((M, 64 - nin), np.float32)], axis=1)
-    T = rng.normal(0, 1, (M, 2)).astype(np.float32)
+    T = rng.normal(0, 1, (M, nout)).astype(np.float32)
     y = wide.forward(Xw)
     np.testing.assert_array_equal(wide.infer(Xw), y)
     np.testing.assert_array_equal(net.forward(X), y)
